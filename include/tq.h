@@ -272,6 +272,41 @@ int tq_decode_attention_groups(const uint16_t* q, int batch, int q_heads, int kv
                                float* out_f32, uint16_t* out_bf16, float* lse_out,
                                void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * Attention over bf16 key / value rows (decoded rows of a packed layer, tokens kept dense), any
+ * number of query tokens, over one range of tokens at a time.  Replaces the fp32 products and
+ * elementwise launches of reference chunked_turboquant_attention (runtime/attention.py:215-304) and
+ * of the dense-buffer merge (runtime/triton_kernels.py:338-366).  Logits and softmax weights are
+ * fp32; weights are not rounded before they meet the values.
+ *
+ *   q        bf16 or (q_is_f32) fp32 [batch][q_heads][q_len][dim] with element strides
+ *            (q_sb, q_sh, q_ss), dim contiguous, rows 16-byte aligned
+ *   k, v     bf16 [batch][kv_heads][tokens][dim] with element strides, rows 16-byte aligned
+ *   mask     added to the scaled logits; element (b, q head, query, token) at
+ *            b mask_sb + head mask_sh + query mask_ss + token (a stride of 0 broadcasts).
+ *            mask_type 0: none; 1: one byte each, 0 = not attended; 2: fp32, added
+ *   seq_starts, seq_ends  int32 [batch] (nullable): only positions [start, end) are attended,
+ *            token t being position pos0 + t
+ *   scale    logit scale, > 0
+ *   partials fp32 scratch of slots * batch * q_heads * q_len * (dim + 2) floats (16-byte aligned):
+ *            unnormalised outputs of every slot, then (maximum, sum of weights) of every slot
+ *   first_slot, n_split  the tokens are cut into n_split ranges, whose partials are the slots
+ *            [first_slot, first_slot + n_split) of 1..64
+ *   accumulate  0: the partials are written; 1: they are continued (the next tokens of the same
+ *            rows, with the same slots)
+ *   out_f32, out_bf16  [batch][q_heads][q_len][dim] (nullable): when given, all slots are added up
+ *            and normalised after this call's tokens; a row with nothing attended is 0.  prev /
+ *            prev_lse (nullable together): another part of the same softmax, normalised fp32 rows
+ *            and their log-sum-exp (tq_decode_attention's out_f32 and lse_out), weighed in
+ */
+int tq_dense_attention(const void* q, int q_is_f32, int batch, int q_heads, int kv_heads, int q_len, int dim,
+                       int64_t q_sb, int64_t q_sh, int64_t q_ss, const uint16_t* k, const uint16_t* v,
+                       int64_t tokens, int64_t k_sb, int64_t k_sh, int64_t k_st, int64_t v_sb, int64_t v_sh,
+                       int64_t v_st, const void* mask, int mask_type, int64_t mask_sb, int64_t mask_sh,
+                       int64_t mask_ss, const int32_t* seq_starts, const int32_t* seq_ends, int64_t pos0,
+                       float scale, float* partials, int slots, int first_slot, int n_split, int accumulate,
+                       const float* prev, const float* prev_lse, float* out_f32, uint16_t* out_bf16, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,122 @@
+"""Attention over bf16 rows (tq_dense_attention) against fp64 softmax attention:
+tile and split edges, every mask form, strided operands, position bounds, continued splits, and
+the routes of the chunked path and the dense-buffer merge onto it."""
+
+import math
+
+import pytest
+import torch
+
+from turboquant.runtime import attention as A
+from turboquant.runtime import kernels as K
+from turboquant.runtime.packed_qmse_cache import PackedMSELayer
+from turboquant.runtime.synthetic import kv_bf16
+
+pytestmark = pytest.mark.gpu
+
+D = 128
+SCALE = 1.0 / math.sqrt(D)
+#: fp32 logits (128 exact products, error <= 128 * 2^-24 * sum |q k| / sqrt(D)), weights and sums:
+#: with |logits| below ~10 the weights are within 1e-6, the normalised output within 1e-5 of its maximum
+TOL32 = 1e-5
+
+
+def randn(shape, seed, dtype=torch.float32):
+    return torch.randn(shape, generator=torch.Generator(device="cuda").manual_seed(seed), device="cuda").to(dtype)
+
+
+def oracle(q, k, v, add):
+    """fp64 attention; add [B or 1, Q or 1, Sq or 1, n] additive (or None); rows without tokens are 0."""
+    g = q.shape[1] // k.shape[1]
+    lg = q.double() @ k.double().repeat_interleave(g, 1).transpose(-1, -2) * SCALE
+    if add is not None:
+        lg = lg + add.double()
+    m = lg.amax(-1, keepdim=True)
+    p = torch.exp(lg - torch.where(torch.isfinite(m), m, torch.zeros_like(m)))
+    return (p @ v.double().repeat_interleave(g, 1)) / p.sum(-1, keepdim=True).clamp(min=1e-30)
+
+
+def check(got, ref, dtype):
+    tol = TOL32 if dtype == torch.float32 else 2 ** -8  # bf16 output: half an ulp of the largest value
+    assert got.dtype == dtype and got.shape == ref.shape
+    assert torch.isfinite(got).all()
+    assert (got.double() - ref).abs().max() <= tol * ref.abs().max()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,Hkv,g,Sq,n,mask,splits", [
+    (1, 1, 1, 1, 1, None, 1), (2, 2, 4, 1, 31, "bool", 1), (1, 2, 5, 3, 32, "f32", 1), (2, 1, 16, 2, 33, "lowest", 2),
+    (1, 2, 4, 9, 1000, "bool", 7), (2, 2, 7, 9, 129, "heads", 3), (1, 1, 4, 33, 4097, None, 64),
+    (1, 2, 2, 100, 257, "row", 9),
+])
+def test_dense_attention_matches_fp64(cuda, dtype, B, Hkv, g, Sq, n, mask, splits):
+    q = randn((B, Sq, Hkv * g, D), 1, dtype).transpose(1, 2)  # strided over heads and tokens
+    buf = randn((B, Hkv, n + 5, 2 * D), 2, torch.bfloat16)
+    k, v = buf[:, :, 2:n + 2, :D], buf[:, :, 3:n + 3, D:]
+    add = m = None
+    if mask in ("bool", "heads"):
+        m = randn((B, Hkv * g if mask == "heads" else 1, Sq, n + 3), 3)[..., 3:] > -0.5  # odd byte offsets
+        m[0, 0, 0] = False  # a row with nothing attended
+        add = torch.zeros(m.shape, device="cuda").masked_fill(~m, float("-inf"))
+    elif mask == "f32":
+        m = add = randn((B, 1, Sq, n), 3)
+    elif mask == "row":
+        m = add = randn((1, 1, 1, n), 3)
+    elif mask == "lowest":  # finite masks of the type's lowest value: a row of them is an even average
+        add = torch.zeros((B, 1, Sq, n), device="cuda")
+        add[:, :, :, ::3] = torch.finfo(torch.float32).min
+        add[1] = torch.finfo(torch.float32).min
+        m = add
+    got = K.DenseAttention(q, Hkv, splits).add(k, v, n, 0, splits, SCALE, mask=m, out=dtype)
+    ref = oracle(q, k, v, add)
+    if mask == "lowest":
+        ref[1] = v[1].double().mean(1).repeat_interleave(g, 0)[:, None]
+    check(got, ref, dtype)
+
+
+@pytest.mark.parametrize("Sq", [1, 20])
+def test_position_bounds_continued_partials_and_another_part(cuda, Sq):
+    B, Hkv, g, n = 3, 2, 4, 300
+    q, k, v = (randn(s, 5 + i, torch.bfloat16) for i, s in
+               enumerate([(B, Hkv * g, Sq, D), (B, Hkv, n, D), (B, Hkv, n, D)]))
+    starts = torch.tensor([0, 150, 90], dtype=torch.int32, device="cuda")
+    ends = torch.tensor([400, 333, 90], dtype=torch.int32, device="cuda")  # the last row attends to nothing
+    pos = torch.arange(n, device="cuda") + 100
+    ok = (pos >= starts[:, None]) & (pos < ends[:, None])
+    add = torch.zeros(B, 1, 1, n, device="cuda").masked_fill(~ok[:, None, None], float("-inf"))
+    att = K.DenseAttention(q, Hkv, 4)
+    for a, b in ((0, 128), (128, 131), (131, n)):  # the same splits over three ranges, one almost empty
+        got = att.add(k[:, :, a:b], v[:, :, a:], b - a, 0, 4, SCALE, starts=starts, ends=ends, pos0=100 + a,
+                      accumulate=a > 0, out=torch.float32 if b == n else None)
+    check(got, oracle(q, k, v, add), torch.float32)
+    # the first 100 tokens as another part, the rest as partials
+    lg = (q.float() @ k[:, :, :100].float().repeat_interleave(g, 1).transpose(-1, -2)) * SCALE
+    prev = torch.softmax(lg, -1) @ v[:, :, :100].float().repeat_interleave(g, 1)
+    got = K.DenseAttention(q, Hkv, 2).add(k[:, :, 100:], v[:, :, 100:], n - 100, 0, 2, SCALE, out=torch.float32, prev=prev,
+                                          prev_lse=torch.logsumexp(lg, -1))
+    check(got, oracle(q, k, v, None), torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_chunked_native_route_agrees_with_torch_operations(cuda, dtype, monkeypatch):
+    """Packed history in several segments, a dense buffer and new tokens under a mask wider than the
+    tokens, against the torch operations of the same function (taken when autograd is on)."""
+    B, Hq, Hkv, N, nd, Sq = 2, 8, 2, 1500, 7, 5
+    layer = PackedMSELayer(bits=3, quantize_decode=False)
+    layer.initialize_from_dense(kv_bf16((B, Hkv, N, D), seed=1), kv_bf16((B, Hkv, N, D), seed=2))
+    layer._lazy_update = True
+    layer.update(kv_bf16((B, Hkv, nd, D), seed=3), kv_bf16((B, Hkv, nd, D), seed=4))
+    nk, nv = kv_bf16((B, Hkv, 3, D), seed=5), kv_bf16((B, Hkv, 3, D), seed=6)
+    q = randn((B, Hq, Sq, D), 7, dtype)
+    mask = randn((B, 1, Sq, N + nd + 9), 8) > -1.0
+    monkeypatch.setattr(A, "_ROW_BYTES", 700 * B * Hkv * D * 4)
+    kw = dict(new_key=nk, new_value=nv, n_kv_groups=Hq // Hkv, attention_mask=mask, chunk_size=64)
+    native = A._native_chunked
+    calls = []
+    monkeypatch.setattr(A, "_native_chunked", lambda *a: calls.append(1) or native(*a))
+    got = A.chunked_turboquant_attention(q, layer, **kw)
+    assert calls
+    qg = q.clone().requires_grad_()
+    ref = A.chunked_turboquant_attention(qg, layer, **kw)
+    assert len(calls) == 1 and ref.requires_grad
+    check(got, ref.detach().double(), dtype)

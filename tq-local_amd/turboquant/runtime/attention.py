@@ -30,6 +30,7 @@ from typing import TYPE_CHECKING
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from turboquant.runtime import _lib
 from turboquant.runtime import kernels as K
@@ -139,7 +140,7 @@ def fused_attention(query_states: torch.Tensor, packed_layer: "PackedMSELayer", 
     if Hq // Hkv > K.MAX_GROUP:
         return None
     n_packed = packed_layer.packed_seq_length()
-    n_dense = 0 if packed_layer._dense_keys is None else int(packed_layer._dense_keys.shape[-2])
+    n_dense = packed_layer._dense_len
     scale = 1.0 / math.sqrt(D)
     known = getattr(packed_layer, "_tq_mask_contiguous", None)
     if attention_mask is not None and known is False:
@@ -167,6 +168,16 @@ def fused_attention(query_states: torch.Tensor, packed_layer: "PackedMSELayer", 
         out = outs[1] if f32 else outs
         return out.to(query_states.dtype).view(B, Hq, 1, D)
     _, o_packed, lse_packed = outs
+    dk, dv = packed_layer._dense_buf  # capacity buffers: the first n_dense tokens are attended
+    if _native_rows(query_states, dk, dv) and dk.shape[1] * n_kv_groups == Hq:
+        # two launches: the dense tokens' partials, and their merge with the packed part.  The torch
+        # operations below take ~22 (at B=4, Hq=32, N=8192 and 203 dense tokens 278 us a call, of
+        # which the packed part takes 17)
+        q = query_states if query_states.dtype == torch.bfloat16 else query_states.float()
+        n = K.DenseAttention.split_count(q, dk.shape[1], n_dense, K.DENSE_SPLITS)
+        return K.DenseAttention(q, dk.shape[1], n).add(dk, dv, n_dense, 0, n, scale, starts=starts, ends=ends,
+                                                       pos0=n_packed, out=query_states.dtype, prev=o_packed,
+                                                       prev_lse=lse_packed)
     # dense decode buffer: exact attention on the few generated tokens, merged by LSE
     dk = packed_layer._dense_keys.float().repeat_interleave(n_kv_groups, dim=1)  # [B, Hq, n, D]
     dv = packed_layer._dense_values.float().repeat_interleave(n_kv_groups, dim=1)
@@ -202,6 +213,75 @@ def _repeat_kv(t: torch.Tensor, n_rep: int) -> torch.Tensor:
     return t if n_rep == 1 else t.repeat_interleave(n_rep, dim=1)
 
 
+def _native_rows(query: torch.Tensor, *rows: torch.Tensor) -> bool:
+    """Whether libtq's attention over bf16 rows takes this query and these keys and values.
+    Autograd, transforms, tracing and dispatch modes need torch operations; rows of another
+    dtype would be rounded."""
+    dev, grad = query.device, torch.is_grad_enabled()
+    if (dev.type != "cuda" or query.shape[-1] != K.HEAD_DIM or query.dtype == torch.float64 or query.numel() == 0
+            or (grad and query.requires_grad) or torch._C._len_torch_dispatch_stack() or torch._C._is_tracing()
+            or torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0):
+        return False
+    for t in rows:
+        if (t.dtype != torch.bfloat16 or t.device != dev or t.dim() != 4 or t.shape[0] != query.shape[0]
+                or t.shape[3] != K.HEAD_DIM or (grad and t.requires_grad) or t.data_ptr() % 16):
+            return False
+        s0, s1, s2, s3 = t.stride()
+        if s3 != 1 or (s0 | s1 | s2) % 8:
+            return False
+    return True
+
+
+def _native_mask(mask: torch.Tensor | None, query: torch.Tensor, total: int) -> bool:
+    """Whether libtq takes the mask: bool or fp32 (after ``_additive_mask``'s conversion), four
+    dimensions that broadcast over [B, Q, Sq] and cover every token."""
+    if mask is None:
+        return True
+    if mask.dim() != 4 or mask.device != query.device or mask.requires_grad or mask.stride(-1) != 1:
+        return False
+    return (mask.dtype == torch.bool or mask.is_floating_point()) and mask.shape[3] >= total and \
+        all(m in (1, n) for m, n in zip(mask.shape[:3], query.shape[:3]))
+
+
+#: bytes of decoded key and value rows held at once by the native chunked path (at least chunk_size
+#: tokens): 64 MiB is 16384 tokens of 8 KV heads, enough to fill the device, and stays in the
+#: 256 MB last-level cache between the decoder and the attention
+_ROW_BYTES = 64 << 20
+
+
+def _native_chunked(query: torch.Tensor, layer: "PackedMSELayer", new_key, new_value, mask, chunk_size: int,
+                    kv_heads: int) -> torch.Tensor:
+    """``chunked_turboquant_attention`` in libtq kernels: per segment of the packed history two
+    decoder launches and one attention launch, one launch per dense part, one merge of the
+    splits."""
+    scale = 1.0 / math.sqrt(query.shape[-1])
+    q = query if query.dtype == torch.bfloat16 else query.float()
+    if mask is not None and mask.dtype != torch.bool:
+        mask = mask.float()
+    n_packed = layer.packed_seq_length()
+    step = max(int(chunk_size), _ROW_BYTES // (query.shape[0] * kv_heads * K.HEAD_DIM * 4), 1)
+    count = lambda n, most: K.DenseAttention.split_count(q, kv_heads, n, most)  # noqa: E731
+    ranges = []  # (keys, values, tokens, slots, first slot, continued): keys are None for packed tokens
+    slots = 0
+    if n_packed:
+        slots = count(min(step, n_packed), K.DENSE_SPLITS - 16)
+        ranges += [(None, None, min(step, n_packed - a), slots, 0, a > 0) for a in range(0, n_packed, step)]
+    for k, v in ((layer._dense_keys, layer._dense_values), (new_key, new_value)):
+        if k is not None and k.shape[2]:
+            n = count(k.shape[2], 8)
+            ranges.append((k, v, k.shape[2], n, slots, False))
+            slots += n
+    att = K.DenseAttention(q, kv_heads, slots)
+    off, out = 0, None
+    for i, (k, v, n, splits, first, more) in enumerate(ranges):
+        if k is None:
+            k, v = layer._key_rows(off, off + n), layer._value_rows(off, off + n)
+        out = att.add(k, v, n, first, splits, scale, mask=None if mask is None else mask[..., off:off + n],
+                      accumulate=more, out=query.dtype if i + 1 == len(ranges) else None)
+        off += n
+    return out
+
+
 def _additive_mask(mask: torch.Tensor | None) -> torch.Tensor | None:
     if mask is None:
         return None
@@ -225,6 +305,18 @@ def chunked_turboquant_attention(query_states: torch.Tensor, packed_layer: "Pack
     to return zeros (the reference's running maximum turns them into NaN).
     """
     B, Q, Sq, D = query_states.shape
+    dense = (packed_layer._dense_keys, packed_layer._dense_values)
+    parts = [t for t in (*dense, new_key, new_value) if t is not None]
+    n_packed = packed_layer.packed_seq_length()
+    total = n_packed + sum(int(t.shape[2]) for t in (dense[0], new_key) if t is not None)
+    if (total and chunk_size > 0 and Q % max(n_kv_groups, 1) == 0 and (new_key is None) == (new_value is None)
+            and (n_packed == 0 or packed_layer.dtype in (torch.bfloat16, torch.float32))
+            and _native_rows(query_states, *parts) and _native_mask(attention_mask, query_states, total)
+            and all(t.shape[1] * n_kv_groups == Q for t in parts)
+            and all(a is None or a.shape == b.shape for a, b in ((dense[0], dense[1]), (new_key, new_value)))
+            and (n_packed == 0 or packed_layer._shape == (B, Q // n_kv_groups, D))):
+        return _native_chunked(query_states, packed_layer, new_key, new_value, attention_mask, chunk_size,
+                               Q // n_kv_groups)
     scale = 1.0 / math.sqrt(D)
     qf = query_states.float()
     mask = _additive_mask(attention_mask)
@@ -248,7 +340,6 @@ def chunked_turboquant_attention(query_states: torch.Tensor, packed_layer: "Pack
         m = new_m
         off += n
 
-    n_packed = packed_layer.packed_seq_length()
     for a in range(0, n_packed, chunk_size):
         b = min(a + chunk_size, n_packed)
         attend(packed_layer._decode_keys_range(a, b), packed_layer._decode_values_range(a, b))

@@ -424,3 +424,78 @@ def decode_attention_groups(q: torch.Tensor, groups: list[dict], *, n_tokens: in
               _stream(q.device))
     outs = (out_bf16,) + ((out_f32,) if want_f32 else ()) + ((lse,) if want_lse else ())
     return outs if len(outs) > 1 else out_bf16
+
+
+#: most partials per row that ``DenseAttention`` keeps (tq_dense_attention takes 1..64 slots)
+DENSE_SPLITS = 64
+
+
+class DenseAttention:
+    """Attention over bf16 key / value rows (tq_dense_attention), for all query rows of ``q``
+    [B, Hq, Sq, D] (bf16 or fp32, head dimension 128).
+
+    ``add`` attends to one range of tokens with splits of its own, or continues the splits of an
+    earlier range; the last ``add`` returns the output.  The scratch lives for one attention call.
+    """
+
+    def __init__(self, q: torch.Tensor, kv_heads: int, slots: int):
+        self.q = q = rows16(q)
+        self.kv_heads = kv_heads
+        self.slots = slots
+        self.partials = torch.empty(slots * (q.numel() + 2 * (q.numel() // HEAD_DIM)), dtype=torch.float32,
+                                    device=q.device)
+
+    @staticmethod
+    def split_count(q: torch.Tensor, kv_heads: int, tokens: int, most: int) -> int:
+        """Splits of ``tokens`` tokens that fill the device without leaving any of them empty.
+        Few query rows per KV head run one wave per workgroup, one of which fits a SIMD;
+        otherwise two workgroups of four waves fit a CU."""
+        B, Hq, Sq, _ = q.shape
+        rows = Hq // kv_heads * Sq
+        waves = 1 if rows <= 32 else 2 if rows <= 64 else 4
+        blocks = B * kv_heads * -(-rows // (32 * waves))
+        tiles = max(1, -(-tokens // 32))
+        n = max(1, min(most, tiles, -(-(1024 if waves == 1 else 512) // blocks)))
+        return -(-tiles // -(-tiles // n))
+
+    def add(self, k: torch.Tensor, v: torch.Tensor, tokens: int, first: int, splits: int, scale: float, *,
+            mask: torch.Tensor | None = None, starts: torch.Tensor | None = None, ends: torch.Tensor | None = None,
+            pos0: int = 0, accumulate: bool = False, out: torch.dtype | None = None, prev: torch.Tensor | None = None,
+            prev_lse: torch.Tensor | None = None) -> torch.Tensor | None:
+        """Attend to the first ``tokens`` tokens of k, v [B, Hkv, n, D] (bf16) with the slots
+        [first, first + splits).  ``mask`` is bool or fp32, [B or 1, Hq or 1, Sq or 1, n];
+        ``starts`` / ``ends`` int32 [B] bound the attended positions, k's first token being position
+        ``pos0``.  With ``out`` (a dtype) the slots are added up and the output [B, Hq, Sq, D] is
+        returned; ``prev`` / ``prev_lse`` are another part of the same softmax (normalised fp32
+        output and log-sum-exp)."""
+        q = self.q
+        B, Hq, Sq, D = q.shape
+        if mask is None:
+            mp, mtype, m0, m1, m2 = None, 0, 0, 0, 0
+        else:
+            mp, mtype = mask.data_ptr(), 1 if mask.dtype == torch.bool else 2
+            m0, m1, m2 = (0 if mask.shape[i] == 1 else mask.stride(i) for i in range(3))
+        o = o32 = o16 = None
+        if out is not None:
+            o = torch.empty(q.shape, dtype=torch.bfloat16 if out == torch.bfloat16 else torch.float32, device=q.device)
+            if out == torch.bfloat16:
+                o16 = o.data_ptr()
+            else:
+                o32 = o.data_ptr()
+        qs, ks, vs = q.stride(), k.stride(), v.stride()
+        st = _lib.load().tq_dense_attention(
+            q.data_ptr(), int(q.dtype == torch.float32), B, Hq, self.kv_heads, Sq, D, qs[0], qs[1], qs[2], k.data_ptr(),
+            v.data_ptr(), tokens, ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], mp, mtype, m0, m1, m2, _ptr(starts),
+            _ptr(ends), pos0, scale, self.partials.data_ptr(), self.slots, first, splits, int(accumulate), _ptr(prev),
+            _ptr(prev_lse), o32, o16, _stream_handle(q.device))
+        if st != _lib.TQ_OK:
+            _lib.check("tq_dense_attention", st)
+        return None if o is None else o.to(out)
+
+
+def rows16(t: torch.Tensor) -> torch.Tensor:
+    """``t`` with rows of its last dimension contiguous and 16-byte aligned (itself when it is)."""
+    n = 16 // t.element_size()
+    if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and not any(s % n for s in t.stride()[:-1]):
+        return t
+    return t.clone(memory_format=torch.contiguous_format)

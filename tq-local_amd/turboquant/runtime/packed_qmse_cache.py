@@ -471,23 +471,30 @@ class PackedMSELayer(CacheLayerMixin):
                                rnorms=getattr(s, "kr" + sfx) if qjl else None, start=start)
         return out
 
-    def _decode_keys_range(self, start: int, end: int) -> torch.Tensor:
-        """Keys of packed positions [start, end) (reference :564-584)."""
+    def _key_rows(self, start: int, end: int) -> torch.Tensor:
+        """bf16 key rows of packed positions [start, end)."""
         s = self._store
         if self._split is not None:
-            return self._decode_split("k", self._split.key_normal, self._split.key_outlier, start, end).to(self.dtype)
+            return self._decode_split("k", self._split.key_normal, self._split.key_outlier, start, end)
         c = self.codecs
         if c.use_qjl_keys:
-            return K.dequantize_prod(s.kc, s.kn, s.ks, s.kr, end - start, c.key, c.qjl, start=start).to(self.dtype)
-        return K.dequantize_mse(s.kc, s.kn, end - start, c.key, start=start).to(self.dtype)
+            return K.dequantize_prod(s.kc, s.kn, s.ks, s.kr, end - start, c.key, c.qjl, start=start)
+        return K.dequantize_mse(s.kc, s.kn, end - start, c.key, start=start)
+
+    def _value_rows(self, start: int, end: int) -> torch.Tensor:
+        """bf16 value rows of packed positions [start, end)."""
+        s = self._store
+        if self._split is not None:
+            return self._decode_split("v", self._split.value_normal, self._split.value_outlier, start, end)
+        return K.dequantize_mse(s.vc, s.vn, end - start, self.codecs.value, start=start)
+
+    def _decode_keys_range(self, start: int, end: int) -> torch.Tensor:
+        """Keys of packed positions [start, end) (reference :564-584)."""
+        return self._key_rows(start, end).to(self.dtype)
 
     def _decode_values_range(self, start: int, end: int) -> torch.Tensor:
         """Values of packed positions [start, end) (reference :586-592)."""
-        s = self._store
-        if self._split is not None:
-            return self._decode_split("v", self._split.value_normal, self._split.value_outlier, start,
-                                      end).to(self.dtype)
-        return K.dequantize_mse(s.vc, s.vn, end - start, self.codecs.value, start=start).to(self.dtype)
+        return self._value_rows(start, end).to(self.dtype)
 
     def _decode_keys_full(self) -> torch.Tensor | None:
         return None if self._store is None else self._decode_keys_range(0, self._store.length)
