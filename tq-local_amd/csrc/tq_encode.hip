@@ -1,0 +1,858 @@
+// tq_encode.hip -- prefill encoders for gfx950: the fp32 encoder's bits from bf16 matrix products.
+//
+// The encoder's results are fixed by its fp32 evaluation order (tq_quantize.hip): a code is the
+// bucket of an fma chain over 128 dims, a sign the sign of one.  Running those chains costs 32
+// v_mfma_f32_16x16x4_f32 (1024 cycles) per 16 x 16 outputs, at the fp32 rate, and nothing else can
+// use the SIMD meanwhile.  But a bucket only needs its chain when the value is close to a boundary.
+// So the products run on the bf16 matrix cores (3 x 4 instructions of 16 cycles; the bf16 input is
+// exact, the matrix enters as three bf16 terms that add up to it), the value z' comes with a
+// bound eps on its distance from the chain's z, and
+//   |z' - b| >= eps for the one boundary b in reach:  the bucket of z' is the bucket of z;
+//   otherwise (about one output in 1000): the chain itself is run for that output.
+// The results are the chain's, bit for bit; only which outputs need it is decided by bounds.
+//
+// The bound, for rows of norm <= r and a vector of norm n (u = x / n has norm 1 up to 2^-20):
+//   the chain: 128 roundings, each at most 2^-24 of a partial sum, which Cauchy-Schwarz keeps
+//     below r: 7.63e-6 r, and u's own rounding 2^-24 r;
+//   z': the matrix instruction sums groups of 8 products aligned to the group's largest at 2^-24
+//     of it, and rounds after each group (probed: products below that are cut off, the sum of a
+//     group meets the accumulator with one rounding).  Over the groups of the leading term that is
+//     7 * 2^-24 r + 16 * 2^-24 r, over the others less than 2^-7 of it: 1.4e-6 r, taken as 1.6e-6 r;
+//   1 / n: the sum of squares is within 4e-6 of the exact one here and 7.7e-6 in the chain, half of
+//     which (and 3e-7 of square root and reciprocal) scales z', and |z| is at most the largest
+//     boundary's magnitude B where it matters: 6.3e-6 B;
+//   the table's boundaries, whose low bits hold a code: 2^bits * 2^-23 B.
+// r is measured when the matrix is staged; a matrix or vector outside the range where these
+// hold (not finite, squares that under- or overflow) takes the chain for every output.  The fp16
+// norm is handled alike: where the bound straddles a rounding boundary of fp16, the chain decides.
+//
+// Outputs that need their chain wait in a per-wave queue in LDS, their row of codes with them, and
+// are run 64 at a time, one lane each, so that the chains' latency is shared.
+
+#include <algorithm>
+#include <atomic>
+#include <type_traits>
+#include <utility>
+
+#include "tq_encode.h"
+
+namespace {
+
+using namespace tqmx;
+using tqenc::EncodeArgs;
+constexpr int D = TQ_DIM;
+constexpr int QPAIRS = 192;    // outputs waiting in a wave's queue
+constexpr uint32_t NORM_ONLY = 255;
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+union Frag {
+    uint32_t u[4];
+    uint4 q;
+    bf16x8 b;
+};
+__device__ __forceinline__ f32x4 mfma_bf16(const Frag& a, const Frag& b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, b.b, c, 0, 0, 0);
+}
+// fp32 -> bf16, nearest even (v_cvt_pk_bf16_f32: the bits of tq::f32_to_bf16 for every input).
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const bf16x2 p = {(__bf16)a, (__bf16)b};
+    return __builtin_bit_cast(uint32_t, p);
+}
+__device__ __forceinline__ float lo_half(uint32_t p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float hi_half(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
+// Truncated bf16 terms of two floats: a - hi is exact, and two truncations leave 8 bits.
+__device__ __forceinline__ uint32_t top_halves(float a, float b) {
+    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+__device__ __forceinline__ float below_top(float a) { return a - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u); }
+
+// The wave's LDS accesses complete in issue order; this keeps the compiler from moving them.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Largest row norm squared of an LDS-staged matrix: 16 neighbouring threads hold a row's partial
+// sums of squares.  Norms compare as their bits; a NaN compares above every number.
+__device__ __forceinline__ void row_norm_max(uint32_t* s_max, float part) {
+#pragma unroll
+    for (int k = 1; k < 16; k <<= 1) part += __shfl_xor(part, k);
+    if ((threadIdx.x & 15) == 0) atomicMax(s_max, __float_as_uint(part));
+}
+
+// Folds a 64-lane predicate (lane 16 g + v) to one bit per vector v.
+__device__ __forceinline__ uint32_t fold_vectors(uint64_t b) {
+    const uint32_t h = (uint32_t)b | (uint32_t)(b >> 32);
+    return (h | (h >> 16)) & 0xFFFFu;
+}
+
+__device__ __forceinline__ const uint16_t* row_of(const EncodeArgs& a, uint32_t vi, int64_t* slot) {
+    const uint32_t gh = fdiv(vi, a.tok_div), t = vi - gh * (uint32_t)a.tokens;
+    const uint32_t b = fdiv(gh, a.head_div), h = gh - b * (uint32_t)a.heads;
+    *slot = (int64_t)gh * a.out_cap + a.out_offset + t;
+    return a.x + (int64_t)b * a.x_sb + (int64_t)h * a.x_sh + (int64_t)t * a.x_st;
+}
+
+// Bits 16 (2 k), 16 (2 k + 1) of a group's channel mask as halves of a word: channels 2k, 2k + 1.
+__device__ __forceinline__ uint32_t pair_mask(uint32_t m, int k) {
+    return (((m >> (2 * k)) & 1u) ? 0x0000FFFFu : 0u) | (((m >> (2 * k + 1)) & 1u) ? 0xFFFF0000u : 0u);
+}
+
+// #{i : b_i < z} by binary search over the boundaries in LDS (the encoders' search).
+__device__ __forceinline__ uint32_t bucket_lds(float z, const float* s_b, int bits) {
+    uint32_t c = 0;
+#pragma unroll 1
+    for (uint32_t s = 1u << (bits - 1); s > 0; s >>= 1) c += (s_b[c + s - 1] < z) ? s : 0u;
+    return c;
+}
+
+// ------------------------------------------------------------------ codes and norms
+// Bucketize through a uniform grid.  Cells of width w = (smallest gap between neighbouring
+// boundaries) / 4 start at e0 = b_0 - 2w; cell k holds c0 = #{i : b_i < e0 + (k - 1) w} and b_{c0}.
+// z' goes to the cell k = clamp(floor((z' - e0) / w)); the quotient is computed within 1e-3
+// (|e0| / w and |b_NB-1| / w stay below 4096) and z' is within w / 16 of z (eps < w / 16 or the grid is
+// not used), so z lies in (e0 + (k - 1.1) w, e0 + (k + 2.1) w), a window of 3.2 w that holds at most one
+// boundary (the gap is 4w), b_{c0} if any: code(z) = c0 + [b_{c0} < z].  The clamped ends: the first
+// cell is 2w below b_0, the last more than w above b_NB-1, where b is a number above all z.  A cell is
+// one word, the boundary with its low `bits` bits replaced by c0.
+template <int BITS, bool GROUP, int NT>
+__global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
+    constexpr int NB = (1 << BITS) - 1;
+    constexpr int RW = 4 * BITS;  // dwords of a plain row; a queued row holds 32 codes per lane, BITS words
+    constexpr uint32_t CMASK = NB;
+    constexpr int LUT_MAX = BITS <= 6 ? 512 : 2048;  // cells of the bucketize grid
+    constexpr int QROWS = BITS <= 6 ? 48 : 32;       // vectors waiting in a wave's queue
+    __shared__ uint4 s_img[8 * 4 * 3 * 64];  // [row tile][k-step][term][lane]
+    __shared__ float s_lut[LUT_MAX];
+    __shared__ float s_bound[NB];
+    __shared__ uint32_t s_max;
+    __shared__ uint32_t s_row[MQ_WAVES][QROWS][RW];
+    __shared__ uint32_t s_vec[MQ_WAVES][QROWS];
+    __shared__ uint32_t s_pair[MQ_WAVES][QPAIRS];
+
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int v = lane & 15, g = lane >> 4;
+    const int sub_dim = GROUP ? a.sub_dim : D;
+    if (threadIdx.x == 0) s_max = 0u;
+    for (int i = threadIdx.x; i < NB; i += MQ_THREADS) s_bound[i] = a.boundaries[i];
+    __syncthreads();
+    // ---- the matrix as three bf16 terms: index j = 32 q + 4 t + i is row 4 q + i of tile t, so that
+    // lane 16 q + v ends with the codes [32 q, 32 q + 32) of its vector
+    for (int idx = threadIdx.x; idx < D * D / 8; idx += MQ_THREADS) {
+        const int j = idx >> 4, c = idx & 15;  // dims 8 c .. 8 c + 7
+        float e[8];
+        if (!GROUP || j < sub_dim) {
+            const float4 p = reinterpret_cast<const float4*>(a.R)[j * (D / 4) + 2 * c];
+            const float4 q = reinterpret_cast<const float4*>(a.R)[j * (D / 4) + 2 * c + 1];
+            e[0] = p.x, e[1] = p.y, e[2] = p.z, e[3] = p.w, e[4] = q.x, e[5] = q.y, e[6] = q.z, e[7] = q.w;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) e[k] = 0.0f;
+        }
+        float part = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) part = __builtin_fmaf(e[k], e[k], part);
+        row_norm_max(&s_max, part);
+        const int t = (j >> 2) & 7, m = 4 * (j >> 5) + (j & 3), s = c >> 2, l = 16 * (c & 3) + m;
+        uint4* dst = s_img + (t * 4 + s) * 3 * 64 + l;
+#pragma unroll
+        for (int term = 0; term < 3; ++term) {
+            uint32_t w[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                w[k] = top_halves(e[2 * k], e[2 * k + 1]);
+                e[2 * k] = below_top(e[2 * k]);
+                e[2 * k + 1] = below_top(e[2 * k + 1]);
+            }
+            dst[term * 64] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    }
+    // ---- bucket grid
+    float gap = __builtin_inff();
+    bool sorted = true;
+    for (int i = 1; i < NB; ++i) {
+        const float d = s_bound[i] - s_bound[i - 1];
+        sorted = sorted && d > 0.0f;
+        gap = fminf(gap, d);
+    }
+    __syncthreads();
+    const float r_norm = __builtin_sqrtf(__uint_as_float(s_max)) * 1.0001f;
+    float b_max = 0.0f;
+    for (int i = 0; i < NB; ++i) b_max = fmaxf(b_max, fabsf(s_bound[i]));
+    const float eps = r_norm * 9.5e-6f + (b_max + 1e-4f * r_norm) * (6.5e-6f + (float)(1 << BITS) * 1.2e-7f);
+    const float w = NB > 1 ? gap * 0.25f : 1.0f;
+    const float e0 = s_bound[0] - 2.0f * w;
+    const float span = (s_bound[NB - 1] - e0) / w;
+    const float g_scale = 1.0f / w;
+    const float g_off = -e0 * g_scale;
+    // outside the bounds' range every output takes its chain
+    const bool exact_all = !(r_norm < 1e18f) || !(b_max < 1e18f);
+    const bool use_grid = sorted && w > 16.0f * eps && span < (float)(LUT_MAX - 5) && fabsf(g_off) < 4096.0f &&
+                          fabsf(s_bound[NB - 1] * g_scale) < 4096.0f;
+    const int cells = use_grid ? (int)ceilf(span) + 4 : 0;
+    for (int k = threadIdx.x; k < cells; k += MQ_THREADS) {
+        const float start = e0 + (float)(k - 1) * w;
+        uint32_t c0 = 0;
+        for (int i = 0; i < NB; ++i) c0 += s_bound[i] < start ? 1u : 0u;
+        const float b = c0 < NB ? s_bound[c0] + 0.0f : 3e38f;
+        s_lut[k] = __uint_as_float((__float_as_uint(b) & ~CMASK) | c0);
+    }
+    __syncthreads();  // the last barrier: each wave then works on its own tiles
+
+    // f = cell + 2^23 in the low bits of a float: one fma and one med3, and the bits are the index
+    constexpr float MAGIC = 8388608.0f;
+    const float f_off = g_off + (MAGIC - 0.5f);
+    const float f_top = MAGIC + (float)(cells - 1);
+    const float s_b0 = s_bound[0];
+    const uint32_t mw[4] = {a.mask[0], a.mask[1], a.mask[2], a.mask[3]};
+    const int row_bytes = GROUP ? (sub_dim * BITS + 7) >> 3 : D * BITS / 8;
+    // this lane's outputs 32 g + jj with jj < mine count
+    const int mine = GROUP ? std::min(std::max(sub_dim - 32 * g, 0), 32) : 32;
+    const int n_t = GROUP && sub_dim < 32 ? (sub_dim + 3) >> 2 : 8;
+
+    uint32_t q_rows = 0, q_pairs = 0;  // wave-uniform
+    auto store_row = [&](uint8_t* codes, const uint32_t* words) {  // this lane's BITS words of a row
+        if constexpr (!GROUP) {
+            uint32_t* dst = reinterpret_cast<uint32_t*>(codes) + BITS * g;
+            if constexpr (BITS == 4) *reinterpret_cast<uint4*>(dst) = make_uint4(words[0], words[1], words[2], words[3]);
+            else if constexpr (BITS == 2) *reinterpret_cast<uint2*>(dst) = make_uint2(words[0], words[1]);
+            else
+#pragma unroll
+                for (int k = 0; k < BITS; ++k) dst[k] = words[k];
+        } else {
+            const int first = 4 * BITS * g;
+#pragma unroll
+            for (int k = 0; k < BITS; ++k) {
+                const int left = row_bytes - (first + 4 * k);
+                uint8_t* dst = codes + first + 4 * k;
+                if (left >= 4) {
+                    __builtin_memcpy(dst, &words[k], 4);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 3; ++e)
+                        if (e < left) dst[e] = (uint8_t)(words[k] >> (8 * e));
+                }
+            }
+        }
+    };
+    // the queued outputs' chains, one lane each
+    auto run_pairs = [&]() {
+        wave_lds_fence();
+        for (uint32_t base = 0; base < q_pairs; base += 64) {
+            if (base + lane < q_pairs) {
+                const uint32_t e = s_pair[wave][base + lane], qr = e >> 8, j = e & 255u;
+                const uint32_t vi = s_vec[wave][qr];
+                int64_t slot;
+                const uint4* x4 = reinterpret_cast<const uint4*>(row_of(a, vi, &slot));
+                auto channels = [&](int c, float* o) {  // channels 8 c .. 8 c + 7, masked
+                    const uint4 p = x4[c];
+                    const uint32_t h[4] = {p.x, p.y, p.z, p.w};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        uint32_t hk = h[k];
+                        if constexpr (GROUP) hk &= pair_mask(a.mask[c >> 2] >> (8 * (c & 3)), k);
+                        o[2 * k] = lo_half(hk);
+                        o[2 * k + 1] = hi_half(hk);
+                    }
+                };
+                float ss = 0.0f;
+#pragma unroll 4
+                for (int c = 0; c < D / 8; ++c) {
+                    float o[8];
+                    channels(c, o);
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) ss = __builtin_fmaf(o[k], o[k], ss);
+                }
+                float n = tq::sqrt_rn(ss);
+                if (!(n > 0.0f)) n = 1.0f;
+                if (j == NORM_ONLY) {
+                    a.norms[slot] = (uint16_t)tq::f32_to_f16(n);
+                } else {
+                    const float4* rj = reinterpret_cast<const float4*>(a.R) + j * (D / 4);
+                    float z = 0.0f;
+#pragma unroll 4
+                    for (int c = 0; c < D / 8; ++c) {
+                        float o[8];
+                        channels(c, o);
+                        const float4 p = rj[2 * c], q = rj[2 * c + 1];
+                        const float rr[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) z = __builtin_fmaf(tq::div_rn(o[k], n), rr[k], z);
+                    }
+                    const uint32_t code = bucket_lds(z, s_bound, BITS);
+                    uint32_t* row = s_row[wave][qr];
+                    const uint32_t bit = j * BITS, wi = bit >> 5, sh = bit & 31;
+                    uint64_t old = row[wi];
+                    if (sh + BITS > 32) old |= (uint64_t)row[wi + 1] << 32;
+                    const uint64_t diff = (uint64_t)(((uint32_t)(old >> sh) & CMASK) ^ code) << sh;
+                    // other lanes may change other codes of the same word
+                    if ((uint32_t)diff) atomicXor(&row[wi], (uint32_t)diff);
+                    if ((uint32_t)(diff >> 32)) atomicXor(&row[wi + 1], (uint32_t)(diff >> 32));
+                }
+            }
+        }
+        q_pairs = 0;
+        wave_lds_fence();
+    };
+    auto store_queued = [&]() {  // the waiting rows, their outputs run
+        for (uint32_t r0 = 0; r0 < q_rows; r0 += 16) {
+            const uint32_t qr = r0 + v;
+            if (qr < q_rows) {
+                int64_t slot;
+                row_of(a, s_vec[wave][qr], &slot);
+                uint32_t words[BITS];
+#pragma unroll
+                for (int k = 0; k < BITS; ++k) words[k] = s_row[wave][qr][BITS * g + k];
+                store_row(a.codes + slot * row_bytes, words);
+            }
+        }
+        q_rows = 0;
+        wave_lds_fence();
+    };
+
+    const int64_t n_items = (a.n_vec + 16 * NT - 1) / (16 * NT);
+    for (int64_t item = (int64_t)blockIdx.x * MQ_WAVES + wave;; item += (int64_t)gridDim.x * MQ_WAVES) {
+        // past the last item the vectors are all dead: one more round to empty the queue
+        const bool last = item >= n_items;
+        // ---- NT tiles of 16 vectors: lane 16 g + v holds dims 32 s + 8 g + (0..7) of vector v, the B operand
+        Frag x[NT][4];
+        int64_t slot[NT];
+        float rn[NT], mg[NT];
+        bool live[NT];
+        uint32_t n_amb = 0, special = 0;  // per tile bit: the fp16 norm, or everything, needs the chain
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const uint32_t vi = (uint32_t)item * (16u * NT) + 16u * n + (uint32_t)v;  // n_vec < 2^31
+            live[n] = !last && vi < (uint64_t)a.n_vec;
+            slot[n] = 0;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) x[n][s].q = make_uint4(0u, 0u, 0u, 0u);
+            if (live[n]) {
+                const uint4* x4 = reinterpret_cast<const uint4*>(row_of(a, vi, &slot[n]));
+#pragma unroll
+                for (int s = 0; s < 4; ++s) x[n][s].q = x4[4 * s + g];
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            float ss = 0.0f;
+            uint32_t any = 0u;
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if constexpr (GROUP) x[n][s].u[k] &= pair_mask(mw[s] >> (8 * g), k);
+                    const uint32_t p = x[n][s].u[k];
+                    ss = __builtin_fmaf(lo_half(p), lo_half(p), ss);
+                    ss = __builtin_fmaf(hi_half(p), hi_half(p), ss);
+                    any |= p;
+                }
+            ss += __shfl_xor(ss, 16);
+            ss += __shfl_xor(ss, 32);
+            any &= 0x7FFF7FFFu;
+            any |= (uint32_t)__shfl_xor((int)any, 16);
+            any |= (uint32_t)__shfl_xor((int)any, 32);
+            const bool zero = any == 0u;  // norm 1, every chain 0
+            const float n_ = zero ? 1.0f : __builtin_sqrtf(ss);
+            rn[n] = __builtin_amdgcn_rcpf(n_);
+            mg[n] = zero ? -1.0f : eps;
+            const bool bad = !zero && (!(ss > 1e-24f) || !(ss < 1e30f) || exact_all);
+            const uint32_t h0 = tq::f32_to_f16(n_ * (1.0f - 7e-6f)), h1 = tq::f32_to_f16(n_ * (1.0f + 7e-6f));
+            if (bad || (h0 != h1 && !zero)) n_amb |= 1u << n;
+            if (bad) special |= 1u << n;
+            if (live[n] && g == 0 && !((n_amb >> n) & 1u)) a.norms[slot[n]] = (uint16_t)tq::f32_to_f16(n_);
+        }
+
+        // ---- products, codes; bit 31 - jj of amb: output 32 g + jj needs its chain
+        uint32_t out[NT][BITS], amb[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            amb[n] = 0u;
+#pragma unroll
+            for (int k = 0; k < BITS; ++k) out[n][k] = 0u;
+        }
+        auto emit = [&](int n, int jj, uint32_t code, bool close) {
+            amb[n] = amb[n] + amb[n] + (close ? 1u : 0u);
+            const int bit = jj * BITS, wi = bit >> 5, sh = bit & 31;
+            out[n][wi] |= code << sh;
+            if (sh + BITS > 32) out[n][wi + 1] |= code >> (32 - sh);
+        };
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            if (GROUP && t >= n_t) break;
+            f32x4 acc[NT];
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int term = 2; term >= 0; --term)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    Frag m;
+                    m.q = s_img[((t * 4 + s) * 3 + term) * 64 + lane];
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(m, x[n][s], acc[n]);
+                }
+            if (NB == 1 || use_grid) {
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        float b = s_b0;
+                        uint32_t code = 0u;
+                        if constexpr (NB > 1) {
+                            float f = __builtin_fmaf(acc[n][i], rn[n] * g_scale, f_off);
+                            f = __builtin_amdgcn_fmed3f(f, MAGIC, f_top);
+                            b = s_lut[__float_as_uint(f) & (LUT_MAX - 1)];
+                            code = __float_as_uint(b) & CMASK;
+                        }
+                        const float d = __builtin_fmaf(acc[n][i], rn[n], -b);
+                        emit(n, 4 * t + i, code + (d > 0.0f ? 1u : 0u), !(fabsf(d) >= mg[n]));
+                    }
+            } else {
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float z = acc[n][i] * rn[n];
+                        bool close = false;
+#pragma unroll 1
+                        for (int k = 0; k < NB; ++k) close = close || !(fabsf(z - s_bound[k]) >= mg[n]);
+                        emit(n, 4 * t + i, bucket_lds(z, s_bound, BITS), close);
+                    }
+            }
+            __builtin_amdgcn_sched_barrier(0);  // not every tile's matrix fragments at once
+        }
+        if (GROUP && n_t < 8) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n) amb[n] <<= 32 - 4 * n_t;
+        }
+
+        // ---- outputs beyond the group's rows are no outputs
+        if constexpr (GROUP) {
+#pragma unroll
+            for (int k = 0; k < BITS; ++k) {
+                const int left = mine * BITS - 32 * k;
+                const uint32_t keep = left >= 32 ? 0xFFFFFFFFu : left <= 0 ? 0u : (1u << left) - 1u;
+#pragma unroll
+                for (int n = 0; n < NT; ++n) out[n][k] &= keep;
+            }
+        }
+        const uint32_t valid = mine >= 32 ? 0xFFFFFFFFu : mine == 0 ? 0u : ~(0xFFFFFFFFu >> mine);
+
+        // ---- rows without a doubtful output leave; the others queue with the outputs to run
+        uint32_t pend = 0, given = 0, first[NT], queued[NT];  // wave-uniform, a bit per tile
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            if ((special >> n) & 1u) amb[n] = 0xFFFFFFFFu;
+            amb[n] = live[n] ? amb[n] & valid : 0u;
+            if (!live[n]) n_amb &= ~(1u << n);
+            const uint32_t rows = fold_vectors(__builtin_amdgcn_ballot_w64(amb[n] != 0u));
+            if (live[n] && !((rows >> v) & 1u)) store_row(a.codes + slot[n] * row_bytes, out[n]);
+            queued[n] = rows | fold_vectors(__builtin_amdgcn_ballot_w64((n_amb >> n) & 1u));
+            first[n] = 0u;
+            if (queued[n]) pend |= 1u << n;
+        }
+        // normally one round; more when the queue fills (vectors whose every output is doubtful)
+        for (;;) {
+            bool full = false;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                if (!((pend >> n) & 1u)) continue;
+                const uint32_t below = __popc(queued[n] & ((1u << v) - 1u));
+                if (!((given >> n) & 1u)) {
+                    if (q_rows + __popc(queued[n]) > QROWS) {
+                        full = true;
+                        continue;
+                    }
+                    given |= 1u << n;
+                    first[n] = q_rows;
+                    q_rows += __popc(queued[n]);
+                    if ((queued[n] >> v) & 1u) {
+                        if (g == 0) s_vec[wave][first[n] + below] = (uint32_t)item * (16u * NT) + 16u * n + (uint32_t)v;
+#pragma unroll
+                        for (int k = 0; k < BITS; ++k) s_row[wave][first[n] + below][BITS * g + k] = out[n][k];
+                    }
+                }
+                for (;;) {
+                    const bool norm = ((n_amb >> n) & 1u) && g == 0;
+                    const bool p = norm || amb[n] != 0u;
+                    const uint64_t who = __builtin_amdgcn_ballot_w64(p);
+                    if (who == 0) {
+                        pend &= ~(1u << n);
+                        break;
+                    }
+                    if (q_pairs + 64 > QPAIRS) break;
+                    const uint32_t at = q_pairs + __builtin_amdgcn_mbcnt_hi((uint32_t)(who >> 32),
+                                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)who, 0));
+                    const int top = __clz((int)amb[n]);  // jj of the first doubtful output
+                    if (p) s_pair[wave][at] = ((first[n] + below) << 8) | (norm ? NORM_ONLY : 32u * g + (uint32_t)top);
+                    if (!norm) amb[n] &= ~(0x80000000u >> (top & 31));
+                    if (norm || g != 0) n_amb &= ~(1u << n);
+                    q_pairs += __popcll(who);
+                }
+            }
+            if (!last && pend == 0 && q_pairs < QPAIRS - 64) break;
+            run_pairs();
+            if (last || full) {
+                // a tile given rows and still holding outputs keeps them
+                if ((pend & given) == 0) store_queued();
+            }
+            if (pend == 0) break;
+        }
+        if (last) break;
+    }
+}
+
+// ------------------------------------------------------------------ residual sketch of Q_prod keys
+// khat_d = bf16((fma chain j of C[code_j] R[j][d]) * f32(f16(n))) must be the chain itself: its bf16
+// rounding has a boundary within the bound of one value in twenty.  So this product stays on the
+// fp32 matrix cores (the decoder's image, tq_mfma.h; 8192 of a tile's ~12500 cycles), and the QJL
+// projection, of which only signs are kept, runs on the bf16 ones: r = x - khat as two bf16
+// terms (nearest even, r within 2^-18), S as two, three products.  With |r| factored out the bound is
+// s (7.63e-6 chain + 3 * 2^-18 terms + 1.6e-6 + rounding) = 2.2e-5 s, s the largest row norm of S; a
+// projection inside it, one in 4000, is run as the chain, with rhat from the division the chain uses.
+template <int BITS, int... I>
+__device__ __forceinline__ void plain_centers(const uint32_t* w, int g, const float* cent, float* cv,
+                                              std::integer_sequence<int, I...>) {
+    constexpr uint32_t MASK = (1u << BITS) - 1u;
+    ((cv[I] = cent[(uint32_t)(((uint64_t)w[(4 * I * BITS) >> 5] | ((uint64_t)w[((4 * I * BITS) >> 5) + 1] << 32)) >>
+                               (((4 * I * BITS) & 31) + g * BITS)) &
+                   MASK]),
+     ...);
+}
+
+template <int BITS, bool GROUP>
+__global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
+    constexpr int RW = 4 * BITS;
+    constexpr int GRW = RW + 2;  // staged dwords of a group row: a misaligned start, one spare
+    __shared__ float4 s_img[D * D / 4];       // R^T, fp32
+    __shared__ uint4 s_s[8 * 4 * 2 * 64];     // S, two bf16 terms: [row tile][k-step][term][lane]
+    __shared__ float s_cent[1 << BITS];
+    __shared__ uint32_t s_code[GROUP ? MQ_WAVES : 1][GROUP ? 16 : 1][GRW];
+    __shared__ float4 s_r[MQ_WAVES][2][D / 4];
+    __shared__ uint32_t s_max;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int v = lane & 15, g = lane >> 4;
+    const int sub_dim = GROUP ? a.sub_dim : D;
+    const int pad = D - sub_dim;
+    if (threadIdx.x == 0) s_max = 0u;
+    __syncthreads();
+    build_image_transposed(reinterpret_cast<float*>(s_img), a.R, sub_dim);
+    for (int i = threadIdx.x; i < (1 << BITS); i += MQ_THREADS) s_cent[i] = a.centers[i];
+    // lane 16 g + m of k-step s: dims 32 g + 8 s + (0..7), the dims in which lane 16 g + v holds r
+    for (int idx = threadIdx.x; idx < D * D / 8; idx += MQ_THREADS) {
+        const int j = idx >> 4, c = idx & 15;
+        float e[8];
+        if (!GROUP || j < sub_dim) {
+            const float4 p = reinterpret_cast<const float4*>(a.S)[j * (D / 4) + 2 * c];
+            const float4 q = reinterpret_cast<const float4*>(a.S)[j * (D / 4) + 2 * c + 1];
+            e[0] = p.x, e[1] = p.y, e[2] = p.z, e[3] = p.w, e[4] = q.x, e[5] = q.y, e[6] = q.z, e[7] = q.w;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) e[k] = 0.0f;
+        }
+        float part = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) part = __builtin_fmaf(e[k], e[k], part);
+        row_norm_max(&s_max, part);
+        const int t = (j >> 2) & 7, m = 4 * (j >> 5) + (j & 3), s = c & 3, l = 16 * (c >> 2) + m;
+        uint32_t hi[4], lo[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            hi[k] = bf16_pair(e[2 * k], e[2 * k + 1]);
+            lo[k] = bf16_pair(e[2 * k] - lo_half(hi[k]), e[2 * k + 1] - hi_half(hi[k]));
+        }
+        s_s[((t * 4 + s) * 2 + 0) * 64 + l] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        s_s[((t * 4 + s) * 2 + 1) * 64 + l] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    }
+    __syncthreads();  // the last barrier: each wave then works on its own tiles
+    const float s_norm = __builtin_sqrtf(__uint_as_float(s_max)) * 1.0001f;
+    const float eps = s_norm * 2.25e-5f;
+    const bool exact_all = !(s_norm < 1e15f);
+    const float4* a_img = s_img + (lane ^ g);
+    const uint32_t mw = g == 0 ? a.mask[0] : g == 1 ? a.mask[1] : g == 2 ? a.mask[2] : a.mask[3];
+    const int row_bytes = GROUP ? (sub_dim * BITS + 7) >> 3 : D * BITS / 8;
+    const int sign_bytes = (sub_dim + 7) >> 3;
+    const int mine = std::min(std::max(sub_dim - 32 * g, 0), 32);
+    const uint32_t valid = mine >= 32 ? 0xFFFFFFFFu : (1u << mine) - 1u;
+
+    const int64_t n_tiles = (a.n_vec + 15) / 16;
+    for (int64_t tile = (int64_t)blockIdx.x * MQ_WAVES + wave; tile < n_tiles;
+         tile += (int64_t)gridDim.x * MQ_WAVES) {
+        const uint32_t vi = (uint32_t)tile * 16u + (uint32_t)v;
+        const bool live = vi < (uint64_t)a.n_vec;
+        int64_t slot = 0;
+        uint4 xr[4];
+        float nf = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) xr[c] = make_uint4(0u, 0u, 0u, 0u);
+        if (live) {
+            const uint4* x4 = reinterpret_cast<const uint4*>(row_of(a, vi, &slot));
+#pragma unroll
+            for (int c = 0; c < 4; ++c) xr[c] = x4[4 * g + c];
+            nf = tq::f16_to_f32(a.norms[slot]);
+        }
+        // ---- C[code] of index 4s + g (behind `pad` zeros for a group)
+        float cv[32];
+        if constexpr (!GROUP) {
+            uint32_t w[RW + 1];
+            const uint4* c4 = reinterpret_cast<const uint4*>(a.codes + slot * row_bytes);
+#pragma unroll
+            for (int c = 0; c < BITS; ++c) {
+                uint4 q = make_uint4(0u, 0u, 0u, 0u);
+                if (live) q = c4[c];
+                w[4 * c] = q.x, w[4 * c + 1] = q.y, w[4 * c + 2] = q.z, w[4 * c + 3] = q.w;
+            }
+            w[RW] = 0u;
+            plain_centers<BITS>(w, g, s_cent, cv, std::make_integer_sequence<int, 32>{});
+        } else {
+            // the row byte by byte where it does not fill a dword, so nothing outside it is read
+            uint32_t* row = s_code[wave][v];
+            const uint8_t* src = a.codes + slot * row_bytes;
+            for (int k = g; k < GRW; k += 4) {
+                uint32_t w = 0u;
+                if (live) {
+                    if (4 * k + 4 <= row_bytes) {
+                        __builtin_memcpy(&w, src + 4 * k, 4);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 3; ++e)
+                            if (4 * k + e < row_bytes) w |= (uint32_t)src[4 * k + e] << (8 * e);
+                    }
+                }
+                row[k] = w;
+            }
+            wave_lds_fence();
+#pragma unroll
+            for (int s = 0; s < 32; ++s) {
+                const int j = 4 * s + g - pad;
+                const uint32_t bit = (uint32_t)(j * BITS);
+                cv[s] = 0.0f;
+                if (j >= 0)
+                    cv[s] = s_cent[__builtin_amdgcn_ubfe(
+                        __builtin_amdgcn_alignbit(row[(bit >> 5) + 1], row[bit >> 5], bit & 31), 0, BITS)];
+            }
+            wave_lds_fence();
+        }
+        f32x4 acc[8];
+        image_products(a_img, cv, acc);
+        // ---- r = x - bf16(khat), dims 32 g + (0..31)
+        float r[32];
+        float rs = 0.0f;
+        const uint32_t xw[16] = {xr[0].x, xr[0].y, xr[0].z, xr[0].w, xr[1].x, xr[1].y, xr[1].z, xr[1].w,
+                                 xr[2].x, xr[2].y, xr[2].z, xr[2].w, xr[3].x, xr[3].y, xr[3].z, xr[3].w};
+#pragma unroll
+        for (int p = 0; p < 16; ++p) {
+            uint32_t xp = xw[p];
+            if constexpr (GROUP) xp &= pair_mask(mw, p);
+            const uint32_t kh = bf16_pair(acc[p >> 1][2 * (p & 1)] * nf, acc[p >> 1][2 * (p & 1) + 1] * nf);
+            r[2 * p] = lo_half(xp) - lo_half(kh);
+            r[2 * p + 1] = hi_half(xp) - hi_half(kh);
+            rs = __builtin_fmaf(r[2 * p], r[2 * p], rs);
+            rs = __builtin_fmaf(r[2 * p + 1], r[2 * p + 1], rs);
+        }
+        rs += __shfl_xor(rs, 16);
+        rs += __shfl_xor(rs, 32);
+        const bool bad = rs != 0.0f && (!(rs > 1e-24f) || !(rs < 1e30f) || exact_all);
+        // a sum of squares of 0 can hide residuals whose squares vanish; the chain's does as well
+        const float rho = rs == 0.0f ? 1.0f : __builtin_sqrtf(rs);
+        const uint32_t h0 = tq::f32_to_f16(rho * (1.0f - 7e-6f)), h1 = tq::f32_to_f16(rho * (1.0f + 7e-6f));
+        const bool tiny = rs == 0.0f;
+        bool rho_amb = bad || (h0 != h1 && !tiny);
+        Frag rh[4], rl[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float e0 = r[8 * s + 2 * k], e1 = r[8 * s + 2 * k + 1];
+                rh[s].u[k] = bf16_pair(e0, e1);
+                rl[s].u[k] = bf16_pair(e0 - lo_half(rh[s].u[k]), e1 - hi_half(rh[s].u[k]));
+            }
+        // ---- projections: lane g holds signs [32 g, 32 g + 32)
+        uint32_t sb = 0u, amb = 0u;
+        const float mg = eps * rho;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            f32x4 p = {0.0f, 0.0f, 0.0f, 0.0f};
+            Frag m;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                m.q = s_s[((t * 4 + s) * 2 + 1) * 64 + lane];
+                p = mfma_bf16(m, rh[s], p);
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                m.q = s_s[(t * 4 + s) * 2 * 64 + lane];
+                p = mfma_bf16(m, rl[s], p);
+                p = mfma_bf16(m, rh[s], p);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                sb |= (p[i] >= 0.0f ? 1u : 0u) << (4 * t + i);
+                amb |= (!(fabsf(p[i]) >= mg) ? 1u : 0u) << (4 * t + i);
+            }
+        }
+        // every r of magnitude 0: the projections are +0 in the chain too.  Otherwise, with squares that
+        // vanish, the chain decides.
+        uint32_t nz = 0u;
+#pragma unroll
+        for (int k = 0; k < 32; ++k) nz |= __float_as_uint(r[k]);
+        nz &= 0x7FFFFFFFu;
+        nz |= (uint32_t)__shfl_xor((int)nz, 16);
+        nz |= (uint32_t)__shfl_xor((int)nz, 32);
+        if (tiny) {
+            amb = nz ? 0xFFFFFFFFu : 0u;
+            if (!nz) sb = 0xFFFFFFFFu;
+        }
+        if (bad) amb = 0xFFFFFFFFu;
+        amb &= valid;
+        if (!live) amb = 0u, rho_amb = false;
+
+        uint32_t todo = fold_vectors(__builtin_amdgcn_ballot_w64(amb != 0u || rho_amb));
+        uint32_t rho16 = tq::f32_to_f16(rho);
+        while (todo) {  // uniform: one vector at a time, its residual in LDS
+            const int vv = __builtin_ctz(todo);
+            todo &= todo - 1u;
+            float4* sr = s_r[wave][0];
+            float4* sh = s_r[wave][1];
+            wave_lds_fence();
+            if (v == vv) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    sr[8 * g + k] = make_float4(r[4 * k], r[4 * k + 1], r[4 * k + 2], r[4 * k + 3]);
+            }
+            wave_lds_fence();
+            float ss = 0.0f;
+#pragma unroll 8
+            for (int k = 0; k < D / 4; ++k) {
+                const float4 e = sr[k];
+                ss = __builtin_fmaf(e.x, e.x, ss);
+                ss = __builtin_fmaf(e.y, e.y, ss);
+                ss = __builtin_fmaf(e.z, e.z, ss);
+                ss = __builtin_fmaf(e.w, e.w, ss);
+            }
+            float rx = tq::sqrt_rn(ss);
+            if (!(rx > 0.0f)) rx = 1.0f;
+            if (v == vv) rho16 = tq::f32_to_f16(rx);
+            uint32_t aw[4], any = 0u;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                aw[k] = (uint32_t)__builtin_amdgcn_readlane((int)amb, vv + 16 * k);
+                any |= aw[k];
+            }
+            if (!any) continue;
+            float* fr = reinterpret_cast<float*>(sr);
+            float* fh = reinterpret_cast<float*>(sh);
+            fh[lane] = tq::div_rn(fr[lane], rx);
+            fh[lane + 64] = tq::div_rn(fr[lane + 64], rx);
+            wave_lds_fence();
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const uint32_t mine_w = lane < 32 ? aw[2 * half] : aw[2 * half + 1];
+                const bool need = (mine_w >> (lane & 31)) & 1u;
+                bool pos = false;
+                if (need) {
+                    const float4* si = reinterpret_cast<const float4*>(a.S) + (64 * half + lane) * (D / 4);
+                    float p = 0.0f;
+#pragma unroll 8
+                    for (int k = 0; k < D / 4; ++k) {
+                        const float4 e = sh[k], c = si[k];
+                        p = __builtin_fmaf(e.x, c.x, p);
+                        p = __builtin_fmaf(e.y, c.y, p);
+                        p = __builtin_fmaf(e.z, c.z, p);
+                        p = __builtin_fmaf(e.w, c.w, p);
+                    }
+                    pos = p >= 0.0f;
+                }
+                const uint64_t bits = __builtin_amdgcn_ballot_w64(pos);
+                if (v == vv && (g >> 1) == half)
+                    sb = (sb & ~amb) | ((uint32_t)(bits >> (32 * (g & 1))) & amb);
+            }
+        }
+        if (live) {
+            if (g == 0) a.rnorms[slot] = (uint16_t)rho16;
+            if constexpr (!GROUP) {
+                reinterpret_cast<uint32_t*>(a.signs + slot * (D / 8))[g] = sb;
+            } else {
+                sb &= valid;
+                uint8_t* dst = a.signs + slot * sign_bytes + 4 * g;
+                const int left = sign_bytes - 4 * g;
+                if (left >= 4) {
+                    __builtin_memcpy(dst, &sb, 4);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 3; ++e)
+                        if (e < left) dst[e] = (uint8_t)(sb >> (8 * e));
+                }
+            }
+        }
+    }
+}
+
+// Workgroups of a kernel that fit on the device at once (each loops over tiles, so more would only
+// repeat the LDS set-up).
+template <auto KERNEL>
+int64_t resident() {
+    static std::atomic<int64_t> cached[tq::MAX_DEVICES];
+    return tq::once_per_device(cached, 256, [](int dev) {
+        int cus = 0, per_cu = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, KERNEL, MQ_THREADS, 0) != hipSuccess || per_cu < 1)
+            per_cu = 1;
+        return (int64_t)cus * per_cu;
+    });
+}
+
+template <auto KERNEL>
+int launch(const EncodeArgs& a, int64_t items, hipStream_t s) {
+    const int64_t groups = std::min<int64_t>((items + MQ_WAVES - 1) / MQ_WAVES, resident<KERNEL>());
+    hipLaunchKernelGGL(KERNEL, dim3((unsigned)groups), dim3(MQ_THREADS), 0, s, a);
+    TQ_CHECK_LAUNCH();
+    return TQ_OK;
+}
+
+template <int BITS, bool GROUP>
+int encode(const EncodeArgs& a, hipStream_t s) {
+    const int64_t tiles = (a.n_vec + 15) / 16;
+    // four tiles per wave share each matrix fragment read from LDS; a call with fewer tiles than the
+    // device has waves spreads them instead
+    const int64_t waves = resident<codes_kernel<BITS, GROUP, 4>>() * MQ_WAVES;
+    const int st = tiles >= 2 * waves ? launch<codes_kernel<BITS, GROUP, 4>>(a, (tiles + 3) / 4, s)
+                                      : launch<codes_kernel<BITS, GROUP, 1>>(a, tiles, s);
+    if (st != TQ_OK || !a.S) return st;
+    if constexpr (GROUP || BITS <= 3) return launch<residual_kernel<BITS, GROUP>>(a, tiles, s);
+    return TQ_ERR_INVALID_ARGUMENT;
+}
+
+}  // namespace
+
+namespace tqenc {
+
+int launch_encode(EncodeArgs a, int bits, bool group, hipStream_t s) {
+    a.tok_div = make_fastdiv((uint32_t)a.tokens);
+    a.head_div = make_fastdiv((uint32_t)a.heads);
+    if (!group) {
+        switch (bits) {
+            case 1: return encode<1, false>(a, s);
+            case 2: return encode<2, false>(a, s);
+            case 3: return encode<3, false>(a, s);
+            case 4: return encode<4, false>(a, s);
+            default: return TQ_ERR_INVALID_ARGUMENT;
+        }
+    }
+    switch (bits) {
+        case 1: return encode<1, true>(a, s);
+        case 2: return encode<2, true>(a, s);
+        case 3: return encode<3, true>(a, s);
+        case 4: return encode<4, true>(a, s);
+        case 5: return encode<5, true>(a, s);
+        case 6: return encode<6, true>(a, s);
+        case 7: return encode<7, true>(a, s);
+        case 8: return encode<8, true>(a, s);
+        default: return TQ_ERR_INVALID_ARGUMENT;
+    }
+}
+
+}  // namespace tqenc

@@ -9,8 +9,8 @@
 // (:498-515, :456-479) decode each group (:404-435, :312-330) and scatter it back
 // into the full row.
 //
-// The kernels never gather.  One lane owns one token vector and holds the whole
-// 128-channel row with the channels outside the group set to zero; the group's d x d
+// The kernels never gather.  They hold the whole 128-channel row of a token vector
+// with the channels outside the group set to zero; the group's d x d
 // matrices arrive in channel space (tq_group_matrix: row j < d carries the group
 // matrix row j at the group's channels, every other entry 0).  Every fp32 reduction is
 // an fma chain over the channels in ascending order, the group's channels ascend, and
@@ -20,21 +20,20 @@
 // therefore bit-identical to the plain encoder / decoder run at D = d on the gathered
 // sub-vectors, which is how the CPU oracle states them.
 //
-// The decoder of groups wider than 24 channels runs on the fp32 matrix cores instead
-// (dequantize_group_mfma_kernel below, with the chains of tq_mfma.h): same chains, same
-// bits.
+// Calls of at least GQ_SMALL vectors take the prefill encoder of tq_encode.hip.  The decoder of
+// groups up to 24 channels holds a vector per lane; wider ones run on the fp32 matrix cores
+// (dequantize_group_mfma_kernel below, with the chains of tq_mfma.h): same chains, same bits.
 //
 // Packed rows are ceil(d*bits/8) code bytes and ceil(d/8) sign bytes per token, LSB
-// first, zero padded (runtime/packed_qmse_cache.py:13-43, 148-154); lanes write them
-// byte by byte, so no alignment is required of those buffers.
+// first, zero padded (runtime/packed_qmse_cache.py:13-43, 148-154); no alignment is required
+// of those buffers.
 
 #include <math.h>
 
 #include <algorithm>
 #include <type_traits>
 
-#include "tq_common.h"
-#include "tq_mfma.h"
+#include "tq_encode.h"
 
 namespace {
 
@@ -50,20 +49,6 @@ struct ChanMask {
 
 __device__ __forceinline__ bool in_group(const ChanMask& m, int c) { return (m.w[c >> 5] >> (c & 31)) & 1u; }
 
-// Channels 8i..8i+7 of the lane's row, those outside the group zeroed, bf16 -> fp32.
-__device__ __forceinline__ void load_masked8(const uint16_t* xv, int i, const ChanMask& m, float* o) {
-    const uint4 w = reinterpret_cast<const uint4*>(xv)[i];
-    const uint32_t h[8] = {w.x & 0xFFFFu, w.x >> 16, w.y & 0xFFFFu, w.y >> 16,
-                           w.z & 0xFFFFu, w.z >> 16, w.w & 0xFFFFu, w.w >> 16};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) o[k] = in_group(m, 8 * i + k) ? tq::bf16_to_f32(h[k]) : 0.0f;
-}
-
-__device__ __forceinline__ void load_masked(const uint16_t* xv, const ChanMask& m, float* o) {
-#pragma unroll
-    for (int i = 0; i < D / 8; ++i) load_masked8(xv, i, m, o + 8 * i);
-}
-
 // #{i : b[i] < z} (torch.bucketize right=False) by binary search over the sorted
 // boundaries in LDS: the predicate holds on a prefix, `bits` probes.
 __device__ __forceinline__ uint32_t bucket_lds(float z, const float* s_b, int bits) {
@@ -72,125 +57,10 @@ __device__ __forceinline__ uint32_t bucket_lds(float z, const float* s_b, int bi
     return c;
 }
 
-// LSB-first bit stream written byte by byte into the lane's own row.
-struct ByteWriter {
-    uint8_t* dst;
-    uint32_t acc = 0;
-    int fill = 0;
-    __device__ __forceinline__ explicit ByteWriter(uint8_t* d) : dst(d) {}
-    __device__ __forceinline__ void put(uint32_t v, int nbits) {  // nbits <= 8: at most one byte
-        acc |= v << fill;
-        fill += nbits;
-        if (fill >= 8) {
-            *dst++ = (uint8_t)acc;
-            acc >>= 8;
-            fill -= 8;
-        }
-    }
-    __device__ __forceinline__ void flush() {
-        if (fill > 0) *dst = (uint8_t)acc;
-    }
-};
-
-template <bool PROD>
-__global__ __launch_bounds__(GBLOCK) void quantize_group_kernel(
-    const uint16_t* __restrict__ x, int heads, int64_t tokens, int64_t n_vec, int64_t x_sb, int64_t x_sh,
-    int64_t x_st, ChanMask mask, int sub_dim, int bits, const float* __restrict__ R,
-    const float* __restrict__ centers, const float* __restrict__ boundaries, const float* __restrict__ S,
-    uint8_t* __restrict__ codes, uint16_t* __restrict__ norms, uint8_t* __restrict__ signs,
-    uint16_t* __restrict__ rnorms, int64_t out_cap, int64_t out_offset) {
-    __shared__ float s_bound[(1 << MAX_BITS) - 1];
-    __shared__ float s_centers[PROD ? (1 << MAX_BITS) : 1];
-    __shared__ uint8_t s_code[PROD ? D : 1][GBLOCK];  // PROD: codes of each lane, column per lane
-    const int nb = (1 << bits) - 1;
-    for (int i = threadIdx.x; i < nb; i += GBLOCK) s_bound[i] = boundaries[i];
-    if (PROD)
-        for (int i = threadIdx.x; i <= nb; i += GBLOCK) s_centers[i] = centers[i];
-    __syncthreads();
-
-    const int64_t v = (int64_t)blockIdx.x * GBLOCK + threadIdx.x;
-    if (v >= n_vec) return;  // no barrier below this point
-    const int64_t t = v % tokens;
-    const int64_t gh = v / tokens;
-    const int64_t h = gh % heads;
-    const int64_t b = gh / heads;
-    const uint16_t* xv = x + b * x_sb + h * x_sh + t * x_st;
-    const int64_t slot = gh * out_cap + out_offset + t;
-
-    // ---- norm and direction of the group's sub-vector
-    float u[D];
-    load_masked(xv, mask, u);
-    float ss = 0.0f;
-#pragma unroll
-    for (int d = 0; d < D; ++d) ss = __builtin_fmaf(u[d], u[d], ss);
-    float n = tq::sqrt_rn(ss);
-    if (!(n > 0.0f)) n = 1.0f;
-#pragma unroll
-    for (int d = 0; d < D; ++d) u[d] = tq::div_rn(u[d], n);
-    const uint32_t n16 = tq::f32_to_f16(n);
-    norms[slot] = (uint16_t)n16;
-
-    // ---- rotate (rows j < d), bucketize, pack
-    ByteWriter bw(codes + slot * (int64_t)((sub_dim * bits + 7) >> 3));
-    for (int j = 0; j < sub_dim; ++j) {
-        const float* rj = R + j * D;
-        float z = 0.0f;
-#pragma unroll
-        for (int d = 0; d < D; ++d) z = __builtin_fmaf(u[d], rj[d], z);
-        const uint32_t c = bucket_lds(z, s_bound, bits);
-        bw.put(c, bits);
-        if (PROD) s_code[j][threadIdx.x] = (uint8_t)c;
-    }
-    bw.flush();
-
-    if constexpr (PROD) {
-        // ---- residual decode khat = bf16((C[code] @ R) * f32(f16(n))), rows j < d
-        float* acc = u;  // u is dead after the rotation
-#pragma unroll
-        for (int d = 0; d < D; ++d) acc[d] = 0.0f;
-        for (int j = 0; j < sub_dim; ++j) {
-            const float cj = s_centers[s_code[j][threadIdx.x]];
-            const float* rj = R + j * D;
-#pragma unroll
-            for (int d = 0; d < D; ++d) acc[d] = __builtin_fmaf(cj, rj[d], acc[d]);
-        }
-        const float nf = tq::f16_to_f32(n16);
-        __asm__ volatile("" ::: "memory");  // x is re-read here, 16 bytes at a time, not held
-        float rs = 0.0f;
-#pragma unroll
-        for (int i = 0; i < D / 8; ++i) {
-            float xr[8];
-            load_masked8(xv, i, mask, xr);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int d = 8 * i + k;
-                const float kh = tq::bf16_to_f32(tq::f32_to_bf16(acc[d] * nf));
-                acc[d] = xr[k] - kh;  // 0 - 0 outside the group: R's columns there are zero
-                rs = __builtin_fmaf(acc[d], acc[d], rs);
-            }
-        }
-        float rho = tq::sqrt_rn(rs);
-        if (!(rho > 0.0f)) rho = 1.0f;
-#pragma unroll
-        for (int d = 0; d < D; ++d) acc[d] = tq::div_rn(acc[d], rho);
-        rnorms[slot] = (uint16_t)tq::f32_to_f16(rho);
-        ByteWriter sw(signs + slot * (int64_t)((sub_dim + 7) >> 3));
-        for (int i = 0; i < sub_dim; ++i) {
-            const float* si = S + i * D;
-            float p = 0.0f;
-#pragma unroll
-            for (int d = 0; d < D; ++d) p = __builtin_fmaf(acc[d], si[d], p);
-            sw.put(p >= 0.0f ? 1u : 0u, 1);
-        }
-        sw.flush();
-    }
-}
-
 // Decode-append sizes (below GQ_SMALL vectors): a workgroup encodes GAV vectors with D threads
 // each.  Thread (v, j) runs output j's chains of vector v -- z_j and p_j for j < d, khat_j for
 // every channel j -- and every thread of a vector runs the two norm chains over the masked row
-// held in LDS (the same operands in the same order: one value in all of them).  These are the
-// lane kernel's chains term for term, so the outputs are bit-identical to it.  The channel-space
+// held in LDS (the same operands in the same order: one value in all of them).  The channel-space
 // matrices are staged in LDS with a row stride of GMS = 132 floats (rows read 16 bytes at a time
 // and columns read one float at a time both spread over the banks).
 constexpr int GAV = 4;                 // vectors per workgroup
@@ -459,7 +329,7 @@ extern "C" int tq_quantize_group(const uint16_t* x, int batch, int heads, int64_
     if (n_vec == 0) return TQ_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (!aligned16(rotation) || (prod && !aligned16(qjl))) return TQ_ERR_UNSUPPORTED;
-    if (n_vec < GQ_SMALL) {
+    if (n_vec < GQ_SMALL || n_vec >= ((int64_t)1 << 31)) {
         const int64_t sblocks = (n_vec + GAV - 1) / GAV;
         if (prod)
             hipLaunchKernelGGL((quantize_group_small_kernel<true>), dim3((unsigned)sblocks), dim3(GAT), 0, s, x,
@@ -472,17 +342,10 @@ extern "C" int tq_quantize_group(const uint16_t* x, int batch, int heads, int64_
         TQ_CHECK_LAUNCH();
         return TQ_OK;
     }
-    const int64_t blocks = (n_vec + GBLOCK - 1) / GBLOCK;
-    if (prod)
-        hipLaunchKernelGGL((quantize_group_kernel<true>), dim3((unsigned)blocks), dim3(GBLOCK), 0, s, x, heads,
-                           tokens, n_vec, x_sb, x_sh, x_st, mask, sub_dim, bits, rotation, centers, boundaries, qjl,
-                           codes, norms, signs, rnorms, out_cap, out_offset);
-    else
-        hipLaunchKernelGGL((quantize_group_kernel<false>), dim3((unsigned)blocks), dim3(GBLOCK), 0, s, x, heads,
-                           tokens, n_vec, x_sb, x_sh, x_st, mask, sub_dim, bits, rotation, nullptr, boundaries,
-                           nullptr, codes, norms, nullptr, nullptr, out_cap, out_offset);
-    TQ_CHECK_LAUNCH();
-    return TQ_OK;
+    return tqenc::launch_encode({x, heads, tokens, n_vec, x_sb, x_sh, x_st, rotation, centers, boundaries, qjl, codes, norms,
+                                 signs, rnorms, out_cap, out_offset, {mask.w[0], mask.w[1], mask.w[2], mask.w[3]},
+                                 sub_dim, {}, {}},
+                                bits, true, s);
 }
 
 namespace {
