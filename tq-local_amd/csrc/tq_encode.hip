@@ -4,16 +4,17 @@
 // bucket of an fma chain over 128 dims, a sign the sign of one.  Running those chains costs 32
 // v_mfma_f32_16x16x4_f32 (1024 cycles) per 16 x 16 outputs, at the fp32 rate, and nothing else can
 // use the SIMD meanwhile.  But a bucket only needs its chain when the value is close to a boundary.
-// So the products run on the bf16 matrix cores (3 x 4 instructions of 16 cycles; the bf16 input is
-// exact, the matrix enters as three bf16 terms that add up to it), the value z' comes with a
-// bound eps on its distance from the chain's z, and
+// So the products run on the bf16 matrix cores (2 x 4 instructions of 16 cycles; the bf16 input is
+// exact, the matrix enters as two bf16 terms), the value z' comes with a bound eps on its distance
+// from the chain's z, and
 //   |z' - b| >= eps for the one boundary b in reach:  the bucket of z' is the bucket of z;
-//   otherwise (about one output in 1000): the chain itself is run for that output.
+//   otherwise (one output in 800 at 4 bits, in 1600 at 3): the chain itself is run for that output.
 // The results are the chain's, bit for bit; only which outputs need it is decided by bounds.
 //
 // The bound, for rows of norm <= r and a vector of norm n (u = x / n has norm 1 up to 2^-20):
 //   the chain: 128 roundings, each at most 2^-24 of a partial sum, which Cauchy-Schwarz keeps
 //     below r: 7.63e-6 r, and u's own rounding 2^-24 r;
+//   the matrix's terms (nearest even) leave 2^-18 of each entry: 3.8e-6 r;
 //   z': the matrix instruction sums groups of 8 products aligned to the group's largest at 2^-24
 //     of it, and rounds after each group (probed: products below that are cut off, the sum of a
 //     group meets the accumulator with one rounding).  Over the groups of the leading term that is
@@ -41,31 +42,35 @@ namespace {
 using namespace tqmx;
 using tqenc::EncodeArgs;
 constexpr int D = TQ_DIM;
-constexpr int QPAIRS = 192;    // outputs waiting in a wave's queue
+constexpr int CW = 12;          // waves per workgroup of the codes kernel
+constexpr int CT = 64 * CW;
 constexpr uint32_t NORM_ONLY = 255;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 union Frag {
     uint32_t u[4];
     uint4 q;
+    u32x4 w;
     bf16x8 b;
 };
 __device__ __forceinline__ f32x4 mfma_bf16(const Frag& a, const Frag& b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, b.b, c, 0, 0, 0);
 }
-// fp32 -> bf16, nearest even (v_cvt_pk_bf16_f32: the bits of tq::f32_to_bf16 for every input).
+// fp32 -> bf16, nearest even (v_cvt_pk_bf16_f32: the bits of tq::f32_to_bf16 for all 2^32 inputs).
 __device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    const bf16x2 p = {(__bf16)a, (__bf16)b};
-    return __builtin_bit_cast(uint32_t, p);
+    const f32x2 p = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2));
 }
 __device__ __forceinline__ float lo_half(uint32_t p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float hi_half(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
-// Truncated bf16 terms of two floats: a - hi is exact, and two truncations leave 8 bits.
-__device__ __forceinline__ uint32_t top_halves(float a, float b) {
-    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+// a.lo b.lo + a.hi b.hi + c over bf16 pairs; within 3 * 2^-24 of the sum (positive terms; probed).
+__device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), c, false);
 }
-__device__ __forceinline__ float below_top(float a) { return a - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u); }
 
 // The wave's LDS accesses complete in issue order; this keeps the compiler from moving them.
 __device__ __forceinline__ void wave_lds_fence() {
@@ -111,36 +116,42 @@ __device__ __forceinline__ uint32_t bucket_lds(float z, const float* s_b, int bi
 // ------------------------------------------------------------------ codes and norms
 // Bucketize through a uniform grid.  Cells of width w = (smallest gap between neighbouring
 // boundaries) / 4 start at e0 = b_0 - 2w; cell k holds c0 = #{i : b_i < e0 + (k - 1) w} and b_{c0}.
-// z' goes to the cell k = clamp(floor((z' - e0) / w)); the quotient is computed within 1e-3
-// (|e0| / w and |b_NB-1| / w stay below 4096) and z' is within w / 16 of z (eps < w / 16 or the grid is
-// not used), so z lies in (e0 + (k - 1.1) w, e0 + (k + 2.1) w), a window of 3.2 w that holds at most one
-// boundary (the gap is 4w), b_{c0} if any: code(z) = c0 + [b_{c0} < z].  The clamped ends: the first
-// cell is 2w below b_0, the last more than w above b_NB-1, where b is a number above all z.  A cell is
-// one word, the boundary with its low `bits` bits replaced by c0.
+// z' goes to the cell k = clamp(floor(q)), q the quotient (z' - e0) / w, computed within 1/8 (rounded
+// to quarters) + 1e-3 (|e0| / w and |b_NB-1| / w stay below 4096); z' is within w / 16 of z (eps < w / 16
+// or the grid is not used).  So z lies in (e0 + (k - 0.2) w, e0 + (k + 1.2) w): every b_i below
+// e0 + (k - 1) w is below z, b_{c0 + 1} >= b_{c0} + 4w is above it, and b_{c0} decides:
+// code(z) = c0 + [b_{c0} < z].  The clamped ends: the first cell is 2w below b_0, the last more than w
+// above b_NB-1, where b is a number above all z.  A cell is one word, the boundary with its low
+// `bits` bits replaced by c0.
 template <int BITS, bool GROUP, int NT>
-__global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
+__global__ __launch_bounds__(CT) void codes_kernel(EncodeArgs a) {
     constexpr int NB = (1 << BITS) - 1;
     constexpr int RW = 4 * BITS;  // dwords of a plain row; a queued row holds 32 codes per lane, BITS words
     constexpr uint32_t CMASK = NB;
     constexpr int LUT_MAX = BITS <= 6 ? 512 : 2048;  // cells of the bucketize grid
-    constexpr int QROWS = BITS <= 6 ? 48 : 32;       // vectors waiting in a wave's queue
-    __shared__ uint4 s_img[8 * 4 * 3 * 64];  // [row tile][k-step][term][lane]
-    __shared__ float s_lut[LUT_MAX];
-    __shared__ float s_bound[NB];
-    __shared__ uint32_t s_max;
-    __shared__ uint32_t s_row[MQ_WAVES][QROWS][RW];
-    __shared__ uint32_t s_vec[MQ_WAVES][QROWS];
-    __shared__ uint32_t s_pair[MQ_WAVES][QPAIRS];
+    // a wave's queue: vectors waiting, and single outputs; the next item may bring 16 NT and 64
+    constexpr int QROWS = BITS <= 4 ? 96 : BITS <= 6 ? 64 : 48;
+    constexpr int QPAIRS = 128;
+    __shared__ struct {
+        float lut[LUT_MAX];  // first, in reach of a read's immediate offset
+        float bound[NB];
+        uint32_t r_max;
+        uint32_t row[CW][QROWS][RW];
+        uint32_t vec[CW][QROWS];
+        uint32_t pair[CW][QPAIRS];
+        uint32_t all[CW][QROWS];
+        uint4 img[8 * 4 * 2 * 64];  // [row tile][k-step][term][lane]
+    } sh;
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int v = lane & 15, g = lane >> 4;
     const int sub_dim = GROUP ? a.sub_dim : D;
-    if (threadIdx.x == 0) s_max = 0u;
-    for (int i = threadIdx.x; i < NB; i += MQ_THREADS) s_bound[i] = a.boundaries[i];
+    if (threadIdx.x == 0) sh.r_max = 0u;
+    for (int i = threadIdx.x; i < NB; i += CT) sh.bound[i] = a.boundaries[i];
     __syncthreads();
-    // ---- the matrix as three bf16 terms: index j = 32 q + 4 t + i is row 4 q + i of tile t, so that
+    // ---- the matrix as two bf16 terms: index j = 32 q + 4 t + i is row 4 q + i of tile t, so that
     // lane 16 q + v ends with the codes [32 q, 32 q + 32) of its vector
-    for (int idx = threadIdx.x; idx < D * D / 8; idx += MQ_THREADS) {
+    for (int idx = threadIdx.x; idx < D * D / 8; idx += CT) {
         const int j = idx >> 4, c = idx & 15;  // dims 8 c .. 8 c + 7
         float e[8];
         if (!GROUP || j < sub_dim) {
@@ -154,65 +165,75 @@ __global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
         float part = 0.0f;
 #pragma unroll
         for (int k = 0; k < 8; ++k) part = __builtin_fmaf(e[k], e[k], part);
-        row_norm_max(&s_max, part);
+        row_norm_max(&sh.r_max, part);
         const int t = (j >> 2) & 7, m = 4 * (j >> 5) + (j & 3), s = c >> 2, l = 16 * (c & 3) + m;
-        uint4* dst = s_img + (t * 4 + s) * 3 * 64 + l;
+        uint32_t hi[4], lo[4];
 #pragma unroll
-        for (int term = 0; term < 3; ++term) {
-            uint32_t w[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                w[k] = top_halves(e[2 * k], e[2 * k + 1]);
-                e[2 * k] = below_top(e[2 * k]);
-                e[2 * k + 1] = below_top(e[2 * k + 1]);
-            }
-            dst[term * 64] = make_uint4(w[0], w[1], w[2], w[3]);
+        for (int k = 0; k < 4; ++k) {
+            hi[k] = bf16_pair(e[2 * k], e[2 * k + 1]);
+            lo[k] = bf16_pair(e[2 * k] - lo_half(hi[k]), e[2 * k + 1] - hi_half(hi[k]));
+        }
+        sh.img[((t * 4 + s) * 2 + 0) * 64 + l] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        sh.img[((t * 4 + s) * 2 + 1) * 64 + l] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    }
+    // ---- bucket grid: one lane per gap between boundaries
+    float gap = __builtin_inff(), b_max = 0.0f;
+    bool sorted = true;
+    for (int i = lane; i < NB; i += 64) {
+        b_max = fmaxf(b_max, fabsf(sh.bound[i]));
+        if (i > 0) {
+            const float d = sh.bound[i] - sh.bound[i - 1];
+            sorted = sorted && d > 0.0f;
+            gap = fminf(gap, d);
         }
     }
-    // ---- bucket grid
-    float gap = __builtin_inff();
-    bool sorted = true;
-    for (int i = 1; i < NB; ++i) {
-        const float d = s_bound[i] - s_bound[i - 1];
-        sorted = sorted && d > 0.0f;
-        gap = fminf(gap, d);
+    sorted = __all(sorted);
+#pragma unroll
+    for (int k = 1; k < 64; k <<= 1) {
+        gap = fminf(gap, __shfl_xor(gap, k));
+        b_max = fmaxf(b_max, __shfl_xor(b_max, k));
     }
     __syncthreads();
-    const float r_norm = __builtin_sqrtf(__uint_as_float(s_max)) * 1.0001f;
-    float b_max = 0.0f;
-    for (int i = 0; i < NB; ++i) b_max = fmaxf(b_max, fabsf(s_bound[i]));
-    const float eps = r_norm * 9.5e-6f + (b_max + 1e-4f * r_norm) * (6.5e-6f + (float)(1 << BITS) * 1.2e-7f);
+    const float r_norm = __builtin_sqrtf(__uint_as_float(sh.r_max)) * 1.0001f;
+    const float eps = r_norm * 1.33e-5f + (b_max + 1e-4f * r_norm) * (6.5e-6f + (float)(1 << BITS) * 1.2e-7f);
     const float w = NB > 1 ? gap * 0.25f : 1.0f;
-    const float e0 = s_bound[0] - 2.0f * w;
-    const float span = (s_bound[NB - 1] - e0) / w;
+    const float e0 = sh.bound[0] - 2.0f * w;
+    const float span = (sh.bound[NB - 1] - e0) / w;
     const float g_scale = 1.0f / w;
     const float g_off = -e0 * g_scale;
     // outside the bounds' range every output takes its chain
     const bool exact_all = !(r_norm < 1e18f) || !(b_max < 1e18f);
     const bool use_grid = sorted && w > 16.0f * eps && span < (float)(LUT_MAX - 5) && fabsf(g_off) < 4096.0f &&
-                          fabsf(s_bound[NB - 1] * g_scale) < 4096.0f;
+                          fabsf(sh.bound[NB - 1] * g_scale) < 4096.0f;
     const int cells = use_grid ? (int)ceilf(span) + 4 : 0;
-    for (int k = threadIdx.x; k < cells; k += MQ_THREADS) {
+    for (int k = threadIdx.x; k < cells; k += CT) {
         const float start = e0 + (float)(k - 1) * w;
         uint32_t c0 = 0;
-        for (int i = 0; i < NB; ++i) c0 += s_bound[i] < start ? 1u : 0u;
-        const float b = c0 < NB ? s_bound[c0] + 0.0f : 3e38f;
-        s_lut[k] = __uint_as_float((__float_as_uint(b) & ~CMASK) | c0);
+        for (int i = 0; i < NB; ++i) c0 += sh.bound[i] < start ? 1u : 0u;
+        const float b = c0 < NB ? sh.bound[c0] + 0.0f : 3e38f;
+        sh.lut[k] = __uint_as_float((__float_as_uint(b) & ~CMASK) | c0);
     }
     __syncthreads();  // the last barrier: each wave then works on its own tiles
 
-    // f = cell + 2^23 in the low bits of a float: one fma and one med3, and the bits are the index
+    // f = 4 * quotient + 2^23: one fma and one med3, and the low bits of f are the quotient's, in
+    // quarters of a cell: without the last two, the byte offset of its word
     constexpr float MAGIC = 8388608.0f;
-    const float f_off = g_off + (MAGIC - 0.5f);
-    const float f_top = MAGIC + (float)(cells - 1);
-    const float s_b0 = s_bound[0];
+    const float q_scale = 4.0f * g_scale;
+    const float f_off = 4.0f * g_off + MAGIC;
+    const float f_top = MAGIC + (float)(4 * cells - 1);
+    const float s_b0 = sh.bound[0];
     const uint32_t mw[4] = {a.mask[0], a.mask[1], a.mask[2], a.mask[3]};
     const int row_bytes = GROUP ? (sub_dim * BITS + 7) >> 3 : D * BITS / 8;
     // this lane's outputs 32 g + jj with jj < mine count
     const int mine = GROUP ? std::min(std::max(sub_dim - 32 * g, 0), 32) : 32;
-    const int n_t = GROUP && sub_dim < 32 ? (sub_dim + 3) >> 2 : 8;
+    const int n_t = a.sub_dim < 32 ? (a.sub_dim + 3) >> 2 : 8;
 
-    uint32_t q_rows = 0, q_pairs = 0;  // wave-uniform
+    // this lane's fragments, all in reach of a read's immediate offset
+    typedef __attribute__((address_space(3))) const u32x4* LdsFrags;
+    LdsFrags img = (LdsFrags)(sh.img + lane);
+    __asm__("" : "+v"(img));
+
+    uint32_t q_rows = 0, q_pairs = 0, q_all = 0;  // wave-uniform
     auto store_row = [&](uint8_t* codes, const uint32_t* words) {  // this lane's BITS words of a row
         if constexpr (!GROUP) {
             uint32_t* dst = reinterpret_cast<uint32_t*>(codes) + BITS * g;
@@ -237,15 +258,27 @@ __global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
             }
         }
     };
-    // the queued outputs' chains, one lane each
-    auto run_pairs = [&]() {
+    // The queue's chains: 64 single outputs at a time, one lane each, then the vectors whose every output
+    // is wanted, half a vector at a time; then the rows leave.
+    auto run_queue = [&]() {
         wave_lds_fence();
-        for (uint32_t base = 0; base < q_pairs; base += 64) {
-            if (base + lane < q_pairs) {
-                const uint32_t e = s_pair[wave][base + lane], qr = e >> 8, j = e & 255u;
-                const uint32_t vi = s_vec[wave][qr];
+        const uint32_t singles = (q_pairs + 63) >> 6, batches = singles + 2 * q_all;
+        for (uint32_t batch = 0; batch < batches; ++batch) {
+            const bool whole = batch >= singles;
+            uint32_t qr = 0, j = 0;
+            bool act;
+            if (whole) {
+                qr = sh.all[wave][(batch - singles) >> 1];
+                j = 64 * ((batch - singles) & 1) + lane;
+                act = !GROUP || (int)j < sub_dim;
+            } else {
+                act = 64 * batch + lane < q_pairs;
+                const uint32_t e = act ? sh.pair[wave][64 * batch + lane] : 0u;
+                qr = e >> 8, j = e & 255u;
+            }
+            if (act) {
                 int64_t slot;
-                const uint4* x4 = reinterpret_cast<const uint4*>(row_of(a, vi, &slot));
+                const uint4* x4 = reinterpret_cast<const uint4*>(row_of(a, sh.vec[wave][qr], &slot));
                 auto channels = [&](int c, float* o) {  // channels 8 c .. 8 c + 7, masked
                     const uint4 p = x4[c];
                     const uint32_t h[4] = {p.x, p.y, p.z, p.w};
@@ -258,7 +291,7 @@ __global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
                     }
                 };
                 float ss = 0.0f;
-#pragma unroll 4
+#pragma unroll 8
                 for (int c = 0; c < D / 8; ++c) {
                     float o[8];
                     channels(c, o);
@@ -267,9 +300,8 @@ __global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
                 }
                 float n = tq::sqrt_rn(ss);
                 if (!(n > 0.0f)) n = 1.0f;
-                if (j == NORM_ONLY) {
-                    a.norms[slot] = (uint16_t)tq::f32_to_f16(n);
-                } else {
+                if (j == NORM_ONLY || (whole && j == 0)) a.norms[slot] = (uint16_t)tq::f32_to_f16(n);
+                if (j != NORM_ONLY) {
                     const float4* rj = reinterpret_cast<const float4*>(a.R) + j * (D / 4);
                     float z = 0.0f;
 #pragma unroll 4
@@ -281,60 +313,74 @@ __global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
 #pragma unroll
                         for (int k = 0; k < 8; ++k) z = __builtin_fmaf(tq::div_rn(o[k], n), rr[k], z);
                     }
-                    const uint32_t code = bucket_lds(z, s_bound, BITS);
-                    uint32_t* row = s_row[wave][qr];
-                    const uint32_t bit = j * BITS, wi = bit >> 5, sh = bit & 31;
-                    uint64_t old = row[wi];
-                    if (sh + BITS > 32) old |= (uint64_t)row[wi + 1] << 32;
-                    const uint64_t diff = (uint64_t)(((uint32_t)(old >> sh) & CMASK) ^ code) << sh;
+                    const uint32_t code = bucket_lds(z, sh.bound, BITS);
+                    uint32_t* words = sh.row[wave][qr];
+                    const uint32_t bit = j * BITS, wi = bit >> 5, at = bit & 31;
+                    uint64_t old = words[wi];
+                    if (at + BITS > 32) old |= (uint64_t)words[wi + 1] << 32;
+                    const uint64_t diff = (uint64_t)(((uint32_t)(old >> at) & CMASK) ^ code) << at;
                     // other lanes may change other codes of the same word
-                    if ((uint32_t)diff) atomicXor(&row[wi], (uint32_t)diff);
-                    if ((uint32_t)(diff >> 32)) atomicXor(&row[wi + 1], (uint32_t)(diff >> 32));
+                    if ((uint32_t)diff) atomicXor(&words[wi], (uint32_t)diff);
+                    if ((uint32_t)(diff >> 32)) atomicXor(&words[wi + 1], (uint32_t)(diff >> 32));
                 }
             }
         }
-        q_pairs = 0;
         wave_lds_fence();
-    };
-    auto store_queued = [&]() {  // the waiting rows, their outputs run
         for (uint32_t r0 = 0; r0 < q_rows; r0 += 16) {
             const uint32_t qr = r0 + v;
             if (qr < q_rows) {
                 int64_t slot;
-                row_of(a, s_vec[wave][qr], &slot);
+                row_of(a, sh.vec[wave][qr], &slot);
                 uint32_t words[BITS];
 #pragma unroll
-                for (int k = 0; k < BITS; ++k) words[k] = s_row[wave][qr][BITS * g + k];
+                for (int k = 0; k < BITS; ++k) words[k] = sh.row[wave][qr][BITS * g + k];
                 store_row(a.codes + slot * row_bytes, words);
             }
         }
-        q_rows = 0;
+        q_rows = q_pairs = q_all = 0;
         wave_lds_fence();
     };
 
     const int64_t n_items = (a.n_vec + 16 * NT - 1) / (16 * NT);
-    for (int64_t item = (int64_t)blockIdx.x * MQ_WAVES + wave;; item += (int64_t)gridDim.x * MQ_WAVES) {
-        // past the last item the vectors are all dead: one more round to empty the queue
-        const bool last = item >= n_items;
-        // ---- NT tiles of 16 vectors: lane 16 g + v holds dims 32 s + 8 g + (0..7) of vector v, the B operand
+    // NT tiles of 16 vectors: lane 16 g + v holds dims 32 s + 8 g + (0..7) of vector v, the B operand.
+    // The next item's are read ahead: a wait for them does not wait for this item's stores.
+    Frag ahead[NT][4];
+    int64_t ahead_slot[NT];
+    auto read_ahead = [&](int64_t item) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const uint32_t vi = (uint32_t)item * (16u * NT) + 16u * n + (uint32_t)v;  // n_vec < 2^31
+            ahead_slot[n] = -1;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) ahead[n][s].q = make_uint4(0u, 0u, 0u, 0u);
+            if (item < n_items && vi < (uint64_t)a.n_vec) {
+                const uint4* x4 = reinterpret_cast<const uint4*>(row_of(a, vi, &ahead_slot[n]));
+#pragma unroll
+                for (int s = 0; s < 4; ++s) ahead[n][s].q = x4[4 * s + g];
+            }
+        }
+    };
+    // items go round over the workgroups first, so that a small call uses every CU
+    const int64_t stride = (int64_t)gridDim.x * CW;
+    int64_t item = (int64_t)wave * gridDim.x + blockIdx.x;
+    // stretches of items until the queue may not take the next one's, then the queue: nothing of an
+    // item is live while the queue runs
+    do {
+        read_ahead(item);
+        for (; item < n_items && q_rows + 16 * NT <= QROWS && q_pairs + 64 <= QPAIRS; item += stride) {
         Frag x[NT][4];
         int64_t slot[NT];
-        float rn[NT], mg[NT];
+        float rn[NT], rg[NT], mg[NT];
         bool live[NT];
         uint32_t n_amb = 0, special = 0;  // per tile bit: the fp16 norm, or everything, needs the chain
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
-            const uint32_t vi = (uint32_t)item * (16u * NT) + 16u * n + (uint32_t)v;  // n_vec < 2^31
-            live[n] = !last && vi < (uint64_t)a.n_vec;
-            slot[n] = 0;
+            slot[n] = ahead_slot[n];
+            live[n] = slot[n] >= 0;
 #pragma unroll
-            for (int s = 0; s < 4; ++s) x[n][s].q = make_uint4(0u, 0u, 0u, 0u);
-            if (live[n]) {
-                const uint4* x4 = reinterpret_cast<const uint4*>(row_of(a, vi, &slot[n]));
-#pragma unroll
-                for (int s = 0; s < 4; ++s) x[n][s].q = x4[4 * s + g];
-            }
+            for (int s = 0; s < 4; ++s) x[n][s] = ahead[n][s];
         }
+        read_ahead(item + stride);
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
             float ss = 0.0f;
@@ -345,8 +391,7 @@ __global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
                 for (int k = 0; k < 4; ++k) {
                     if constexpr (GROUP) x[n][s].u[k] &= pair_mask(mw[s] >> (8 * g), k);
                     const uint32_t p = x[n][s].u[k];
-                    ss = __builtin_fmaf(lo_half(p), lo_half(p), ss);
-                    ss = __builtin_fmaf(hi_half(p), hi_half(p), ss);
+                    ss = dot2_bf16(p, p, ss);
                     any |= p;
                 }
             ss += __shfl_xor(ss, 16);
@@ -357,6 +402,7 @@ __global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
             const bool zero = any == 0u;  // norm 1, every chain 0
             const float n_ = zero ? 1.0f : __builtin_sqrtf(ss);
             rn[n] = __builtin_amdgcn_rcpf(n_);
+            rg[n] = rn[n] * q_scale;
             mg[n] = zero ? -1.0f : eps;
             const bool bad = !zero && (!(ss > 1e-24f) || !(ss < 1e30f) || exact_all);
             const uint32_t h0 = tq::f32_to_f16(n_ * (1.0f - 7e-6f)), h1 = tq::f32_to_f16(n_ * (1.0f + 7e-6f));
@@ -365,7 +411,7 @@ __global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
             if (live[n] && g == 0 && !((n_amb >> n) & 1u)) a.norms[slot[n]] = (uint16_t)tq::f32_to_f16(n_);
         }
 
-        // ---- products, codes; bit 31 - jj of amb: output 32 g + jj needs its chain
+        // ---- products, codes; bit jj of amb: output 32 g + jj needs its chain
         uint32_t out[NT][BITS], amb[NT];
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
@@ -373,60 +419,96 @@ __global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
 #pragma unroll
             for (int k = 0; k < BITS; ++k) out[n][k] = 0u;
         }
-        auto emit = [&](int n, int jj, uint32_t code, bool close) {
-            amb[n] = amb[n] + amb[n] + (close ? 1u : 0u);
-            const int bit = jj * BITS, wi = bit >> 5, sh = bit & 31;
-            out[n][wi] |= code << sh;
-            if (sh + BITS > 32) out[n][wi + 1] |= code >> (32 - sh);
-        };
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            if (GROUP && t >= n_t) break;
-            f32x4 acc[NT];
+        auto products = [&](int t, f32x4* acc) {
 #pragma unroll
             for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int term = 2; term >= 0; --term)
+            for (int term = 1; term >= 0; --term)
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
                     Frag m;
-                    m.q = s_img[((t * 4 + s) * 3 + term) * 64 + lane];
+                    m.w = img[((t * 4 + s) * 2 + term) * 64];
 #pragma unroll
                     for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(m, x[n][s], acc[n]);
                 }
-            if (NB == 1 || use_grid) {
-#pragma unroll
-                for (int n = 0; n < NT; ++n)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        float b = s_b0;
-                        uint32_t code = 0u;
-                        if constexpr (NB > 1) {
-                            float f = __builtin_fmaf(acc[n][i], rn[n] * g_scale, f_off);
-                            f = __builtin_amdgcn_fmed3f(f, MAGIC, f_top);
-                            b = s_lut[__float_as_uint(f) & (LUT_MAX - 1)];
-                            code = __float_as_uint(b) & CMASK;
-                        }
-                        const float d = __builtin_fmaf(acc[n][i], rn[n], -b);
-                        emit(n, 4 * t + i, code + (d > 0.0f ? 1u : 0u), !(fabsf(d) >= mg[n]));
-                    }
-            } else {
-#pragma unroll
-                for (int n = 0; n < NT; ++n)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float z = acc[n][i] * rn[n];
-                        bool close = false;
-#pragma unroll 1
-                        for (int k = 0; k < NB; ++k) close = close || !(fabsf(z - s_bound[k]) >= mg[n]);
-                        emit(n, 4 * t + i, bucket_lds(z, s_bound, BITS), close);
-                    }
+        };
+        // the boundary in reach of a product: its low bits hold c0, the code below it
+        auto boundary = [&](int n, float acc) -> float {
+            if constexpr (NB == 1) {
+                return s_b0;
             }
-            __builtin_amdgcn_sched_barrier(0);  // not every tile's matrix fragments at once
-        }
-        if (GROUP && n_t < 8) {
+            float f = __builtin_fmaf(acc, rg[n], f_off);
+            f = __builtin_amdgcn_fmed3f(f, MAGIC, f_top);
+            return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(sh.lut) +
+                                                   (__float_as_uint(f) & (4 * LUT_MAX - 4)));
+        };
+        if ((NB == 1 || use_grid) && n_t == 8) {
+            // Products and buckets in turn, not interleaved: matrix and vector instructions of different
+            // waves overlap (61% of the shorter one with four waves on a SIMD, groups of 4 and 16),
+            // those of one wave hardly do (37% in groups of 1 and 4).
+            uint32_t ch[NT];  // codes enter at the top, the first ends lowest
 #pragma unroll
-            for (int n = 0; n < NT; ++n) amb[n] <<= 32 - 4 * n_t;
+            for (int n = 0; n < NT; ++n) ch[n] = 0u;
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                f32x4 acc[NT];
+                products(t, acc);
+                __builtin_amdgcn_sched_barrier(0);
+                float b[NT][4];
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) b[n][i] = boundary(n, acc[n][i]);
+#pragma unroll
+                for (int n = 0; n < NT; ++n) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float d = __builtin_fmaf(acc[n][i], rn[n], -b[n][i]);
+                        const uint32_t code = (NB > 1 ? __float_as_uint(b[n][i]) : 0u) + (d > 0.0f ? 1u : 0u);
+                        ch[n] = __builtin_amdgcn_alignbit(code, ch[n], BITS);
+                        amb[n] |= fabsf(d) < mg[n] ? 1u << (4 * t + i) : 0u;
+                    }
+                    const int bit = 4 * t * BITS, wi = bit >> 5, at = bit & 31;  // 4 codes from here on
+                    if constexpr (32 % BITS == 0) {
+                        if (((bit + 4 * BITS) & 31) == 0) out[n][wi] = ch[n];
+                    } else {
+                        const uint32_t four = ch[n] >> (32 - 4 * BITS);
+                        out[n][wi] |= four << at;
+                        if (at + 4 * BITS > 32) out[n][wi + 1] |= four >> (32 - at);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                if (t >= n_t) break;
+                f32x4 acc[NT];
+                products(t, acc);
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        uint32_t code;
+                        float d;
+                        if (NB == 1 || use_grid) {
+                            const float b = boundary(n, acc[n][i]);
+                            d = __builtin_fmaf(acc[n][i], rn[n], -b);
+                            code = ((NB > 1 ? __float_as_uint(b) : 0u) + (d > 0.0f ? 1u : 0u)) & CMASK;
+                        } else {  // no grid: the distance to the closest boundary
+                            const float z = acc[n][i] * rn[n];
+                            d = __builtin_inff();
+#pragma unroll 1
+                            for (int k = 0; k < NB; ++k) d = fminf(d, fabsf(z - sh.bound[k]));
+                            code = bucket_lds(z, sh.bound, BITS);
+                        }
+                        amb[n] |= fabsf(d) < mg[n] ? 1u << (4 * t + i) : 0u;
+                        const int bit = (4 * t + i) * BITS, wi = bit >> 5, at = bit & 31;
+                        out[n][wi] |= code << at;
+                        if (at + BITS > 32) out[n][wi + 1] |= code >> (32 - at);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
 
         // ---- outputs beyond the group's rows are no outputs
@@ -439,70 +521,62 @@ __global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
                 for (int n = 0; n < NT; ++n) out[n][k] &= keep;
             }
         }
-        const uint32_t valid = mine >= 32 ? 0xFFFFFFFFu : mine == 0 ? 0u : ~(0xFFFFFFFFu >> mine);
+        const uint32_t valid = mine >= 32 ? 0xFFFFFFFFu : (1u << mine) - 1u;
 
-        // ---- rows without a doubtful output leave; the others queue with the outputs to run
-        uint32_t pend = 0, given = 0, first[NT], queued[NT];  // wave-uniform, a bit per tile
+        // ---- rows without a doubtful output leave; the others queue, with those outputs or, where the
+        // item has more than the queue takes, with all of theirs
+        uint32_t queued[NT], mine_q = 0u;
+        bool any = false;
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
             if ((special >> n) & 1u) amb[n] = 0xFFFFFFFFu;
             amb[n] = live[n] ? amb[n] & valid : 0u;
             if (!live[n]) n_amb &= ~(1u << n);
+            const bool norm = ((n_amb >> n) & 1u) && g == 0;
+            mine_q += __popc(amb[n]) + (norm ? 1u : 0u);
             const uint32_t rows = fold_vectors(__builtin_amdgcn_ballot_w64(amb[n] != 0u));
             if (live[n] && !((rows >> v) & 1u)) store_row(a.codes + slot[n] * row_bytes, out[n]);
             queued[n] = rows | fold_vectors(__builtin_amdgcn_ballot_w64((n_amb >> n) & 1u));
-            first[n] = 0u;
-            if (queued[n]) pend |= 1u << n;
+            any = any || queued[n] != 0u;
         }
-        // normally one round; more when the queue fills (vectors whose every output is doubtful)
-        for (;;) {
-            bool full = false;
+        if (any) {
+#pragma unroll
+            for (int k = 1; k < 64; k <<= 1) mine_q += (uint32_t)__shfl_xor((int)mine_q, k);
+            const bool whole = mine_q > 64u;
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
-                if (!((pend >> n) & 1u)) continue;
-                const uint32_t below = __popc(queued[n] & ((1u << v) - 1u));
-                if (!((given >> n) & 1u)) {
-                    if (q_rows + __popc(queued[n]) > QROWS) {
-                        full = true;
-                        continue;
+                const uint32_t below = __popc(queued[n] & ((1u << v) - 1u)), qr = q_rows + below;
+                if ((queued[n] >> v) & 1u) {
+                    if (g == 0) {
+                        sh.vec[wave][qr] = (uint32_t)item * (16u * NT) + 16u * n + (uint32_t)v;
+                        if (whole) sh.all[wave][q_all + below] = qr;
                     }
-                    given |= 1u << n;
-                    first[n] = q_rows;
-                    q_rows += __popc(queued[n]);
-                    if ((queued[n] >> v) & 1u) {
-                        if (g == 0) s_vec[wave][first[n] + below] = (uint32_t)item * (16u * NT) + 16u * n + (uint32_t)v;
 #pragma unroll
-                        for (int k = 0; k < BITS; ++k) s_row[wave][first[n] + below][BITS * g + k] = out[n][k];
-                    }
+                    for (int k = 0; k < BITS; ++k) sh.row[wave][qr][BITS * g + k] = out[n][k];
+                }
+                q_rows += __popc(queued[n]);
+                if (whole) {
+                    q_all += __popc(queued[n]);
+                    continue;
                 }
                 for (;;) {
                     const bool norm = ((n_amb >> n) & 1u) && g == 0;
                     const bool p = norm || amb[n] != 0u;
                     const uint64_t who = __builtin_amdgcn_ballot_w64(p);
-                    if (who == 0) {
-                        pend &= ~(1u << n);
-                        break;
-                    }
-                    if (q_pairs + 64 > QPAIRS) break;
+                    if (who == 0) break;
                     const uint32_t at = q_pairs + __builtin_amdgcn_mbcnt_hi((uint32_t)(who >> 32),
                                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)who, 0));
-                    const int top = __clz((int)amb[n]);  // jj of the first doubtful output
-                    if (p) s_pair[wave][at] = ((first[n] + below) << 8) | (norm ? NORM_ONLY : 32u * g + (uint32_t)top);
-                    if (!norm) amb[n] &= ~(0x80000000u >> (top & 31));
-                    if (norm || g != 0) n_amb &= ~(1u << n);
+                    const uint32_t jj = (uint32_t)__builtin_ctz(amb[n] | 0x80000000u);  // the first doubtful output
+                    if (p) sh.pair[wave][at] = (qr << 8) | (norm ? NORM_ONLY : 32u * g + jj);
+                    if (!norm) amb[n] &= ~(1u << jj);
+                    n_amb &= ~(1u << n);
                     q_pairs += __popcll(who);
                 }
             }
-            if (!last && pend == 0 && q_pairs < QPAIRS - 64) break;
-            run_pairs();
-            if (last || full) {
-                // a tile given rows and still holding outputs keeps them
-                if ((pend & given) == 0) store_queued();
-            }
-            if (pend == 0) break;
         }
-        if (last) break;
-    }
+        }
+        if (q_rows) run_queue();
+    } while (item < n_items);
 }
 
 // ------------------------------------------------------------------ residual sketch of Q_prod keys
@@ -513,14 +587,13 @@ __global__ __launch_bounds__(MQ_THREADS) void codes_kernel(EncodeArgs a) {
 // terms (nearest even, r within 2^-18), S as two, three products.  With |r| factored out the bound is
 // s (7.63e-6 chain + 3 * 2^-18 terms + 1.6e-6 + rounding) = 2.2e-5 s, s the largest row norm of S; a
 // projection inside it, one in 4000, is run as the chain, with rhat from the division the chain uses.
+
+// cv[s] = C[code of index 4 s + g]: the row is shifted down by g codes once, after which index 4 s + g
+// sits at the fixed bit 4 s BITS.  w has a zero word past the row's end.
 template <int BITS, int... I>
-__device__ __forceinline__ void plain_centers(const uint32_t* w, int g, const float* cent, float* cv,
+__device__ __forceinline__ void plain_centers(const uint32_t* w, const float* cent, float* cv,
                                               std::integer_sequence<int, I...>) {
-    constexpr uint32_t MASK = (1u << BITS) - 1u;
-    ((cv[I] = cent[(uint32_t)(((uint64_t)w[(4 * I * BITS) >> 5] | ((uint64_t)w[((4 * I * BITS) >> 5) + 1] << 32)) >>
-                               (((4 * I * BITS) & 31) + g * BITS)) &
-                   MASK]),
-     ...);
+    ((cv[I] = cent[tq::extract_bits<BITS>(w, 4 * I * BITS)]), ...);
 }
 
 template <int BITS, bool GROUP>
@@ -531,7 +604,7 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
     __shared__ uint4 s_s[8 * 4 * 2 * 64];     // S, two bf16 terms: [row tile][k-step][term][lane]
     __shared__ float s_cent[1 << BITS];
     __shared__ uint32_t s_code[GROUP ? MQ_WAVES : 1][GROUP ? 16 : 1][GRW];
-    __shared__ float4 s_r[MQ_WAVES][2][D / 4];
+    __shared__ float4 s_r[MQ_WAVES][D / 4];
     __shared__ uint32_t s_max;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int v = lane & 15, g = lane >> 4;
@@ -606,7 +679,9 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
                 w[4 * c] = q.x, w[4 * c + 1] = q.y, w[4 * c + 2] = q.z, w[4 * c + 3] = q.w;
             }
             w[RW] = 0u;
-            plain_centers<BITS>(w, g, s_cent, cv, std::make_integer_sequence<int, 32>{});
+#pragma unroll
+            for (int c = 0; c < RW; ++c) w[c] = __builtin_amdgcn_alignbit(w[c + 1], w[c], g * BITS);
+            plain_centers<BITS>(w, s_cent, cv, std::make_integer_sequence<int, 32>{});
         } else {
             // the row byte by byte where it does not fill a dword, so nothing outside it is read
             uint32_t* row = s_code[wave][v];
@@ -671,8 +746,9 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
                 rl[s].u[k] = bf16_pair(e0 - lo_half(rh[s].u[k]), e1 - hi_half(rh[s].u[k]));
             }
         // ---- projections: lane g holds signs [32 g, 32 g + 32)
-        uint32_t sb = 0u, amb = 0u;
-        const float mg = eps * rho;
+        f32x4 proj[8];
+        uint32_t neg = 0u;  // sign bits, the first output's highest
+        float closest = __builtin_inff();
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             f32x4 p = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -688,87 +764,95 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
                 p = mfma_bf16(m, rl[s], p);
                 p = mfma_bf16(m, rh[s], p);
             }
+            proj[t] = p;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                sb |= (p[i] >= 0.0f ? 1u : 0u) << (4 * t + i);
-                amb |= (!(fabsf(p[i]) >= mg) ? 1u : 0u) << (4 * t + i);
+                neg = __builtin_amdgcn_alignbit(neg, __float_as_uint(p[i]), 31);
+                if (!GROUP || 4 * t + i < mine) closest = fminf(closest, fabsf(p[i]));
             }
+        }
+        uint32_t sb = ~__brev(neg), amb = 0u;
+        const float mg = eps * rho;
+        if (__any(closest < mg)) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) amb |= fabsf(proj[t][i]) < mg ? 1u << (4 * t + i) : 0u;
         }
         // every r of magnitude 0: the projections are +0 in the chain too.  Otherwise, with squares that
         // vanish, the chain decides.
-        uint32_t nz = 0u;
+        if (__any(tiny)) {
+            uint32_t nz = 0u;
 #pragma unroll
-        for (int k = 0; k < 32; ++k) nz |= __float_as_uint(r[k]);
-        nz &= 0x7FFFFFFFu;
-        nz |= (uint32_t)__shfl_xor((int)nz, 16);
-        nz |= (uint32_t)__shfl_xor((int)nz, 32);
-        if (tiny) {
-            amb = nz ? 0xFFFFFFFFu : 0u;
-            if (!nz) sb = 0xFFFFFFFFu;
+            for (int k = 0; k < 32; ++k) nz |= __float_as_uint(r[k]);
+            nz &= 0x7FFFFFFFu;
+            nz |= (uint32_t)__shfl_xor((int)nz, 16);
+            nz |= (uint32_t)__shfl_xor((int)nz, 32);
+            if (tiny) {
+                amb = nz ? 0xFFFFFFFFu : 0u;
+                if (!nz) sb = 0xFFFFFFFFu;
+            }
         }
         if (bad) amb = 0xFFFFFFFFu;
         amb &= valid;
         if (!live) amb = 0u, rho_amb = false;
 
-        uint32_t todo = fold_vectors(__builtin_amdgcn_ballot_w64(amb != 0u || rho_amb));
         uint32_t rho16 = tq::f32_to_f16(rho);
-        while (todo) {  // uniform: one vector at a time, its residual in LDS
-            const int vv = __builtin_ctz(todo);
-            todo &= todo - 1u;
-            float4* sr = s_r[wave][0];
-            float4* sh = s_r[wave][1];
-            wave_lds_fence();
-            if (v == vv) {
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    sr[8 * g + k] = make_float4(r[4 * k], r[4 * k + 1], r[4 * k + 2], r[4 * k + 3]);
-            }
-            wave_lds_fence();
+        if (__any(amb != 0u || rho_amb)) {
+            // the tile's sums of squares as chains: lane group p runs dims [32 p, 32 p + 32) on from group p - 1
             float ss = 0.0f;
-#pragma unroll 8
-            for (int k = 0; k < D / 4; ++k) {
-                const float4 e = sr[k];
-                ss = __builtin_fmaf(e.x, e.x, ss);
-                ss = __builtin_fmaf(e.y, e.y, ss);
-                ss = __builtin_fmaf(e.z, e.z, ss);
-                ss = __builtin_fmaf(e.w, e.w, ss);
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+#pragma unroll
+                for (int k = 0; k < 32; ++k) ss = __builtin_fmaf(r[k], r[k], ss);
+                ss = __shfl(ss, 16 * p + v);
             }
             float rx = tq::sqrt_rn(ss);
             if (!(rx > 0.0f)) rx = 1.0f;
-            if (v == vv) rho16 = tq::f32_to_f16(rx);
-            uint32_t aw[4], any = 0u;
+            rho16 = tq::f32_to_f16(rx);
+            uint32_t todo = fold_vectors(__builtin_amdgcn_ballot_w64(amb != 0u));
+            while (todo) {  // uniform: one vector at a time, its residual over rho in LDS
+                const int vv = __builtin_ctz(todo);
+                todo &= todo - 1u;
+                float4* sr = s_r[wave];
+                float* fr = reinterpret_cast<float*>(sr);
+                wave_lds_fence();
+                if (v == vv) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                aw[k] = (uint32_t)__builtin_amdgcn_readlane((int)amb, vv + 16 * k);
-                any |= aw[k];
-            }
-            if (!any) continue;
-            float* fr = reinterpret_cast<float*>(sr);
-            float* fh = reinterpret_cast<float*>(sh);
-            fh[lane] = tq::div_rn(fr[lane], rx);
-            fh[lane + 64] = tq::div_rn(fr[lane + 64], rx);
-            wave_lds_fence();
-#pragma unroll
-            for (int half = 0; half < 2; ++half) {
-                const uint32_t mine_w = lane < 32 ? aw[2 * half] : aw[2 * half + 1];
-                const bool need = (mine_w >> (lane & 31)) & 1u;
-                bool pos = false;
-                if (need) {
-                    const float4* si = reinterpret_cast<const float4*>(a.S) + (64 * half + lane) * (D / 4);
-                    float p = 0.0f;
-#pragma unroll 8
-                    for (int k = 0; k < D / 4; ++k) {
-                        const float4 e = sh[k], c = si[k];
-                        p = __builtin_fmaf(e.x, c.x, p);
-                        p = __builtin_fmaf(e.y, c.y, p);
-                        p = __builtin_fmaf(e.z, c.z, p);
-                        p = __builtin_fmaf(e.w, c.w, p);
-                    }
-                    pos = p >= 0.0f;
+                    for (int k = 0; k < 8; ++k)
+                        sr[8 * g + k] = make_float4(r[4 * k], r[4 * k + 1], r[4 * k + 2], r[4 * k + 3]);
                 }
-                const uint64_t bits = __builtin_amdgcn_ballot_w64(pos);
-                if (v == vv && (g >> 1) == half)
-                    sb = (sb & ~amb) | ((uint32_t)(bits >> (32 * (g & 1))) & amb);
+                wave_lds_fence();
+                const float rv = __shfl(rx, vv);
+                const float h0_ = tq::div_rn(fr[lane], rv), h1_ = tq::div_rn(fr[lane + 64], rv);
+                wave_lds_fence();
+                fr[lane] = h0_;
+                fr[lane + 64] = h1_;
+                wave_lds_fence();
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    const uint32_t w0 = (uint32_t)__builtin_amdgcn_readlane((int)amb, vv + 32 * half);
+                    const uint32_t w1 = (uint32_t)__builtin_amdgcn_readlane((int)amb, vv + 32 * half + 16);
+                    if ((w0 | w1) == 0u) continue;
+                    const bool need = ((lane < 32 ? w0 : w1) >> (lane & 31)) & 1u;
+                    bool pos = false;
+                    if (need) {
+                        const float4* si = reinterpret_cast<const float4*>(a.S) + (64 * half + lane) * (D / 4);
+                        float p = 0.0f;
+#pragma unroll 8
+                        for (int k = 0; k < D / 4; ++k) {
+                            const float4 e = sr[k], c = si[k];
+                            p = __builtin_fmaf(e.x, c.x, p);
+                            p = __builtin_fmaf(e.y, c.y, p);
+                            p = __builtin_fmaf(e.z, c.z, p);
+                            p = __builtin_fmaf(e.w, c.w, p);
+                        }
+                        pos = p >= 0.0f;
+                    }
+                    const uint64_t bits = __builtin_amdgcn_ballot_w64(pos);
+                    if (v == vv && (g >> 1) == half)
+                        sb = (sb & ~amb) | ((uint32_t)(bits >> (32 * (g & 1))) & amb);
+                }
             }
         }
         if (live) {
@@ -794,21 +878,20 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
 // Workgroups of a kernel that fit on the device at once (each loops over tiles, so more would only
 // repeat the LDS set-up).
 template <auto KERNEL>
-int64_t resident() {
+int64_t resident(int threads) {
     static std::atomic<int64_t> cached[tq::MAX_DEVICES];
-    return tq::once_per_device(cached, 256, [](int dev) {
+    return tq::once_per_device(cached, 256, [threads](int dev) {
         int cus = 0, per_cu = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, KERNEL, MQ_THREADS, 0) != hipSuccess || per_cu < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, KERNEL, threads, 0) != hipSuccess || per_cu < 1)
             per_cu = 1;
         return (int64_t)cus * per_cu;
     });
 }
 
 template <auto KERNEL>
-int launch(const EncodeArgs& a, int64_t items, hipStream_t s) {
-    const int64_t groups = std::min<int64_t>((items + MQ_WAVES - 1) / MQ_WAVES, resident<KERNEL>());
-    hipLaunchKernelGGL(KERNEL, dim3((unsigned)groups), dim3(MQ_THREADS), 0, s, a);
+int launch(const EncodeArgs& a, int64_t groups, int threads, hipStream_t s) {
+    hipLaunchKernelGGL(KERNEL, dim3((unsigned)std::min(groups, resident<KERNEL>(threads))), dim3(threads), 0, s, a);
     TQ_CHECK_LAUNCH();
     return TQ_OK;
 }
@@ -816,13 +899,14 @@ int launch(const EncodeArgs& a, int64_t items, hipStream_t s) {
 template <int BITS, bool GROUP>
 int encode(const EncodeArgs& a, hipStream_t s) {
     const int64_t tiles = (a.n_vec + 15) / 16;
-    // four tiles per wave share each matrix fragment read from LDS; a call with fewer tiles than the
+    // two tiles per wave share each matrix fragment read from LDS; a call with fewer tiles than the
     // device has waves spreads them instead
-    const int64_t waves = resident<codes_kernel<BITS, GROUP, 4>>() * MQ_WAVES;
-    const int st = tiles >= 2 * waves ? launch<codes_kernel<BITS, GROUP, 4>>(a, (tiles + 3) / 4, s)
-                                      : launch<codes_kernel<BITS, GROUP, 1>>(a, tiles, s);
+    const int64_t waves = resident<codes_kernel<BITS, GROUP, 2>>(CT) * CW;
+    const int st = tiles > waves ? launch<codes_kernel<BITS, GROUP, 2>>(a, (tiles + 1) / 2, CT, s)
+                                 : launch<codes_kernel<BITS, GROUP, 1>>(a, tiles, CT, s);
     if (st != TQ_OK || !a.S) return st;
-    if constexpr (GROUP || BITS <= 3) return launch<residual_kernel<BITS, GROUP>>(a, tiles, s);
+    if constexpr (GROUP || BITS <= 3)
+        return launch<residual_kernel<BITS, GROUP>>(a, (tiles + MQ_WAVES - 1) / MQ_WAVES, MQ_THREADS, s);
     return TQ_ERR_INVALID_ARGUMENT;
 }
 
