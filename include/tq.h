@@ -201,6 +201,18 @@ int tq_dequantize_prod(const uint8_t* codes, const uint16_t* norms, const uint8_
 int tq_group_matrix(const float* sub, int sub_dim, const int32_t* channels, int dim, float* out);
 
 /*
+ * Channel energies of a layer's prompt: out[c] = sum over all vectors of k_c^2 + v_c^2, fp32 [dim]
+ * (device).  What the outlier channels are chosen by; replaces the reductions of reference
+ * detect_outlier_channels (runtime/packed_qmse_cache.py:95-114).  k, v: bf16 [batch][heads][tokens][dim]
+ * with element strides, rows 16-byte aligned.  partials: device scratch of
+ * 2 * TQ_ENERGY_BLOCKS * dim floats.
+ */
+#define TQ_ENERGY_BLOCKS 256
+int tq_channel_energy(const uint16_t* k, const uint16_t* v, int batch, int heads, int64_t tokens, int dim,
+                      int64_t k_sb, int64_t k_sh, int64_t k_st, int64_t v_sb, int64_t v_sh, int64_t v_st,
+                      float* partials, float* out, void* stream);
+
+/*
  * Encode one channel group: Q_mse at `bits` when qjl is NULL, else Q_prod keys with
  * `bits` MSE bits plus the QJL sketch (centers, signs and rnorms then required).
  * Results are those of tq_quantize_mse / tq_quantize_prod applied to the gathered

@@ -108,3 +108,13 @@ def test_group_prefill_encoder_on_hard_rows(cuda, d, bits, extra, qjl):
             compare(x, (kc, kn), O.encode_mse(rows, g.bits, h[0], h[2]), T)
         for t in (kc, ks) if g.qjl is not None else (kc,):
             assert int(t[:, :, :2].count_nonzero()) == 0 and int(t[:, :, T + 2:].count_nonzero()) == 0
+
+
+@pytest.mark.parametrize("B,H,T", [(1, 1, 1), (2, 3, 17), (1, 8, 1000), (3, 2, 40001)])
+def test_channel_energy_matches_fp64(cuda, B, H, T):
+    """Strided keys and values, workgroups whose runs cross heads; fp32 sums of at most
+    B * H * T / 4096 + 32 squares per thread, 512 of them: 1e-5 of each energy."""
+    k = kv_bf16((B, T, H, D), seed=1, device=cuda).transpose(1, 2)
+    v = kv_bf16((B, H, T, D), seed=2, device=cuda, outlier_channels=3)
+    ref = sum(t.double().square().sum(dim=(0, 1, 2)) for t in (k, v))
+    assert ((K.channel_energy(k, v).double() - ref).abs() <= 1e-5 * ref).all()

@@ -650,6 +650,7 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
     const int sign_bytes = (sub_dim + 7) >> 3;
     const int mine = std::min(std::max(sub_dim - 32 * g, 0), 32);
     const uint32_t valid = mine >= 32 ? 0xFFFFFFFFu : (1u << mine) - 1u;
+    const int n_t = sub_dim < 32 ? (sub_dim + 3) >> 2 : 8;
 
     const int64_t n_tiles = (a.n_vec + 15) / 16;
     for (int64_t tile = (int64_t)blockIdx.x * MQ_WAVES + wave; tile < n_tiles;
@@ -712,7 +713,28 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
             wave_lds_fence();
         }
         f32x4 acc[8];
-        image_products(a_img, cv, acc);
+        if constexpr (!GROUP) {
+            image_products(a_img, cv, acc);
+        } else {
+            // a group's chains start behind `pad` zero products, which leave +0 as it is: whole blocks of
+            // 16 of them are skipped (a group of 4 channels runs one block of eight)
+#pragma unroll
+            for (int t = 0; t < 8; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int sb = 0; sb < 8; ++sb) {
+                if (16 * sb + 16 <= pad) continue;
+                float4 m[8];
+#pragma unroll
+                for (int t = 0; t < 8; ++t) m[t] = a_img[(t * 8 + sb) * 64];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int t = 0; t < 8; ++t)
+                        acc[t] = mfma_f32(e == 0 ? m[t].x : e == 1 ? m[t].y : e == 2 ? m[t].z : m[t].w, cv[4 * sb + e],
+                                          acc[t]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
         // ---- r = x - bf16(khat), dims 32 g + (0..31)
         float r[32];
         float rs = 0.0f;
@@ -752,6 +774,11 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             f32x4 p = {0.0f, 0.0f, 0.0f, 0.0f};
+            proj[t] = p;
+            if (GROUP && t >= n_t) {  // rows past the group's
+                neg <<= 4;
+                continue;
+            }
             Frag m;
 #pragma unroll
             for (int s = 0; s < 4; ++s) {

@@ -281,6 +281,82 @@ __global__ __launch_bounds__(GBLOCK) void dequantize_group_kernel(
     }
 }
 
+// ------------------------------------------------------------------ channel energies
+// sum over all vectors of x_c^2, keys and values together: what the outlier channels are chosen by.
+// Reads each tensor once (as torch operations it took three passes and fp32 copies: 220 us for
+// 2 x 8 x 16384 keys and values of a split prefill, 21 us here).  A thread holds 8 channels and walks
+// rows 16 apart; a workgroup's 16 row lanes meet in LDS, the workgroups in energy_sum_kernel, in a
+// fixed order.
+constexpr int EB = TQ_ENERGY_BLOCKS;
+
+__global__ __launch_bounds__(GBLOCK) void channel_energy_kernel(const uint16_t* __restrict__ k,
+                                                                const uint16_t* __restrict__ v, int heads,
+                                                                int64_t tokens, int64_t n_vec, int64_t k_sb, int64_t k_sh,
+                                                                int64_t k_st, int64_t v_sb, int64_t v_sh, int64_t v_st,
+                                                                float* __restrict__ partials) {
+    __shared__ float s_sum[GBLOCK / 16][D];
+    const int c = threadIdx.x & 15, r = threadIdx.x >> 4;
+    const bool vals = blockIdx.y != 0;
+    const uint16_t* x = vals ? v : k;
+    const int64_t sb = vals ? v_sb : k_sb, sh = vals ? v_sh : k_sh, st = vals ? v_st : k_st;
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
+    // contiguous runs of rows per workgroup: the row index advances without divisions inside a head
+    const int64_t per = (n_vec + gridDim.x - 1) / gridDim.x;
+    const int64_t end = std::min<int64_t>(((int64_t)blockIdx.x + 1) * per, n_vec);
+    for (int64_t i = (int64_t)blockIdx.x * per; i < end;) {
+        const int64_t gh = i / tokens, t0 = i - gh * tokens, b = gh / heads, h = gh - b * heads;
+        const int64_t run = std::min<int64_t>(tokens - t0, end - i);  // rows of this head
+        const uint16_t* base = x + b * sb + h * sh + t0 * st + 8 * c;
+#pragma unroll 4
+        for (int64_t t = r; t < run; t += GBLOCK / 16) {
+            const uint4 w = *reinterpret_cast<const uint4*>(base + t * st);
+            const uint32_t p[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float lo = tq::bf16_to_f32(p[e] & 0xFFFFu), hi = __uint_as_float(p[e] & 0xFFFF0000u);
+                acc[2 * e] = __builtin_fmaf(lo, lo, acc[2 * e]);
+                acc[2 * e + 1] = __builtin_fmaf(hi, hi, acc[2 * e + 1]);
+            }
+        }
+        i += run;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s_sum[r][8 * c + e] = acc[e];
+    __syncthreads();
+    if (threadIdx.x < D) {
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < GBLOCK / 16; ++i) s += s_sum[i][threadIdx.x];
+        partials[((int64_t)blockIdx.y * EB + blockIdx.x) * D + threadIdx.x] = s;
+    }
+}
+
+__global__ __launch_bounds__(1024) void energy_sum_kernel(const float* __restrict__ partials, int blocks,
+                                                          float* __restrict__ out) {
+    __shared__ float s_sum[1024 / D][D];
+    const int c = threadIdx.x & (D - 1), r = threadIdx.x / D;
+    float s = 0.0f;
+    // one workgroup, so the reads' latency is all there is: all of a thread's in flight at once
+    float p[2 * EB / (1024 / D)];
+#pragma unroll
+    for (int i = 0; i < 2 * EB / (1024 / D); ++i) {
+        const int blk = r + i * (1024 / D);  // keys' blocks, then values'
+        p[i] = (blk & (EB - 1)) < blocks ? partials[(int64_t)blk * D + c] : 0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * EB / (1024 / D); ++i) s += p[i];
+    s_sum[r][c] = s;
+    __syncthreads();
+    if (threadIdx.x < D) {
+        float t = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 1024 / D; ++i) t += s_sum[i][c];
+        out[c] = t;
+    }
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Validates a group's channel list (host memory): 1 <= sub_dim <= dim, strictly
@@ -307,6 +383,24 @@ extern "C" int tq_group_matrix(const float* sub, int sub_dim, const int32_t* cha
     for (int64_t k = 0; k < (int64_t)dim * dim; ++k) out[k] = 0.0f;
     for (int j = 0; j < sub_dim; ++j)
         for (int i = 0; i < sub_dim; ++i) out[(int64_t)j * dim + channels[i]] = sub[(int64_t)j * sub_dim + i];
+    return TQ_OK;
+}
+
+extern "C" int tq_channel_energy(const uint16_t* k, const uint16_t* v, int batch, int heads, int64_t tokens, int dim,
+                                 int64_t k_sb, int64_t k_sh, int64_t k_st, int64_t v_sb, int64_t v_sh, int64_t v_st,
+                                 float* partials, float* out, void* stream) {
+    if (!k || !v || !partials || !out || batch < 1 || heads < 1 || tokens < 1) return TQ_ERR_INVALID_ARGUMENT;
+    if (dim != D) return TQ_ERR_UNSUPPORTED;
+    if (!aligned16(k) || !aligned16(v) || k_sb % 8 || k_sh % 8 || k_st % 8 || v_sb % 8 || v_sh % 8 || v_st % 8)
+        return TQ_ERR_UNSUPPORTED;
+    const int64_t n_vec = (int64_t)batch * heads * tokens;
+    const int blocks = (int)std::min<int64_t>(EB, (n_vec + 63) / 64);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    hipLaunchKernelGGL(channel_energy_kernel, dim3(blocks, 2), dim3(GBLOCK), 0, s, k, v, heads, tokens, n_vec, k_sb, k_sh,
+                       k_st, v_sb, v_sh, v_st, partials);
+    TQ_CHECK_LAUNCH();
+    hipLaunchKernelGGL(energy_sum_kernel, dim3(1), dim3(1024), 0, s, partials, blocks, out);
+    TQ_CHECK_LAUNCH();
     return TQ_OK;
 }
 

@@ -42,6 +42,7 @@ SIGNATURES: dict[str, tuple] = {
                                         _P, _P, _P, _P, _P, _P, _P, _F, _P, _P, _P, _P, _SZ, _P]),
     "tq_quantize_group": (_I, [_P, _I, _I, _I64, _I, _I64, _I64, _I64, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P,
                                _P, _I64, _I64, _P]),
+    "tq_channel_energy": (_I, [_P, _P, _I, _I, _I64, _I, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _P]),
     "tq_dense_attention": (_I, [_P, _I, _I, _I, _I, _I, _I, _I64, _I64, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64,
                                 _I64, _I64, _P, _I, _I64, _I64, _I64, _P, _P, _I64, _F, _P, _I, _I, _I, _I, _P, _P,
                                 _P, _P, _P]),

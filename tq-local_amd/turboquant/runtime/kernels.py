@@ -191,6 +191,21 @@ def quantize_group(x: torch.Tensor, g: GroupCodec, codes: torch.Tensor, norms: t
               _vp(norms), _vp(signs if prod else None), _vp(rnorms if prod else None), cap, offset, _stream(x.device))
 
 
+_ENERGY_BLOCKS = 256  # TQ_ENERGY_BLOCKS
+
+
+def channel_energy(k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
+    """Per channel the sum of squares over all keys and values, fp32 [D]; k, v bf16 [B,H,T,D] on the GPU."""
+    k, v = _as_encoder_input(k), _as_encoder_input(v)
+    _require_gpu(k, v)
+    B, H, T, D = k.shape
+    buf = torch.empty(2 * _ENERGY_BLOCKS * D + D, dtype=torch.float32, device=k.device)
+    out = buf[-D:]
+    _lib.call("tq_channel_energy", _vp(k), _vp(v), B, H, T, D, *k.stride()[:3], *v.stride()[:3], _vp(buf), _vp(out),
+              _stream(k.device))
+    return out
+
+
 def dequantize_group(codes: torch.Tensor, norms: torch.Tensor, tokens: int, g: GroupCodec, out: torch.Tensor,
                      merge: bool, signs: torch.Tensor | None = None, rnorms: torch.Tensor | None = None,
                      start: int = 0) -> None:

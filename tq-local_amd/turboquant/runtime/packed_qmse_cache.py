@@ -106,15 +106,28 @@ def _packed_rows(t: torch.Tensor) -> torch.Tensor:
     return t if t.is_contiguous() else t.contiguous()
 
 
-def detect_outlier_channels(key_states: torch.Tensor, value_states: torch.Tensor,
-                            num_outlier_channels: int) -> tuple[torch.Tensor, torch.Tensor]:
-    """(outlier, normal) channel indices, both ascending: the channels of largest
-    combined key + value energy (reference runtime/packed_qmse_cache.py:95-114)."""
-    combined = key_states.float().pow(2).sum(dim=(0, 1, 2)) + value_states.float().pow(2).sum(dim=(0, 1, 2))
+def _channel_energy(key_states: torch.Tensor, value_states: torch.Tensor) -> torch.Tensor:
+    """Key plus value energy of each channel, fp32 [D].  bf16 prompts on the GPU take libtq's one-pass
+    kernel; other dtypes, devices and shapes torch's reductions."""
+    if all(t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 4 and t.shape[-1] == K.HEAD_DIM and t.numel()
+           for t in (key_states, value_states)) and key_states.shape == value_states.shape:
+        return K.channel_energy(key_states.detach(), value_states.detach())
+    return key_states.float().pow(2).sum(dim=(0, 1, 2)) + value_states.float().pow(2).sum(dim=(0, 1, 2))
+
+
+def _split_channels(combined: torch.Tensor, num_outlier_channels: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """(outlier, normal) channel indices, both ascending, of the channel energies."""
     outlier = torch.topk(combined, num_outlier_channels).indices.sort().values
     keep = torch.ones(combined.shape[0], dtype=torch.bool, device=combined.device)
     keep[outlier] = False
     return outlier, torch.arange(combined.shape[0], device=combined.device)[keep]
+
+
+def detect_outlier_channels(key_states: torch.Tensor, value_states: torch.Tensor,
+                            num_outlier_channels: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """(outlier, normal) channel indices, both ascending: the channels of largest
+    combined key + value energy (reference runtime/packed_qmse_cache.py:95-114)."""
+    return _split_channels(_channel_energy(key_states, value_states), num_outlier_channels)
 
 
 class _Store:
@@ -210,10 +223,11 @@ class PackedMSELayer(CacheLayerMixin):
         self.device = key_states.device
         D = int(key_states.shape[-1])
         if 0 < self.num_outlier_channels < D:
-            outlier, normal = detect_outlier_channels(key_states, value_states, self.num_outlier_channels)
-            self._split = split_codecs(normal.cpu().numpy(), outlier.cpu().numpy(), self.bits,
-                                       self.outlier_extra_bits, self.seed, self.use_qjl_keys, self.device,
-                                       self.grid_size)
+            # the channels are needed on the host: the 128 energies go there, once, and are sorted there
+            outlier, normal = _split_channels(_channel_energy(key_states, value_states).cpu(),
+                                              self.num_outlier_channels)
+            self._split = split_codecs(normal.numpy(), outlier.numpy(), self.bits, self.outlier_extra_bits, self.seed,
+                                       self.use_qjl_keys, self.device, self.grid_size)
         else:
             self.codecs = layer_codecs(D, self.bits, self.seed, self.use_qjl_keys, self.device, self.grid_size)
         self.is_initialized = True
