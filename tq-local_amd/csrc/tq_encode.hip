@@ -32,8 +32,6 @@
 
 #include <algorithm>
 #include <atomic>
-#include <type_traits>
-#include <utility>
 
 #include "tq_encode.h"
 
@@ -57,15 +55,6 @@ union Frag {
 __device__ __forceinline__ f32x4 mfma_bf16(const Frag& a, const Frag& b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, b.b, c, 0, 0, 0);
 }
-// fp32 -> bf16, nearest even (v_cvt_pk_bf16_f32: the bits of tq::f32_to_bf16 for all 2^32 inputs).
-__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    const f32x2 p = {a, b};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2));
-}
-__device__ __forceinline__ float lo_half(uint32_t p) { return __uint_as_float(p << 16); }
-__device__ __forceinline__ float hi_half(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
 // a.lo b.lo + a.hi b.hi + c over bf16 pairs; within 3 * 2^-24 of the sum (positive terms; probed).
 __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -587,15 +576,6 @@ __global__ __launch_bounds__(CT) void codes_kernel(EncodeArgs a) {
 // terms (nearest even, r within 2^-18), S as two, three products.  With |r| factored out the bound is
 // s (7.63e-6 chain + 3 * 2^-18 terms + 1.6e-6 + rounding) = 2.2e-5 s, s the largest row norm of S; a
 // projection inside it, one in 4000, is run as the chain, with rhat from the division the chain uses.
-
-// cv[s] = C[code of index 4 s + g]: the row is shifted down by g codes once, after which index 4 s + g
-// sits at the fixed bit 4 s BITS.  w has a zero word past the row's end.
-template <int BITS, int... I>
-__device__ __forceinline__ void plain_centers(const uint32_t* w, const float* cent, float* cv,
-                                              std::integer_sequence<int, I...>) {
-    ((cv[I] = cent[tq::extract_bits<BITS>(w, 4 * I * BITS)]), ...);
-}
-
 template <int BITS, bool GROUP>
 __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
     constexpr int RW = 4 * BITS;
@@ -680,9 +660,7 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
                 w[4 * c] = q.x, w[4 * c + 1] = q.y, w[4 * c + 2] = q.z, w[4 * c + 3] = q.w;
             }
             w[RW] = 0u;
-#pragma unroll
-            for (int c = 0; c < RW; ++c) w[c] = __builtin_amdgcn_alignbit(w[c + 1], w[c], g * BITS);
-            plain_centers<BITS>(w, s_cent, cv, std::make_integer_sequence<int, 32>{});
+            centers_of<BITS>(w, g, s_cent, cv);
         } else {
             // the row byte by byte where it does not fill a dword, so nothing outside it is read
             uint32_t* row = s_code[wave][v];

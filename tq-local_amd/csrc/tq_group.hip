@@ -560,8 +560,7 @@ __global__ __launch_bounds__(MQ_THREADS) void dequantize_group_mfma_kernel(
         uint32_t kh[2 * NT];  // bf16 pairs of channels 32g + 4 t0 + 2p, + 2p + 1
 #pragma unroll
         for (int p = 0; p < 2 * NT; ++p)
-            kh[p] = tq::f32_to_bf16(acc[p >> 1][2 * (p & 1)] * nf) |
-                    (tq::f32_to_bf16(acc[p >> 1][2 * (p & 1) + 1] * nf) << 16);
+            kh[p] = bf16_pair(acc[p >> 1][2 * (p & 1)] * nf, acc[p >> 1][2 * (p & 1) + 1] * nf);
         if constexpr (QJL) {
             float sv[32];
 #pragma unroll
@@ -574,11 +573,8 @@ __global__ __launch_bounds__(MQ_THREADS) void dequantize_group_mfma_kernel(
             const float rn = live ? tq::f16_to_f32(rnorms[slot]) : 0.0f;
 #pragma unroll
             for (int p = 0; p < 2 * NT; ++p) {
-                const float c0 = tq::bf16_to_f32(tq::f32_to_bf16((pacc[p >> 1][2 * (p & 1)] * rn) * qs));
-                const float c1 = tq::bf16_to_f32(tq::f32_to_bf16((pacc[p >> 1][2 * (p & 1) + 1] * rn) * qs));
-                const float k0 = tq::bf16_to_f32(kh[p] & 0xFFFFu) + c0;
-                const float k1 = tq::bf16_to_f32(kh[p] >> 16) + c1;
-                kh[p] = tq::f32_to_bf16(k0) | (tq::f32_to_bf16(k1) << 16);
+                const uint32_t c = bf16_pair((pacc[p >> 1][2 * (p & 1)] * rn) * qs, (pacc[p >> 1][2 * (p & 1) + 1] * rn) * qs);
+                kh[p] = bf16_pair(lo_half(kh[p]) + lo_half(c), hi_half(kh[p]) + hi_half(c));
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

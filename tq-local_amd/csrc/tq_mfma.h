@@ -16,6 +16,7 @@
 #pragma once
 
 #include <cstdint>
+#include <utility>
 
 #include "tq_common.h"
 
@@ -44,6 +45,32 @@ inline FastDiv make_fastdiv(uint32_t d) {
 }
 __device__ __forceinline__ uint32_t fdiv(uint32_t n, FastDiv f) {
     return (uint32_t)(((uint64_t)n * f.m) >> f.s);
+}
+
+// fp32 -> bf16, nearest even, two at a time (v_cvt_pk_bf16_f32: the bits of tq::f32_to_bf16 for all
+// 2^32 inputs), and back.
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const f32x2 p = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2));
+}
+__device__ __forceinline__ float lo_half(uint32_t p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float hi_half(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
+
+// cv[s] = cent[code of index 4 s + g], s = 0..31, from a vector's code row w (BITS words per 32 codes,
+// one zero word past the row's end).  The row is shifted down by g codes once; index 4 s + g then sits
+// at the fixed bit 4 s BITS, and the words, indexed by constants, stay in registers.
+template <int BITS, int... I>
+__device__ __forceinline__ void take_centers(const uint32_t* w, const float* cent, float* cv,
+                                             std::integer_sequence<int, I...>) {
+    ((cv[I] = cent[tq::extract_bits<BITS>(w, 4 * I * BITS)]), ...);
+}
+template <int BITS>
+__device__ __forceinline__ void centers_of(uint32_t* w, int g, const float* cent, float* cv) {
+#pragma unroll
+    for (int c = 0; c < 4 * BITS; ++c) w[c] = __builtin_amdgcn_alignbit(w[c + 1], w[c], g * BITS);
+    take_centers<BITS>(w, cent, cv, std::make_integer_sequence<int, 32>{});
 }
 
 // Rotation / QJL products of one tile: acc[t][i] = chain over d of b[d] * M[row(t, 4g + i)][d],
@@ -83,14 +110,27 @@ __device__ __forceinline__ void image_products(const float4* __restrict__ a, con
 // k-indices zero.  A chain over the image then starts with that many zero products, which
 // leave its +0 start unchanged (+0 plus a zero of either sign is +0), so it is the fma chain
 // over M's rows, bit for bit.
+// Every thread's reads are in flight together, ahead of the first LDS write: read one at a time they
+// took most of a small call (a 4-bit decode of 32768 rows 16.4 -> 12.4 us).
 __device__ __forceinline__ void build_image_transposed(float* img, const float* __restrict__ M, int rows = MXD) {
     const int pad = MXD - rows;
-    for (int idx = threadIdx.x; idx < MXD * MXD; idx += MQ_THREADS) {
-        const int d = idx / MXD, r = idx % MXD;  // consecutive threads read along one row of M
-        const int q = r >> 5, t = (r >> 2) & 7, m = 4 * q + (r & 3);
-        const int s = d >> 2, k = d & 3;
-        img[(t * 8 + (s >> 2)) * 256 + (s & 3) + 4 * ((16 * k + m) ^ k)] =
-            d >= pad ? M[(size_t)(d - pad) * MXD + r] : 0.0f;
+    constexpr int N = MXD * MXD / 4 / MQ_THREADS;
+    float4 v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int idx = threadIdx.x + i * MQ_THREADS, d = idx / (MXD / 4);  // k-index d, columns 4 (idx % 32) ..
+        v[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (d >= pad)  // M may start at any float
+            __builtin_memcpy(&v[i], M + (size_t)(d - pad) * MXD + 4 * (idx % (MXD / 4)), sizeof(float4));
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int idx = threadIdx.x + i * MQ_THREADS, d = idx / (MXD / 4), c = idx % (MXD / 4);
+        const int q = c >> 3, t = c & 7, s = d >> 2, k = d & 3;  // columns 4 c + (0..3) are rows 4 q + (0..3) of tile t
+        float* blk = img + (t * 8 + (s >> 2)) * 256 + (s & 3);
+        const float e[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) blk[4 * ((16 * k + 4 * q + j) ^ k)] = e[j];
     }
 }
 

@@ -202,20 +202,6 @@ constexpr int64_t MQ_MIN_VECTORS = 4096;
 // The B operand is C[code] of index 4s + g; each of a vector's four lanes loads the whole
 // code row and takes its own indices from it.
 
-// cv[s] = C[code of index 4s + g] for s = 0..31.  Index 4s + g sits at bit (4s + g) BITS of the
-// code row w, inside the 64-bit window that starts at word 4s BITS / 32 (its field ends within
-// 16 bits of bit 4s BITS); w has one zero word past the row's end.  The word indices are
-// template constants so that the row stays in registers.
-template <int BITS, int... S>
-__device__ __forceinline__ void centers_of(const uint32_t* w, int g, const float* cent, float* cv,
-                                           std::integer_sequence<int, S...>) {
-    constexpr uint32_t MASK = (1u << BITS) - 1u;
-    ((cv[S] = cent[(uint32_t)(((uint64_t)w[(4 * S * BITS) >> 5] | ((uint64_t)w[((4 * S * BITS) >> 5) + 1] << 32)) >>
-                               (((4 * S * BITS) & 31) + g * BITS)) &
-                   MASK]),
-     ...);
-}
-
 template <int BITS, bool QJL, int PARTS>
 __global__ __launch_bounds__(MQ_THREADS) void dequantize_kernel(
     const uint8_t* __restrict__ codes, const uint16_t* __restrict__ norms, const uint8_t* __restrict__ signs,
@@ -223,12 +209,6 @@ __global__ __launch_bounds__(MQ_THREADS) void dequantize_kernel(
     const float* __restrict__ centers, const float* __restrict__ S, uint16_t* __restrict__ out, FastDiv tok_div) {
     __shared__ float4 s_img[(QJL ? 2 : 1) * D * D / 4];  // R^T image (+ S^T image)
     __shared__ float s_cent[1 << BITS];
-    float* img = reinterpret_cast<float*>(s_img);
-    build_image_transposed(img, R);
-    if constexpr (QJL) build_image_transposed(img + D * D, S);
-    if (threadIdx.x < (1 << BITS)) s_cent[threadIdx.x] = centers[threadIdx.x];
-    __syncthreads();  // the only barrier: each wave then works on its own tiles
-
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int v = lane & 15, g = lane >> 4;
     constexpr int NT = 8 / PARTS;  // row tiles (16 output dims each) per work item
@@ -238,62 +218,74 @@ __global__ __launch_bounds__(MQ_THREADS) void dequantize_kernel(
 
     // work item = (tile of 16 vectors, part): part p computes row tiles [p NT, p NT + NT), the
     // dims 32g + [4 p NT, 4 p NT + 4 NT) of each of lane 16 g + v's vector
-    for (int64_t item = (int64_t)blockIdx.x * MQ_WAVES + wave; item < n_items;
-         item += (int64_t)gridDim.x * MQ_WAVES) {
+    uint4 raw[BITS], raw_sign;
+    uint32_t raw_norm = 0u, raw_rnorm = 0u;
+    auto fetch = [&](int64_t item) {
+        const uint32_t vi = (uint32_t)(item / PARTS) * 16u + (uint32_t)v;  // n_vec < 2^31
+        // a lane past the end reads slot 0's row, which exists, and stores nothing
+        int64_t slot = 0;
+        if (item < n_items && vi < (uint64_t)n_vec) {
+            const uint32_t gh = fdiv(vi, tok_div);
+            slot = (int64_t)gh * cap + (vi - gh * (uint32_t)tokens);
+        }
+        const uint4* c4 = reinterpret_cast<const uint4*>(codes + slot * ROW);
+#pragma unroll
+        for (int c = 0; c < BITS; ++c) raw[c] = c4[c];
+        raw_norm = norms[slot];
+        if constexpr (QJL) {
+            raw_sign = reinterpret_cast<const uint4*>(signs + slot * (D / 8))[0];
+            raw_rnorm = rnorms[slot];
+        }
+    };
+    // the first item's rows are on their way while the images are built
+    int64_t item = (int64_t)blockIdx.x * MQ_WAVES + wave;
+    fetch(item);
+    float* img = reinterpret_cast<float*>(s_img);
+    build_image_transposed(img, R);
+    if constexpr (QJL) build_image_transposed(img + D * D, S);
+    if (threadIdx.x < (1 << BITS)) s_cent[threadIdx.x] = centers[threadIdx.x];
+    __syncthreads();  // the only barrier: each wave then works on its own tiles
+
+    for (; item < n_items; item += (int64_t)gridDim.x * MQ_WAVES) {
         const int64_t tile = item / PARTS;
         const int t0 = (int)(item % PARTS) * NT;
         const float4* a_img = s_img + t0 * 8 * 64 + (lane ^ g);
         const uint32_t vi = (uint32_t)tile * 16u + (uint32_t)v;  // n_vec < 2^31
         const bool live = vi < (uint64_t)n_vec;
-        int64_t slot = 0;
-        if (live) {
-            const uint32_t gh = fdiv(vi, tok_div);
-            slot = (int64_t)gh * cap + (vi - gh * (uint32_t)tokens);
-        }
-        // the code row (a lane past the end reads slot 0's, which exists, and stores nothing),
-        // one zero word past its end
-        uint32_t w[RW + 1];
-        {
-            const uint4* c4 = reinterpret_cast<const uint4*>(codes + slot * ROW);
+        uint32_t w[RW + 1];  // the code row, one zero word past its end
 #pragma unroll
-            for (int c = 0; c < BITS; ++c) {
-                const uint4 q = c4[c];
-                w[4 * c] = q.x, w[4 * c + 1] = q.y, w[4 * c + 2] = q.z, w[4 * c + 3] = q.w;
-            }
-            w[RW] = 0u;
-        }
+        for (int c = 0; c < BITS; ++c)
+            w[4 * c] = raw[c].x, w[4 * c + 1] = raw[c].y, w[4 * c + 2] = raw[c].z, w[4 * c + 3] = raw[c].w;
+        w[RW] = 0u;
+        const float nf = tq::f16_to_f32(raw_norm);
+        const uint4 sw = raw_sign;
+        const float rn = tq::f16_to_f32(raw_rnorm);
         float cv[32];
-        centers_of<BITS>(w, g, s_cent, cv, std::make_integer_sequence<int, 32>{});
+        centers_of<BITS>(w, g, s_cent, cv);
+        // the next item's rows beside this one's products (Q_mse kernels, four waves on a SIMD, would
+        // lose one to the registers)
+        if (QJL) fetch(item + (int64_t)gridDim.x * MQ_WAVES);
         f32x4 acc[NT];
         image_products<NT>(a_img, cv, acc);
-        const float nf = live ? tq::f16_to_f32(norms[slot]) : 0.0f;
         uint32_t kh[2 * NT];  // bf16 pairs of dims 32g + 4 t0 + 2p, + 2p + 1
 #pragma unroll
         for (int p = 0; p < 2 * NT; ++p)
-            kh[p] = tq::f32_to_bf16(acc[p >> 1][2 * (p & 1)] * nf) |
-                    (tq::f32_to_bf16(acc[p >> 1][2 * (p & 1) + 1] * nf) << 16);
+            kh[p] = bf16_pair(acc[p >> 1][2 * (p & 1)] * nf, acc[p >> 1][2 * (p & 1) + 1] * nf);
         if constexpr (QJL) {
             // sign of index 4s + g: word s / 8, bit 4 (s % 8) + g of the 16-byte sign row
-            uint4 sw = make_uint4(0u, 0u, 0u, 0u);
-            float rn = 0.0f;
-            if (live) {
-                sw = reinterpret_cast<const uint4*>(signs + slot * (D / 8))[0];
-                rn = tq::f16_to_f32(rnorms[slot]);
-            }
-            const uint32_t sws[4] = {sw.x, sw.y, sw.z, sw.w};
+            // +-1: the inverted bit as the sign
+            const uint32_t sws[4] = {~sw.x >> g, ~sw.y >> g, ~sw.z >> g, ~sw.w >> g};
             float sv[32];
 #pragma unroll
-            for (int s = 0; s < 32; ++s) sv[s] = ((sws[s >> 3] >> (4 * (s & 7) + g)) & 1u) ? 1.0f : -1.0f;
+            for (int s = 0; s < 32; ++s)
+                sv[s] = __uint_as_float(((sws[s >> 3] << (31 - 4 * (s & 7))) & 0x80000000u) | 0x3F800000u);
             f32x4 pacc[NT];
             image_products<NT>(a_img + D * D / 4, sv, pacc);
             const float qs = 1.2533141373155003f / D;  // sqrt(pi/2)/D rounded to fp32
 #pragma unroll
             for (int p = 0; p < 2 * NT; ++p) {
-                const float c0 = tq::bf16_to_f32(tq::f32_to_bf16((pacc[p >> 1][2 * (p & 1)] * rn) * qs));
-                const float c1 = tq::bf16_to_f32(tq::f32_to_bf16((pacc[p >> 1][2 * (p & 1) + 1] * rn) * qs));
-                const float k0 = tq::bf16_to_f32(kh[p] & 0xFFFFu) + c0;
-                const float k1 = tq::bf16_to_f32(kh[p] >> 16) + c1;
-                kh[p] = tq::f32_to_bf16(k0) | (tq::f32_to_bf16(k1) << 16);
+                const uint32_t c = bf16_pair((pacc[p >> 1][2 * (p & 1)] * rn) * qs, (pacc[p >> 1][2 * (p & 1) + 1] * rn) * qs);
+                kh[p] = bf16_pair(lo_half(kh[p]) + lo_half(c), hi_half(kh[p]) + hi_half(c));
             }
         }
         if (live) {
@@ -301,6 +293,7 @@ __global__ __launch_bounds__(MQ_THREADS) void dequantize_kernel(
 #pragma unroll
             for (int i = 0; i < NT / 2; ++i) o4[i] = make_uint4(kh[4 * i], kh[4 * i + 1], kh[4 * i + 2], kh[4 * i + 3]);
         }
+        if (!QJL) fetch(item + (int64_t)gridDim.x * MQ_WAVES);
     }
 }
 
