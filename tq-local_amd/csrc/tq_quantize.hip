@@ -52,11 +52,6 @@ __device__ __forceinline__ uint32_t bucket_count(float z, const float* __restric
 // banks for the 16 lanes of an LDS pass, and thread d reading column d (the residual decode)
 // touches consecutive banks.  The norms are fma chains over the vector held in LDS, run by
 // every thread of the vector (the same operands in the same order: one value in all of them).
-//
-// A call of few vectors is a chain of latencies, so the vector is asked for first, then the
-// matrices, whose 128 KB arrive beside its norm chain; the index is divided by multiplication.  A
-// call of more vectors than the device holds workgroups (132 KB of LDS) walks them with the
-// matrices staged once.  K + V of 8 vectors 13.8 -> 11.0 us, of 2408 vectors 36.5 -> 24 us.
 constexpr int AV = 4;          // vectors per workgroup
 constexpr int AT = AV * D;     // threads per workgroup
 constexpr int MS = D + 4;      // LDS row stride of a staged matrix, floats
@@ -67,7 +62,7 @@ __global__ __launch_bounds__(AT) void append_kernel(
     int64_t x_st, const float* __restrict__ R, const float* __restrict__ centers,
     const float* __restrict__ boundaries, const float* __restrict__ S, uint8_t* __restrict__ codes,
     uint16_t* __restrict__ norms, uint8_t* __restrict__ signs, uint16_t* __restrict__ rnorms, int64_t out_cap,
-    int64_t out_offset, FastDiv tok_div, FastDiv head_div) {
+    int64_t out_offset) {
     __shared__ float4 sR[D * MS / 4];
     __shared__ float4 sS[PROD ? D * MS / 4 : 1];
     __shared__ float4 sx[AV][D / 4];    // the vector in fp32, later rhat
@@ -75,153 +70,121 @@ __global__ __launch_bounds__(AT) void append_kernel(
     __shared__ float4 sc[AV][D / 4];    // C[code_j]
     __shared__ uint8_t scode[AV][D];
     __shared__ float scent[1 << BITS];
-    __shared__ float sbound[(1 << BITS) - 1];
 
     const int tid = threadIdx.x;
     const int vi = tid / D, j = tid % D;  // vector of the workgroup (two whole waves), output index
+    const int64_t v = (int64_t)blockIdx.x * AV + vi;
+    const bool active = v < n_vec;        // threads of missing vectors compute on unused LDS, store nothing
     float* const fx = reinterpret_cast<float*>(sx[vi]);
     float* const fu = reinterpret_cast<float*>(su[vi]);
     float* const fc = reinterpret_cast<float*>(sc[vi]);
 
-    // element j of vector v, and its slot; vectors past the end are zeros that store nothing
-    auto element = [&](int64_t v, int64_t* slot) -> uint32_t {
-        if (v >= n_vec) return 0u;
-        int64_t gh, b;
-        if (n_vec < ((int64_t)1 << 31)) {
-            const uint32_t q = fdiv((uint32_t)v, tok_div);
-            gh = q;
-            b = fdiv(q, head_div);
-        } else {
-            gh = v / tokens;
-            b = gh / heads;
-        }
-        const int64_t t = v - gh * tokens, h = gh - b * heads;
-        *slot = gh * out_cap + out_offset + t;
-        return x[b * x_sb + h * x_sh + t * x_st + j];
-    };
-    int64_t v = (int64_t)blockIdx.x * AV + vi, slot = 0;
-    uint32_t xb = element(v, &slot);
-
-    // ---- the matrices on their way (row r at r * MS in LDS), the codebook, the vector
-    constexpr int N = D * D / 4 / AT;
-    f32x4 mR[N], mS[PROD ? N : 1];
-#pragma unroll
-    for (int i = 0; i < N; ++i) mR[i] = reinterpret_cast<const f32x4*>(R)[tid + i * AT];
-    if constexpr (PROD) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) mS[i] = reinterpret_cast<const f32x4*>(S)[tid + i * AT];
-        if (tid < (1 << BITS)) scent[tid] = centers[tid];
+    // ---- the vector, the codebook and the matrices into LDS (row r of a matrix at r * MS)
+    int64_t slot = 0;
+    if (active) {
+        const int64_t t = v % tokens, gh = v / tokens;
+        const int64_t h = gh % heads, b = gh / heads;
+        fx[j] = tq::bf16_to_f32(x[b * x_sb + h * x_sh + t * x_st + j]);
+        slot = gh * out_cap + out_offset + t;
     }
-    if (tid < (1 << BITS) - 1) sbound[tid] = boundaries[tid];
-    bool staged = false;
-    for (; v - vi < n_vec; v += (int64_t)gridDim.x * AV) {
-        const bool active = v < n_vec;
-        const int64_t here = slot;
-        fx[j] = tq::bf16_to_f32(xb);
-        xb = element(v + (int64_t)gridDim.x * AV, &slot);
-        __syncthreads();
+    if (PROD && tid < (1 << BITS)) scent[tid] = centers[tid];
+    for (int k = tid; k < D * D / 4; k += AT) {
+        const int r = k / (D / 4), c4 = k % (D / 4);
+        sR[r * (MS / 4) + c4] = reinterpret_cast<const float4*>(R)[k];
+        if constexpr (PROD) sS[r * (MS / 4) + c4] = reinterpret_cast<const float4*>(S)[k];
+    }
+    __syncthreads();
 
-        // ---- norm, u = x / n
-        float ss = 0.0f;
+    // ---- norm, u = x / n
+    float ss = 0.0f;
+#pragma unroll
+    for (int d4 = 0; d4 < D / 4; ++d4) {
+        const float4 e = sx[vi][d4];
+        ss = __builtin_fmaf(e.x, e.x, ss);
+        ss = __builtin_fmaf(e.y, e.y, ss);
+        ss = __builtin_fmaf(e.z, e.z, ss);
+        ss = __builtin_fmaf(e.w, e.w, ss);
+    }
+    float n = tq::sqrt_rn(ss);
+    if (!(n > 0.0f)) n = 1.0f;
+    const float xj = fx[j];
+    fu[j] = tq::div_rn(xj, n);
+    const uint32_t n16 = tq::f32_to_f16(n);
+    if (active && j == 0) norms[slot] = (uint16_t)n16;
+    __syncthreads();
+
+    // ---- z_j = fma chain d of u_d R[j][d]; code_j
+    float z = 0.0f;
+    {
+        const float4* rj = sR + j * (MS / 4);
 #pragma unroll
         for (int d4 = 0; d4 < D / 4; ++d4) {
-            const float4 e = sx[vi][d4];
-            ss = __builtin_fmaf(e.x, e.x, ss);
-            ss = __builtin_fmaf(e.y, e.y, ss);
-            ss = __builtin_fmaf(e.z, e.z, ss);
-            ss = __builtin_fmaf(e.w, e.w, ss);
+            const float4 uu = su[vi][d4], rr = rj[d4];
+            z = __builtin_fmaf(uu.x, rr.x, z);
+            z = __builtin_fmaf(uu.y, rr.y, z);
+            z = __builtin_fmaf(uu.z, rr.z, z);
+            z = __builtin_fmaf(uu.w, rr.w, z);
         }
-        float n = tq::sqrt_rn(ss);
-        if (!(n > 0.0f)) n = 1.0f;
-        const float xj = fx[j];
-        fu[j] = tq::div_rn(xj, n);
-        const uint32_t n16 = tq::f32_to_f16(n);
-        if (active && j == 0) norms[here] = (uint16_t)n16;
-        if (!staged) {
+    }
+    const uint32_t code = bucket_count<(1 << BITS) - 1>(z, boundaries);
+    scode[vi][j] = (uint8_t)code;
+    if constexpr (PROD) fc[j] = scent[code];
+    __syncthreads();
+
+    // ---- the code row: thread j < ROW / 4 assembles dword j (stream bits [32 j, 32 j + 32))
+    constexpr int ROW = D * BITS / 8;
+    if (active && j < ROW / 4) {
+        const int b0 = 32 * j;
+        uint64_t acc = 0;
+        for (int k = b0 / BITS; k <= (b0 + 31) / BITS; ++k)
+            acc |= (uint64_t)scode[vi][k] << (k * BITS - b0 + 32);  // shift in [33 - BITS, 63]
+        reinterpret_cast<uint32_t*>(codes + slot * ROW)[j] = (uint32_t)(acc >> 32);
+    }
+
+    if constexpr (PROD) {
+        // ---- residual: khat_d = bf16((fma chain jj of C[code_jj] R[jj][d]) * f32(f16(n))), d = j
+        const float* fR = reinterpret_cast<const float*>(sR);
+        float acc = 0.0f;
 #pragma unroll
-            for (int i = 0; i < N; ++i) {
-                const int k = tid + i * AT, at = k / (D / 4) * (MS / 4) + k % (D / 4);
-                reinterpret_cast<f32x4*>(sR)[at] = mR[i];
-                if constexpr (PROD) reinterpret_cast<f32x4*>(sS)[at] = mS[i];
-            }
-            staged = true;
+        for (int k4 = 0; k4 < D / 4; ++k4) {
+            const float4 cc = sc[vi][k4];
+            acc = __builtin_fmaf(cc.x, fR[(4 * k4 + 0) * MS + j], acc);
+            acc = __builtin_fmaf(cc.y, fR[(4 * k4 + 1) * MS + j], acc);
+            acc = __builtin_fmaf(cc.z, fR[(4 * k4 + 2) * MS + j], acc);
+            acc = __builtin_fmaf(cc.w, fR[(4 * k4 + 3) * MS + j], acc);
         }
+        const float kh = tq::bf16_to_f32(tq::f32_to_bf16(acc * tq::f16_to_f32(n16)));
+        const float r = xj - kh;
+        fu[j] = r;  // u was last read by the rotation, before the barrier above
         __syncthreads();
-
-        // ---- z_j = fma chain d of u_d R[j][d]; code_j
-        float z = 0.0f;
-        {
-            const float4* rj = sR + j * (MS / 4);
+        float rs = 0.0f;
 #pragma unroll
-            for (int d4 = 0; d4 < D / 4; ++d4) {
-                const float4 uu = su[vi][d4], rr = rj[d4];
-                z = __builtin_fmaf(uu.x, rr.x, z);
-                z = __builtin_fmaf(uu.y, rr.y, z);
-                z = __builtin_fmaf(uu.z, rr.z, z);
-                z = __builtin_fmaf(uu.w, rr.w, z);
-            }
+        for (int d4 = 0; d4 < D / 4; ++d4) {
+            const float4 e = su[vi][d4];
+            rs = __builtin_fmaf(e.x, e.x, rs);
+            rs = __builtin_fmaf(e.y, e.y, rs);
+            rs = __builtin_fmaf(e.z, e.z, rs);
+            rs = __builtin_fmaf(e.w, e.w, rs);
         }
-        const uint32_t code = bucket_count<(1 << BITS) - 1>(z, sbound);
-        scode[vi][j] = (uint8_t)code;
-        if constexpr (PROD) fc[j] = scent[code];
+        float rho = tq::sqrt_rn(rs);
+        if (!(rho > 0.0f)) rho = 1.0f;
+        fx[j] = tq::div_rn(r, rho);  // x was last read before the first barrier
+        if (active && j == 0) rnorms[slot] = (uint16_t)tq::f32_to_f16(rho);
         __syncthreads();
-
-        // ---- the code row: thread j < ROW / 4 assembles dword j (stream bits [32 j, 32 j + 32))
-        constexpr int ROW = D * BITS / 8;
-        if (active && j < ROW / 4) {
-            const int b0 = 32 * j;
-            uint64_t acc = 0;
-            for (int k = b0 / BITS; k <= (b0 + 31) / BITS; ++k)
-                acc |= (uint64_t)scode[vi][k] << (k * BITS - b0 + 32);  // shift in [33 - BITS, 63]
-            reinterpret_cast<uint32_t*>(codes + here * ROW)[j] = (uint32_t)(acc >> 32);
+        // ---- sign_i = (fma chain d of rhat_d S[i][d]) >= 0, i = j; a wave holds 64 of them
+        float p = 0.0f;
+        const float4* si = sS + j * (MS / 4);
+#pragma unroll
+        for (int d4 = 0; d4 < D / 4; ++d4) {
+            const float4 hh = sx[vi][d4], ww = si[d4];
+            p = __builtin_fmaf(hh.x, ww.x, p);
+            p = __builtin_fmaf(hh.y, ww.y, p);
+            p = __builtin_fmaf(hh.z, ww.z, p);
+            p = __builtin_fmaf(hh.w, ww.w, p);
         }
-
-        if constexpr (PROD) {
-            // ---- residual: khat_d = bf16((fma chain jj of C[code_jj] R[jj][d]) * f32(f16(n))), d = j
-            const float* fR = reinterpret_cast<const float*>(sR);
-            float acc = 0.0f;
-#pragma unroll
-            for (int k4 = 0; k4 < D / 4; ++k4) {
-                const float4 cc = sc[vi][k4];
-                acc = __builtin_fmaf(cc.x, fR[(4 * k4 + 0) * MS + j], acc);
-                acc = __builtin_fmaf(cc.y, fR[(4 * k4 + 1) * MS + j], acc);
-                acc = __builtin_fmaf(cc.z, fR[(4 * k4 + 2) * MS + j], acc);
-                acc = __builtin_fmaf(cc.w, fR[(4 * k4 + 3) * MS + j], acc);
-            }
-            const float kh = tq::bf16_to_f32(tq::f32_to_bf16(acc * tq::f16_to_f32(n16)));
-            const float r = xj - kh;
-            fu[j] = r;  // u was last read by the rotation, before the barrier above
-            __syncthreads();
-            float rs = 0.0f;
-#pragma unroll
-            for (int d4 = 0; d4 < D / 4; ++d4) {
-                const float4 e = su[vi][d4];
-                rs = __builtin_fmaf(e.x, e.x, rs);
-                rs = __builtin_fmaf(e.y, e.y, rs);
-                rs = __builtin_fmaf(e.z, e.z, rs);
-                rs = __builtin_fmaf(e.w, e.w, rs);
-            }
-            float rho = tq::sqrt_rn(rs);
-            if (!(rho > 0.0f)) rho = 1.0f;
-            fx[j] = tq::div_rn(r, rho);  // x was last read before the first barrier
-            if (active && j == 0) rnorms[here] = (uint16_t)tq::f32_to_f16(rho);
-            __syncthreads();
-            // ---- sign_i = (fma chain d of rhat_d S[i][d]) >= 0, i = j; a wave holds 64 of them
-            float p = 0.0f;
-            const float4* si = sS + j * (MS / 4);
-#pragma unroll
-            for (int d4 = 0; d4 < D / 4; ++d4) {
-                const float4 hh = sx[vi][d4], ww = si[d4];
-                p = __builtin_fmaf(hh.x, ww.x, p);
-                p = __builtin_fmaf(hh.y, ww.y, p);
-                p = __builtin_fmaf(hh.z, ww.z, p);
-                p = __builtin_fmaf(hh.w, ww.w, p);
-            }
-            const uint64_t sb = __builtin_amdgcn_ballot_w64(p >= 0.0f);  // bit l: index 64 (j / 64) + l
-            if (active && (j & 63) == 0)
-                reinterpret_cast<uint2*>(signs + here * (D / 8))[j >> 6] = make_uint2((uint32_t)sb, (uint32_t)(sb >> 32));
-        }
-        __syncthreads();  // every thread is done with the vector
+        const uint64_t sb = __builtin_amdgcn_ballot_w64(p >= 0.0f);  // bit l: index 64 (j / 64) + l
+        if (active && (j & 63) == 0)
+            reinterpret_cast<uint2*>(signs + slot * (D / 8))[j >> 6] = make_uint2((uint32_t)sb, (uint32_t)(sb >> 32));
     }
 }
 
@@ -373,12 +336,9 @@ template <int BITS, bool PROD>
 int launch_append(const tqenc::EncodeArgs& a, hipStream_t s) {
     const int64_t blocks = (a.n_vec + AV - 1) / AV;
     if (blocks == 0) return TQ_OK;
-    static_assert(AT == MQ_THREADS, "resident_groups counts workgroups of this size");
-    const int64_t groups = std::min<int64_t>(blocks, resident_groups<append_kernel<BITS, PROD>>());
-    hipLaunchKernelGGL((append_kernel<BITS, PROD>), dim3((unsigned)groups), dim3(AT), 0, s, a.x, a.heads,
+    hipLaunchKernelGGL((append_kernel<BITS, PROD>), dim3((unsigned)blocks), dim3(AT), 0, s, a.x, a.heads,
                        a.tokens, a.n_vec, a.x_sb, a.x_sh, a.x_st, a.R, a.centers, a.boundaries, a.S, a.codes,
-                       a.norms, a.signs, a.rnorms, a.out_cap, a.out_offset,
-                       make_fastdiv((uint32_t)std::min<int64_t>(a.tokens, 0x7FFFFFFF)), make_fastdiv((uint32_t)a.heads));
+                       a.norms, a.signs, a.rnorms, a.out_cap, a.out_offset);
     TQ_CHECK_LAUNCH();
     return TQ_OK;
 }
