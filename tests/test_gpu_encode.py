@@ -58,11 +58,11 @@ def compare(x, got, ref, T):
         assert np.array_equal(a, b), f"{name}: {(a != b).sum()} of {b.size} differ"
 
 
+@pytest.mark.parametrize("T", [521, 12 * 1024 + 5, 25 * 1024 + 5])  # a tile per workgroup, one and two per wave
 @pytest.mark.parametrize("rotation", ["haar", "permutation"])
 @pytest.mark.parametrize("bits,prod", [(1, False), (2, False), (3, False), (4, False), (1, True), (2, True), (3, True)])
-def test_plain_prefill_encoder_on_hard_rows(cuda, bits, prod, rotation):
+def test_plain_prefill_encoder_on_hard_rows(cuda, bits, prod, rotation, T):
     """A permutation matrix as the rotation puts z = u on the boundaries below exactly."""
-    T = 2 * 1024 + 37 if bits % 2 else 17 * 1024 + 5  # one and four tiles per wave
     x = hard_rows(T, 3 * bits + prod)
     lc = layer_codecs(D, bits + 1 if prod else bits, 0, prod, cuda)
     c = lc.key if prod else lc.value
@@ -85,11 +85,11 @@ def test_plain_prefill_encoder_on_hard_rows(cuda, bits, prod, rotation):
         compare(x, (kc, kn), O.encode_mse(rows, bits, h[0], h[2]), T)
 
 
+@pytest.mark.parametrize("T", [521, 8192 + 19, 12 * 1024 + 19])
 @pytest.mark.parametrize("d,bits,extra,qjl", [(3, 4, 1, True), (4, 4, 4, False), (8, 3, 4, True), (13, 2, 3, False),
                                               (33, 1, 1, False), (40, 2, 2, True), (60, 4, 3, True)])
-def test_group_prefill_encoder_on_hard_rows(cuda, d, bits, extra, qjl):
+def test_group_prefill_encoder_on_hard_rows(cuda, d, bits, extra, qjl, T):
     """Both groups of a split, the outlier group up to 8 bits (7 with the sketch)."""
-    T = 4096 + 19 if d % 2 else 16 * 1024 + 19
     outl = np.sort(np.random.default_rng(d).choice(D, d, replace=False))
     sc = split_codecs(np.setdiff1d(np.arange(D), outl), outl, bits, extra, 0, qjl, cuda)
     x = hard_rows(T, d)

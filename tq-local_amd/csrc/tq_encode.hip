@@ -880,6 +880,194 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
     }
 }
 
+// ------------------------------------------------------------------ calls of few vectors
+// The chains themselves, on the fp32 matrix cores: a workgroup of eight waves encodes a tile of 16
+// vectors, wave w the outputs [16 w, 16 w + 16) of each product (32 v_mfma_f32_16x16x4_f32, the fma
+// chain over d = 4 s + k), and the vectors meet in LDS between the products.  Lane 16 g + v feeds
+// element 4 s + g of vector v and gets back outputs 16 w + 4 g + (0..3) of it.  The matrices are staged
+// in LDS once per workgroup, rows MS floats apart (reads of one column block by 16 rows and four
+// columns hit 64 banks).  The norms are chains of 128 fma that every wave runs for all 16 vectors, one
+// lane each (four alike), while its SIMD's other wave does the same.
+//
+// Latency-bound while a CU has one tile (up to 4096 vectors): the matrices' arrival and six barriers'
+// worth of chains; beyond, about 8 us a tile with the sketch and 4 without, of which the products'
+// issue is a quarter.  3-bit keys with the sketch / 4-bit values, us: one thread per output (the kernel
+// below 1024 vectors) 24.5 / 9.2 at 2408 vectors and 31.8 / 11.4 at 4096, this one 11.1 / 6.4 and
+// 11.5 / 6.7.
+//
+// The lines: up to 1024 vectors the one-thread-per-output kernels have a workgroup of four vectors per
+// CU and are ahead (8.6 / 4.6 against 10.1 / 5.8 at 8, 9.8 / 5.3 against 10.7 / 6.3 at 1024); their
+// callers keep those.  From TILE_MAX_* vectors the kernels above are: with the sketch 33.8 here against
+// 46.5 there at 16384, 49.4 against 48.7 at 24576; without, 17.8 against 21.0 at 16384 and 25.3 against
+// 18.9 at 24576 (channel groups the same within 10%).
+constexpr int64_t TILE_MAX_PROD = 24576, TILE_MAX_MSE = 20480;
+constexpr int MS = D + 4;
+constexpr int BS = 36;  // floats between lanes' 32 elements in the exchange buffers
+
+__device__ __forceinline__ int lane_slot(int v, int g) { return (4 * v + g) * BS; }
+
+template <int BITS, bool GROUP, bool PROD>
+__global__ __launch_bounds__(MQ_THREADS) void tile_kernel(EncodeArgs a) {
+    constexpr int NB = (1 << BITS) - 1;
+    __shared__ float s_r[D * MS];
+    __shared__ float s_s[PROD ? D * MS : 1];
+    __shared__ float4 s_a[64 * BS / 4];  // x as rows of MS floats; then C[code], then rhat, by lane
+    __shared__ float4 s_b[64 * BS / 4];  // u by lane; then the residual as rows
+    __shared__ uint8_t s_code[16][D];
+    __shared__ float s_bound[NB];
+    __shared__ float s_cent[PROD ? NB + 1 : 1];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int v = lane & 15, g = lane >> 4;
+    const int sub_dim = GROUP ? a.sub_dim : D;
+    const int row_bytes = GROUP ? (sub_dim * BITS + 7) >> 3 : D * BITS / 8;
+    const int sign_bytes = (sub_dim + 7) >> 3;
+    float* const fa = reinterpret_cast<float*>(s_a);
+    float* const fb = reinterpret_cast<float*>(s_b);
+    const uint32_t mw = a.mask[wave >> 1] >> (16 * (wave & 1) + 4 * g);  // this lane's four channels
+
+    // channels 16 wave + 4 g + (0..3) of vector tile * 16 + v
+    auto fetch = [&](int64_t tile, int64_t* slot) -> uint2 {
+        const int64_t vi = tile * 16 + v;
+        uint2 w = make_uint2(0u, 0u);
+        *slot = -1;
+        if (vi < a.n_vec) {
+            w = reinterpret_cast<const uint2*>(row_of(a, (uint32_t)vi, slot))[4 * wave + g];
+            if constexpr (GROUP) w.x &= pair_mask(mw, 0), w.y &= pair_mask(mw, 1);
+        }
+        return w;
+    };
+    const int64_t n_tiles = (a.n_vec + 15) / 16;
+    int64_t next_slot;
+    uint2 next = fetch(blockIdx.x, &next_slot);
+
+    {
+        constexpr int N = D * D / 4 / MQ_THREADS;
+        f32x4 m[N], p[PROD ? N : 1];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            m[i] = reinterpret_cast<const f32x4*>(a.R)[threadIdx.x + i * MQ_THREADS];
+            if constexpr (PROD) p[i] = reinterpret_cast<const f32x4*>(a.S)[threadIdx.x + i * MQ_THREADS];
+        }
+        for (int i = threadIdx.x; i < NB; i += MQ_THREADS) s_bound[i] = a.boundaries[i];
+        if constexpr (PROD)
+            for (int i = threadIdx.x; i <= NB; i += MQ_THREADS) s_cent[i] = a.centers[i];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int at = threadIdx.x + i * MQ_THREADS, dst = (at >> 5) * MS + 4 * (at & 31);
+            *reinterpret_cast<f32x4*>(s_r + dst) = m[i];
+            if constexpr (PROD) *reinterpret_cast<f32x4*>(s_s + dst) = p[i];
+        }
+    }
+    // product of 16 rows (row m at `rows` + m * step_m, element 4 s + k at 4 s * step_k + k * step_k) with the 16
+    // vectors whose elements lane 16 g + v finds at src
+    auto product = [&](const float* rows, int step_m, int step_k, const float* src) {
+        f32x4 b[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) b[c] = *reinterpret_cast<const f32x4*>(src + lane_slot(v, g) + 4 * c);
+        const float* am = rows + v * step_m + g * step_k;
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < 32; ++s) acc = mfma_f32(am[4 * s * step_k], b[s >> 2][s & 3], acc);
+        return acc;
+    };
+    // sum of squares of row v as a chain, then its root (0 -> 1)
+    auto norm_of = [&](const float* rows) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int c = 0; c < D / 4; ++c) {
+            const f32x4 e = *reinterpret_cast<const f32x4*>(rows + v * MS + 4 * c);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) ss = __builtin_fmaf(e[k], e[k], ss);
+        }
+        const float n = tq::sqrt_rn(ss);
+        return n > 0.0f ? n : 1.0f;
+    };
+    // element i of this lane's four goes to the lane that feeds it: dim 16 wave + 4 g + i = 4 (4 wave + g) + i
+    auto deal = [&](float* dst, int i, float e) { dst[lane_slot(v, i) + 4 * wave + g] = e; };
+
+    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+        const int64_t slot = next_slot;
+        const float x[4] = {lo_half(next.x), hi_half(next.x), lo_half(next.y), hi_half(next.y)};
+        next = fetch(tile + gridDim.x, &next_slot);
+        *reinterpret_cast<f32x4*>(fa + v * MS + 16 * wave + 4 * g) = f32x4{x[0], x[1], x[2], x[3]};
+        __syncthreads();
+        const float n = norm_of(fa);
+        const uint32_t n16 = tq::f32_to_f16(n);
+        if (wave == 0 && g == 0 && slot >= 0) a.norms[slot] = (uint16_t)n16;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) deal(fb, i, tq::div_rn(x[i], n));
+        __syncthreads();
+
+        // ---- z_j, codes
+        const f32x4 z = product(s_r + 16 * wave * MS, MS, 1, fb);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int j = 16 * wave + 4 * g + i;
+            const uint32_t code = !GROUP || j < sub_dim ? bucket_lds(z[i], s_bound, BITS) : 0u;
+            s_code[v][j] = (uint8_t)code;
+            if constexpr (PROD) deal(fa, i, !GROUP || j < sub_dim ? s_cent[code] : 0.0f);
+        }
+        __syncthreads();
+        // ---- the code rows: stream bits [32 k, 32 k + 32) of vector t / 32 by thread t = 32 vector + k
+        {
+            const int t = threadIdx.x >> 5, k = threadIdx.x & 31;
+            // the tile's slots live in the lanes of vector t
+            const int64_t row_slot = __shfl(slot, (t & 15));
+            if (k < 4 * BITS && 4 * k < row_bytes && row_slot >= 0) {
+                const int b0 = 32 * k, last = std::min((b0 + 31) / BITS, sub_dim - 1);
+                uint64_t acc = 0;
+                for (int j = b0 / BITS; j <= last; ++j)
+                    acc |= (uint64_t)s_code[t][j] << (j * BITS - b0 + 32);  // shift in [33 - BITS, 63]
+                const uint32_t word = (uint32_t)(acc >> 32);
+                uint8_t* dst = a.codes + row_slot * row_bytes + 4 * k;
+                const int left = row_bytes - 4 * k;
+                if (!GROUP) {
+                    *reinterpret_cast<uint32_t*>(dst) = word;
+                } else if (left >= 4) {
+                    __builtin_memcpy(dst, &word, 4);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 3; ++e)
+                        if (e < left) dst[e] = (uint8_t)(word >> (8 * e));
+                }
+            }
+        }
+        if constexpr (PROD) {
+            // ---- residual: khat_d = bf16((chain j of C[code_j] R[j][d]) * f32(f16(n))), d = 16 wave + 4 g + i
+            const f32x4 kh = product(s_r + 16 * wave, 1, MS, fa);
+            const float nf = tq::f16_to_f32(n16);
+            f32x4 r;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r[i] = x[i] - tq::bf16_to_f32(tq::f32_to_bf16(kh[i] * nf));
+            *reinterpret_cast<f32x4*>(fb + v * MS + 16 * wave + 4 * g) = r;  // u was read before the barrier above
+            __syncthreads();
+            const float rho = norm_of(fb);
+            if (wave == 0 && g == 0 && slot >= 0) a.rnorms[slot] = (uint16_t)tq::f32_to_f16(rho);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) deal(fa, i, tq::div_rn(r[i], rho));
+            __syncthreads();
+            // ---- signs
+            const f32x4 p = product(s_s + 16 * wave * MS, MS, 1, fa);
+            uint32_t bits = 0u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (!GROUP || 16 * wave + 4 * g + i < sub_dim) bits |= (p[i] >= 0.0f ? 1u : 0u) << (4 * g + i);
+            bits |= (uint32_t)__shfl_xor((int)bits, 16);
+            bits |= (uint32_t)__shfl_xor((int)bits, 32);
+            if (g == 0 && slot >= 0) {
+                uint8_t* dst = a.signs + slot * sign_bytes + 2 * wave;
+                if (!GROUP) {
+                    *reinterpret_cast<uint16_t*>(dst) = (uint16_t)bits;
+                } else {
+                    if (2 * wave < sign_bytes) dst[0] = (uint8_t)bits;
+                    if (2 * wave + 1 < sign_bytes) dst[1] = (uint8_t)(bits >> 8);
+                }
+            }
+        }
+        __syncthreads();  // every wave is done with the tile
+    }
+}
+
 // Workgroups of a kernel that fit on the device at once (each loops over tiles, so more would only
 // repeat the LDS set-up).
 template <auto KERNEL>
@@ -904,6 +1092,10 @@ int launch(const EncodeArgs& a, int64_t groups, int threads, hipStream_t s) {
 template <int BITS, bool GROUP>
 int encode(const EncodeArgs& a, hipStream_t s) {
     const int64_t tiles = (a.n_vec + 15) / 16;
+    if (a.n_vec < (a.S ? TILE_MAX_PROD : TILE_MAX_MSE)) {
+        if (!a.S) return launch<tile_kernel<BITS, GROUP, false>>(a, tiles, MQ_THREADS, s);
+        if constexpr (GROUP || BITS <= 3) return launch<tile_kernel<BITS, GROUP, true>>(a, tiles, MQ_THREADS, s);
+    }
     // two tiles per wave share each matrix fragment read from LDS; a call with fewer tiles than the
     // device has waves spreads them instead
     const int64_t waves = resident<codes_kernel<BITS, GROUP, 2>>(CT) * CW;

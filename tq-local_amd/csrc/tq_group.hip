@@ -20,7 +20,8 @@
 // therefore bit-identical to the plain encoder / decoder run at D = d on the gathered
 // sub-vectors, which is how the CPU oracle states them.
 //
-// Calls of at least GQ_SMALL vectors take the prefill encoder of tq_encode.hip.  The decoder of
+// Calls of at least GQ_SMALL vectors take the prefill encoders of tq_encode.hip, where the line's
+// figures stand.  The decoder of
 // groups up to 24 channels holds a vector per lane; wider ones run on the fp32 matrix cores
 // (dequantize_group_mfma_kernel below, with the chains of tq_mfma.h): same chains, same bits.
 //
@@ -66,7 +67,7 @@ __device__ __forceinline__ uint32_t bucket_lds(float z, const float* s_b, int bi
 constexpr int GAV = 4;                 // vectors per workgroup
 constexpr int GAT = GAV * D;           // threads per workgroup
 constexpr int GMS = D + 4;             // LDS row stride of a staged matrix, floats
-constexpr int64_t GQ_SMALL = 8192;     // below this many vectors the small-batch kernel runs
+constexpr int64_t GQ_SMALL = 1025;     // below this many vectors the small-batch kernel runs
 
 template <bool PROD>
 __global__ __launch_bounds__(GAT) void quantize_group_small_kernel(

@@ -11,8 +11,9 @@
 //                     r = x - khat;  rho = sqrt_rn(fma chain r_d^2) (0 -> 1);  rhat = r /_rn rho
 //                     sign_i = (fma chain d of rhat_d*S[i][d]) >= 0
 //
-// Two encoders: the one of tq_encode.hip for calls of at least MQ_MIN_VECTORS vectors (prefill)
-// and a small-batch kernel with one thread per output index of each vector (decode-append).
+// Two encoders: those of tq_encode.hip for calls of at least MQ_MIN_VECTORS vectors (prefill; the
+// figures at the line stand there) and a small-batch kernel with one thread per output index of each
+// vector (decode-append).
 //
 // Reference: runtime/packed_qmse_cache.py:376-402 (_encode_group), :285-310
 // (_encode_keys_qjl_group), :404-435 (_decode_group), :13-43 (_pack_indices),
@@ -189,7 +190,7 @@ __global__ __launch_bounds__(AT) void append_kernel(
 }
 
 // At least this many vectors take the prefill encoder (tq_encode.hip).
-constexpr int64_t MQ_MIN_VECTORS = 4096;
+constexpr int64_t MQ_MIN_VECTORS = 1025;
 
 // ------------------------------------------------------------------- decoders
 // out = bf16((C[code] @ R) * f32(norm)); with QJL (keys of Q_prod) the reference's
