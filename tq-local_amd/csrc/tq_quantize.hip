@@ -53,17 +53,22 @@ __device__ __forceinline__ uint32_t bucket_count(float z, const float* __restric
 // banks for the 16 lanes of an LDS pass, and thread d reading column d (the residual decode)
 // touches consecutive banks.  The norms are fma chains over the vector held in LDS, run by
 // every thread of the vector (the same operands in the same order: one value in all of them).
-constexpr int AV = 4;          // vectors per workgroup
-constexpr int AT = AV * D;     // threads per workgroup
+//
+// A call of few vectors is bound by one workgroup's LDS reads along five chains of 128 (when the
+// matrices are staged, beside or before the norm, makes no difference).  So the vectors spread over
+// the CUs: one per workgroup while there are that many, the other waves only staging.  3-bit keys with
+// the sketch / 4-bit values at 8 vectors, us: 8.7 / 4.6 with four per workgroup, 8.3 / 4.5 with two,
+// 7.5 / 4.1 with one.
+constexpr int AT = 4 * D;      // threads per workgroup
 constexpr int MS = D + 4;      // LDS row stride of a staged matrix, floats
 
-template <int BITS, bool PROD>
+template <int BITS, bool PROD, int AV>
 __global__ __launch_bounds__(AT) void append_kernel(
     const uint16_t* __restrict__ x, int heads, int64_t tokens, int64_t n_vec, int64_t x_sb, int64_t x_sh,
     int64_t x_st, const float* __restrict__ R, const float* __restrict__ centers,
     const float* __restrict__ boundaries, const float* __restrict__ S, uint8_t* __restrict__ codes,
     uint16_t* __restrict__ norms, uint8_t* __restrict__ signs, uint16_t* __restrict__ rnorms, int64_t out_cap,
-    int64_t out_offset) {
+    int64_t out_offset, FastDiv tok_div, FastDiv head_div) {
     __shared__ float4 sR[D * MS / 4];
     __shared__ float4 sS[PROD ? D * MS / 4 : 1];
     __shared__ float4 sx[AV][D / 4];    // the vector in fp32, later rhat
@@ -74,62 +79,89 @@ __global__ __launch_bounds__(AT) void append_kernel(
 
     const int tid = threadIdx.x;
     const int vi = tid / D, j = tid % D;  // vector of the workgroup (two whole waves), output index
+    const bool works = vi < AV;           // the waves of further vectors only stage and wait
     const int64_t v = (int64_t)blockIdx.x * AV + vi;
-    const bool active = v < n_vec;        // threads of missing vectors compute on unused LDS, store nothing
-    float* const fx = reinterpret_cast<float*>(sx[vi]);
-    float* const fu = reinterpret_cast<float*>(su[vi]);
-    float* const fc = reinterpret_cast<float*>(sc[vi]);
+    const bool active = works && v < n_vec;  // threads of missing vectors compute on unused LDS, store nothing
+    float* const fx = reinterpret_cast<float*>(sx[works ? vi : 0]);
+    float* const fu = reinterpret_cast<float*>(su[works ? vi : 0]);
+    float* const fc = reinterpret_cast<float*>(sc[works ? vi : 0]);
 
-    // ---- the vector, the codebook and the matrices into LDS (row r of a matrix at r * MS)
+    // ---- the matrices, the codebook and the vector into LDS (row r of a matrix at r * MS)
+    constexpr int N = D * D / 4 / AT;
+    f32x4 mR[N], mS[PROD ? N : 1];
+#pragma unroll
+    for (int i = 0; i < N; ++i) mR[i] = reinterpret_cast<const f32x4*>(R)[tid + i * AT];
+    if constexpr (PROD) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) mS[i] = reinterpret_cast<const f32x4*>(S)[tid + i * AT];
+    }
     int64_t slot = 0;
     if (active) {
-        const int64_t t = v % tokens, gh = v / tokens;
-        const int64_t h = gh % heads, b = gh / heads;
+        int64_t gh, b;
+        if (n_vec < ((int64_t)1 << 31)) {
+            const uint32_t q = fdiv((uint32_t)v, tok_div);
+            gh = q;
+            b = fdiv(q, head_div);
+        } else {
+            gh = v / tokens;
+            b = gh / heads;
+        }
+        const int64_t t = v - gh * tokens, h = gh - b * heads;
         fx[j] = tq::bf16_to_f32(x[b * x_sb + h * x_sh + t * x_st + j]);
         slot = gh * out_cap + out_offset + t;
     }
     if (PROD && tid < (1 << BITS)) scent[tid] = centers[tid];
-    for (int k = tid; k < D * D / 4; k += AT) {
-        const int r = k / (D / 4), c4 = k % (D / 4);
-        sR[r * (MS / 4) + c4] = reinterpret_cast<const float4*>(R)[k];
-        if constexpr (PROD) sS[r * (MS / 4) + c4] = reinterpret_cast<const float4*>(S)[k];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int k = tid + i * AT, at = k / (D / 4) * (MS / 4) + k % (D / 4);
+        reinterpret_cast<f32x4*>(sR)[at] = mR[i];
+        if constexpr (PROD) reinterpret_cast<f32x4*>(sS)[at] = mS[i];
     }
     __syncthreads();
 
     // ---- norm, u = x / n
-    float ss = 0.0f;
-#pragma unroll
-    for (int d4 = 0; d4 < D / 4; ++d4) {
-        const float4 e = sx[vi][d4];
-        ss = __builtin_fmaf(e.x, e.x, ss);
-        ss = __builtin_fmaf(e.y, e.y, ss);
-        ss = __builtin_fmaf(e.z, e.z, ss);
-        ss = __builtin_fmaf(e.w, e.w, ss);
-    }
-    float n = tq::sqrt_rn(ss);
-    if (!(n > 0.0f)) n = 1.0f;
-    const float xj = fx[j];
-    fu[j] = tq::div_rn(xj, n);
-    const uint32_t n16 = tq::f32_to_f16(n);
-    if (active && j == 0) norms[slot] = (uint16_t)n16;
-    __syncthreads();
-
-    // ---- z_j = fma chain d of u_d R[j][d]; code_j
-    float z = 0.0f;
-    {
-        const float4* rj = sR + j * (MS / 4);
+    auto norm_of = [](const float4* row) {
+        float ss = 0.0f;
 #pragma unroll
         for (int d4 = 0; d4 < D / 4; ++d4) {
-            const float4 uu = su[vi][d4], rr = rj[d4];
+            const float4 e = row[d4];
+            ss = __builtin_fmaf(e.x, e.x, ss);
+            ss = __builtin_fmaf(e.y, e.y, ss);
+            ss = __builtin_fmaf(e.z, e.z, ss);
+            ss = __builtin_fmaf(e.w, e.w, ss);
+        }
+        const float n = tq::sqrt_rn(ss);
+        return n > 0.0f ? n : 1.0f;
+    };
+    auto chain = [](const float4* a, const float4* b) {
+        float z = 0.0f;
+#pragma unroll
+        for (int d4 = 0; d4 < D / 4; ++d4) {
+            const float4 uu = a[d4], rr = b[d4];
             z = __builtin_fmaf(uu.x, rr.x, z);
             z = __builtin_fmaf(uu.y, rr.y, z);
             z = __builtin_fmaf(uu.z, rr.z, z);
             z = __builtin_fmaf(uu.w, rr.w, z);
         }
+        return z;
+    };
+    float xj = 0.0f, r = 0.0f;
+    uint32_t n16 = 0u;
+    if (works) {
+        const float n = norm_of(sx[vi]);
+        xj = fx[j];
+        fu[j] = tq::div_rn(xj, n);
+        n16 = tq::f32_to_f16(n);
+        if (active && j == 0) norms[slot] = (uint16_t)n16;
     }
-    const uint32_t code = bucket_count<(1 << BITS) - 1>(z, boundaries);
-    scode[vi][j] = (uint8_t)code;
-    if constexpr (PROD) fc[j] = scent[code];
+    __syncthreads();
+
+    // ---- z_j = fma chain d of u_d R[j][d]; code_j
+    if (works) {
+        const uint32_t code = bucket_count<(1 << BITS) - 1>(chain(su[vi], sR + j * (MS / 4)), boundaries);
+        scode[vi][j] = (uint8_t)code;
+        if constexpr (PROD) fc[j] = scent[code];
+    }
     __syncthreads();
 
     // ---- the code row: thread j < ROW / 4 assembles dword j (stream bits [32 j, 32 j + 32))
@@ -144,48 +176,34 @@ __global__ __launch_bounds__(AT) void append_kernel(
 
     if constexpr (PROD) {
         // ---- residual: khat_d = bf16((fma chain jj of C[code_jj] R[jj][d]) * f32(f16(n))), d = j
-        const float* fR = reinterpret_cast<const float*>(sR);
-        float acc = 0.0f;
+        if (works) {
+            const float* fR = reinterpret_cast<const float*>(sR);
+            float acc = 0.0f;
 #pragma unroll
-        for (int k4 = 0; k4 < D / 4; ++k4) {
-            const float4 cc = sc[vi][k4];
-            acc = __builtin_fmaf(cc.x, fR[(4 * k4 + 0) * MS + j], acc);
-            acc = __builtin_fmaf(cc.y, fR[(4 * k4 + 1) * MS + j], acc);
-            acc = __builtin_fmaf(cc.z, fR[(4 * k4 + 2) * MS + j], acc);
-            acc = __builtin_fmaf(cc.w, fR[(4 * k4 + 3) * MS + j], acc);
+            for (int k4 = 0; k4 < D / 4; ++k4) {
+                const float4 cc = sc[vi][k4];
+                acc = __builtin_fmaf(cc.x, fR[(4 * k4 + 0) * MS + j], acc);
+                acc = __builtin_fmaf(cc.y, fR[(4 * k4 + 1) * MS + j], acc);
+                acc = __builtin_fmaf(cc.z, fR[(4 * k4 + 2) * MS + j], acc);
+                acc = __builtin_fmaf(cc.w, fR[(4 * k4 + 3) * MS + j], acc);
+            }
+            r = xj - tq::bf16_to_f32(tq::f32_to_bf16(acc * tq::f16_to_f32(n16)));
+            fu[j] = r;  // u was last read by the rotation, before the barrier above
         }
-        const float kh = tq::bf16_to_f32(tq::f32_to_bf16(acc * tq::f16_to_f32(n16)));
-        const float r = xj - kh;
-        fu[j] = r;  // u was last read by the rotation, before the barrier above
         __syncthreads();
-        float rs = 0.0f;
-#pragma unroll
-        for (int d4 = 0; d4 < D / 4; ++d4) {
-            const float4 e = su[vi][d4];
-            rs = __builtin_fmaf(e.x, e.x, rs);
-            rs = __builtin_fmaf(e.y, e.y, rs);
-            rs = __builtin_fmaf(e.z, e.z, rs);
-            rs = __builtin_fmaf(e.w, e.w, rs);
+        if (works) {
+            const float rho = norm_of(su[vi]);
+            fx[j] = tq::div_rn(r, rho);  // x was last read before the second barrier
+            if (active && j == 0) rnorms[slot] = (uint16_t)tq::f32_to_f16(rho);
         }
-        float rho = tq::sqrt_rn(rs);
-        if (!(rho > 0.0f)) rho = 1.0f;
-        fx[j] = tq::div_rn(r, rho);  // x was last read before the first barrier
-        if (active && j == 0) rnorms[slot] = (uint16_t)tq::f32_to_f16(rho);
         __syncthreads();
         // ---- sign_i = (fma chain d of rhat_d S[i][d]) >= 0, i = j; a wave holds 64 of them
-        float p = 0.0f;
-        const float4* si = sS + j * (MS / 4);
-#pragma unroll
-        for (int d4 = 0; d4 < D / 4; ++d4) {
-            const float4 hh = sx[vi][d4], ww = si[d4];
-            p = __builtin_fmaf(hh.x, ww.x, p);
-            p = __builtin_fmaf(hh.y, ww.y, p);
-            p = __builtin_fmaf(hh.z, ww.z, p);
-            p = __builtin_fmaf(hh.w, ww.w, p);
+        if (works) {
+            const float p = chain(sx[vi], sS + j * (MS / 4));
+            const uint64_t sb = __builtin_amdgcn_ballot_w64(p >= 0.0f);  // bit l: index 64 (j / 64) + l
+            if (active && (j & 63) == 0)
+                reinterpret_cast<uint2*>(signs + slot * (D / 8))[j >> 6] = make_uint2((uint32_t)sb, (uint32_t)(sb >> 32));
         }
-        const uint64_t sb = __builtin_amdgcn_ballot_w64(p >= 0.0f);  // bit l: index 64 (j / 64) + l
-        if (active && (j & 63) == 0)
-            reinterpret_cast<uint2*>(signs + slot * (D / 8))[j >> 6] = make_uint2((uint32_t)sb, (uint32_t)(sb >> 32));
     }
 }
 
@@ -333,15 +351,27 @@ int64_t resident_groups() {
     });
 }
 
-template <int BITS, bool PROD>
-int launch_append(const tqenc::EncodeArgs& a, hipStream_t s) {
-    const int64_t blocks = (a.n_vec + AV - 1) / AV;
-    if (blocks == 0) return TQ_OK;
-    hipLaunchKernelGGL((append_kernel<BITS, PROD>), dim3((unsigned)blocks), dim3(AT), 0, s, a.x, a.heads,
-                       a.tokens, a.n_vec, a.x_sb, a.x_sh, a.x_st, a.R, a.centers, a.boundaries, a.S, a.codes,
-                       a.norms, a.signs, a.rnorms, a.out_cap, a.out_offset);
+template <int BITS, bool PROD, int AV>
+int launch_append_by(const tqenc::EncodeArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL((append_kernel<BITS, PROD, AV>), dim3((unsigned)((a.n_vec + AV - 1) / AV)), dim3(AT), 0, s, a.x,
+                       a.heads, a.tokens, a.n_vec, a.x_sb, a.x_sh, a.x_st, a.R, a.centers, a.boundaries, a.S, a.codes,
+                       a.norms, a.signs, a.rnorms, a.out_cap, a.out_offset, make_fastdiv((uint32_t)a.tokens),
+                       make_fastdiv((uint32_t)a.heads));
     TQ_CHECK_LAUNCH();
     return TQ_OK;
+}
+
+// Vectors per workgroup: as few as leave one workgroup (137 KB of LDS) per CU.  Keys / values, us: 256
+// vectors 8.1 / 4.4 at one, 8.7 / 4.7 at two; 384 14.1 / 5.0 at one, 8.8 / 4.9 at two; 512 8.9 / 4.9 at
+// two, 9.3 / 5.0 at four; 768 16.0 / 5.5 at two, 9.5 / 5.0 at four.
+constexpr int64_t APPEND_ONE = 256, APPEND_TWO = 512;
+
+template <int BITS, bool PROD>
+int launch_append(const tqenc::EncodeArgs& a, hipStream_t s) {
+    if (a.n_vec == 0) return TQ_OK;
+    if (a.n_vec <= APPEND_ONE) return launch_append_by<BITS, PROD, 1>(a, s);
+    if (a.n_vec <= APPEND_TWO) return launch_append_by<BITS, PROD, 2>(a, s);
+    return launch_append_by<BITS, PROD, 4>(a, s);
 }
 
 }  // namespace
