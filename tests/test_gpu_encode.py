@@ -58,8 +58,8 @@ def compare(x, got, ref, T):
         assert np.array_equal(a, b), f"{name}: {(a != b).sum()} of {b.size} differ"
 
 
-# one, two and four vectors per workgroup, a tile per workgroup, one and two tiles per wave
-@pytest.mark.parametrize("T", [1, 128, 129, 257, 521, 12 * 1024 + 5, 25 * 1024 + 5])
+# one, two and four vectors per workgroup, a tile per workgroup, one pass, one and two tiles per wave
+@pytest.mark.parametrize("T", [1, 128, 129, 257, 521, 12 * 1024 + 5, 17 * 1024 + 5, 25 * 1024 + 5])
 @pytest.mark.parametrize("rotation", ["haar", "permutation"])
 @pytest.mark.parametrize("bits,prod", [(1, False), (2, False), (3, False), (4, False), (1, True), (2, True), (3, True)])
 def test_plain_prefill_encoder_on_hard_rows(cuda, bits, prod, rotation, T):

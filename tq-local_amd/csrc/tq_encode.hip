@@ -897,9 +897,10 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
 //
 // The lines: up to 1024 vectors the one-thread-per-output kernels have at most a workgroup of four
 // vectors per CU and are ahead (7.5 / 4.1 against 10.1 / 5.8 at 8, 9.8 / 5.3 against 10.7 / 6.3 at 1024);
-// their callers keep those.  From TILE_MAX_* vectors the kernels above are: with the sketch 33.8 here against
-// 46.5 there at 16384, 49.4 against 48.7 at 24576; without, 17.8 against 21.0 at 16384 and 25.3 against
-// 18.9 at 24576 (channel groups the same within 10%).
+// their callers keep those.  From TILE_MAX_* vectors the kernels above are: with the sketch 33.8 here
+// against 46.5 there at 16384, 49.4 against 48.7 at 24576; without, 17.8 against 21.0 at 16384 and 25.3 against
+// 18.9 at 24576 (channel groups the same within 10%).  Between, a plain call of one tile per wave is ahead
+// of both in one pass (tq_quantize.hip).
 constexpr int64_t TILE_MAX_PROD = 24576, TILE_MAX_MSE = 20480;
 constexpr int MS = D + 4;
 constexpr int BS = 36;  // floats between lanes' 32 elements in the exchange buffers

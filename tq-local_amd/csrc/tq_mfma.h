@@ -110,8 +110,8 @@ __device__ __forceinline__ void image_products(const float4* __restrict__ a, con
 // k-indices zero.  A chain over the image then starts with that many zero products, which
 // leave its +0 start unchanged (+0 plus a zero of either sign is +0), so it is the fma chain
 // over M's rows, bit for bit.
-// Every thread's reads are in flight together, ahead of the first LDS write: read one at a time they
-// took most of a small call (a 4-bit decode of 32768 rows 16.4 -> 12.4 us).
+// Every thread's reads are in flight together, ahead of the first LDS write.  A small call is little
+// helped (a 4-bit decode of 32768 rows 16.5 -> 16.1 us, with the rest of the decoder's change).
 __device__ __forceinline__ void build_image_transposed(float* img, const float* __restrict__ M, int rows = MXD) {
     const int pad = MXD - rows;
     constexpr int N = MXD * MXD / 4 / MQ_THREADS;

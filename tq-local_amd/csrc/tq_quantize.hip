@@ -11,9 +11,9 @@
 //                     r = x - khat;  rho = sqrt_rn(fma chain r_d^2) (0 -> 1);  rhat = r /_rn rho
 //                     sign_i = (fma chain d of rhat_d*S[i][d]) >= 0
 //
-// Two encoders: those of tq_encode.hip for calls of at least MQ_MIN_VECTORS vectors (prefill; the
-// figures at the line stand there) and a small-batch kernel with one thread per output index of each
-// vector (decode-append).
+// Encoders: a small-batch kernel with one thread per output index of each vector (decode-append); from
+// MQ_MIN_VECTORS vectors (prefill) those of tq_encode.hip, where the line's figures stand, and between
+// their two the matrix-core encoder below, where a call is one tile per wave.
 //
 // Reference: runtime/packed_qmse_cache.py:376-402 (_encode_group), :285-310
 // (_encode_keys_qjl_group), :404-435 (_decode_group), :13-43 (_pack_indices),
@@ -30,6 +30,23 @@ namespace {
 using namespace tqmx;
 constexpr int D = TQ_DIM;
 
+// Appends `nbits` bits to a 64-bit staging register; full 32-bit words are
+// written to `dst` (the lane's own output row).
+struct BitWriter {
+    uint64_t acc = 0;
+    int fill = 0;
+    int wi = 0;
+    __device__ __forceinline__ void put(uint32_t v, int nbits, uint32_t* dst) {
+        acc |= (uint64_t)v << fill;
+        fill += nbits;
+        if (fill >= 32) {
+            dst[wi++] = (uint32_t)acc;
+            acc >>= 32;
+            fill -= 32;
+        }
+    }
+};
+
 // #{i : b[i] < z} (torch.bucketize right=False): one compare and one add-with-carry per
 // boundary; the empty asm keeps the count a plain running sum (no bitmask reassociation).
 template <int NB>
@@ -39,6 +56,33 @@ __device__ __forceinline__ uint32_t bucket_count(float z, const float* __restric
     for (int i = 0; i < NB; ++i) {
         c += (b[i] < z) ? 1u : 0u;
         __asm__("" : "+v"(c));
+    }
+    return c;
+}
+
+// The same count by binary search over the sorted boundaries (the predicate b[i] < z holds on
+// a prefix): BITS compares, and at level l a select tree over the 2^l candidate thresholds
+// driven by the earlier outcomes (2^BITS - BITS - 1 selects in all, against 2^BITS - 1
+// compare/add pairs for the linear count).
+template <int BITS>
+__device__ __forceinline__ uint32_t bucket_search(float z, const float* __restrict__ b) {
+    bool p[BITS];
+    uint32_t c = 0;
+#pragma unroll
+    for (int lvl = 0; lvl < BITS; ++lvl) {
+        const int s = 1 << (BITS - 1 - lvl);
+        float cand[1 << (BITS - 1)];
+#pragma unroll
+        for (int m = 0; m < (1 << lvl); ++m) cand[m] = b[s - 1 + 2 * s * m];
+        // candidate m = sum_q p[q] 2^(lvl - 1 - q): reduce by the last outcome first
+#pragma unroll
+        for (int q = lvl - 1; q >= 0; --q) {
+            const int half = 1 << q;  // entries left after this step
+#pragma unroll
+            for (int m = 0; m < half; ++m) cand[m] = p[q] ? cand[2 * m + 1] : cand[2 * m];
+        }
+        p[lvl] = cand[0] < z;
+        c |= p[lvl] ? (uint32_t)s : 0u;
     }
     return c;
 }
@@ -210,6 +254,345 @@ __global__ __launch_bounds__(AT) void append_kernel(
 // At least this many vectors take the prefill encoder (tq_encode.hip).
 constexpr int64_t MQ_MIN_VECTORS = 1025;
 
+// ------------------------------------------------------------------ matrix-core encoder
+// The same encoder with its three D x D matrix-vector products on the fp32 matrix cores:
+// v_mfma_f32_16x16x4_f32 adds the four products of its k = 0..3 to the accumulator one
+// after another, each with one rounding (an fma chain in k order), so a chain of 32 of them
+// over k-steps s = 0..31 covering d = 4s + k is the fma chain d = 0..127 above, bit for bit,
+// denormals and signed zeros included.  The norms come out of the same instruction: with
+// both operands equal to the tile of vectors, the diagonal of the 16 x 16 product is each
+// vector's own fma chain of x_d * x_d.
+//
+// A wave encodes a tile of 16 vectors at a time.  Lane l = 16 g + v (v = l % 16, g = l / 16)
+// holds element 4s + g of vector v for s = 0..31: that is the B operand (k = g, column v) of
+// every product, and a product's accumulator comes back to the lanes of its column v, so a
+// vector never leaves its four lanes.  The matrices are the A operands, read from an LDS
+// image laid out per (16-row tile t, k-step block sb): 64 lanes x 4 consecutive k-steps, one
+// 16-byte read per lane per block, lane slots xor-swizzled (slot = l ^ (l >> 4)) so that
+// the transposed 4-byte reads of the Q_prod residual stage are bank-conflict free as well.
+//
+// Which output index a row m = 4q + i of tile t computes is a free choice (each output is
+// its own chain); it sets which lane ends up holding it:
+//   CONTIG  (Q_mse codes, QJL signs): index 32q + 4t + i -> lane g holds [32g, 32g + 32),
+//           packed and stored by that lane directly;
+//   STRIDED (Q_prod codes): index 4(4t + i) + q -> lane g holds the indices 4s + g, the
+//           B-operand layout of the residual decode that consumes them; one LDS round trip
+//           regroups them for packing.
+//
+// It is bound by the fp32 matrix instructions, 8 x 32 per product and tile, and a call of one tile per
+// wave is a single pass of them.  There, and only there, it beats both neighbours of tq_encode.hip
+// (tiles of a workgroup below, bf16 products in two kernels above); 3-bit keys with the sketch /
+// 4-bit values, us:
+//   vectors   12288        16384        20480        32768        40960
+//   here      39.0 / 17.0  39.7 / 17.3  40.1 / 17.4  41.9 / 18.2  72.9 / 29.3
+//   there     26.8 / 13.9  35.0 / 18.1  42.5 / 18.8  46.8 / 19.4  61.3 / 22.6
+constexpr int64_t PASS_MIN_PROD = 16384, PASS_MIN_MSE = 12288;  // more than this many vectors
+constexpr int LUT_MAX = 512;                // cells of the bucketize grid
+
+// ---- bucketize through a uniform grid
+// code(z) = #{i : b_i < z} for the NB sorted boundaries.  Cells of width w = (smallest gap
+// between neighbouring boundaries) / 4 start at e0 = b_0 - 2w; cell k stores
+// c0 = #{i : b_i < e0 + (k - 1) w} and b_{c0} (+inf when c0 = NB).  z goes to the cell
+// k = clamp(floor((z - e0) / w), 0, cells - 1), and code(z) = c0 + [b_{c0} < z].  Exact, not
+// approximate: the computed (z - e0) / w is within 1e-3 of the real quotient (both |e0| / w and
+// |b_NB-1| / w are kept below 4096), so e0 + (k - 1) w < z < e0 + (k + 2) w, a window of 3w
+// that holds no two boundaries (the gap is 4w).  Every b_i below the window's start is < z,
+// b_{c0 + 1} >= b_{c0} + 4w is above its end, and b_{c0} decides the rest.  The two clamped
+// ends: k = 0 covers z < b_0 - w and NaN (c0 = 0, [b_0 < z] false), and the last cell starts
+// more than w above b_NB-1 (c0 = NB).  A boundary set without that geometry (unsorted,
+// repeated, or too many cells) uses bucket_search instead.
+struct BucketGrid {
+    float scale, offset, top;  // f = z * scale + offset; cells = top + 1
+    float w, e0;
+    int cells;
+    bool ok;
+};
+template <int NB>
+__device__ __forceinline__ BucketGrid bucket_grid(const float* __restrict__ b) {
+    BucketGrid g{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0, false};
+    if constexpr (NB > 1) {
+        float gap = b[1] - b[0];
+        bool sorted = gap > 0.0f;
+#pragma unroll
+        for (int i = 2; i < NB; ++i) {
+            const float d = b[i] - b[i - 1];
+            sorted = sorted && d > 0.0f;
+            gap = fminf(gap, d);
+        }
+        const float w = gap * 0.25f;
+        const float e0 = b[0] - 2.0f * w;
+        const float span = (b[NB - 1] - e0) / w;
+        g.w = w;
+        g.e0 = e0;
+        g.scale = 1.0f / w;
+        g.offset = -e0 * g.scale;
+        g.ok = sorted && w > 0.0f && span < (float)(LUT_MAX - 5) && fabsf(g.offset) < 4096.0f &&
+               fabsf(b[NB - 1] * g.scale) < 4096.0f;
+        g.cells = g.ok ? (int)ceilf(span) + 4 : 0;
+        g.top = (float)(g.cells - 1);
+    }
+    return g;
+}
+template <int NB>
+__device__ __forceinline__ void fill_bucket_grid(float2* lut, const BucketGrid& g, const float* __restrict__ b) {
+    for (int k = threadIdx.x; k < g.cells; k += MQ_THREADS) {
+        const float start = g.e0 + (float)(k - 1) * g.w;
+        uint32_t c0 = 0;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) c0 += b[i] < start ? 1u : 0u;
+        lut[k] = make_float2(c0 < NB ? b[c0] : __builtin_inff(), __uint_as_float(c0));
+    }
+}
+__device__ __forceinline__ uint32_t bucket_lookup(float z, const float2* lut, const BucketGrid& g) {
+    float f = __builtin_fmaf(z, g.scale, g.offset);
+    f = fminf(fmaxf(f, 0.0f), g.top);  // NaN -> 0
+    const float2 e = lut[(uint32_t)f];
+    return __float_as_uint(e.y) + (e.x < z ? 1u : 0u);
+}
+
+// LDS image of the D x D matrix M (row = output index, column = d) for A-operand reads.
+template <bool STRIDED>
+__device__ __forceinline__ void build_image(float* img, const float* __restrict__ M) {
+    for (int idx = threadIdx.x; idx < D * D / 4; idx += MQ_THREADS) {
+        const int row = idx >> 5, s = idx & 31;  // columns 4s .. 4s + 3
+        const float4 val = reinterpret_cast<const float4*>(M)[idx];
+        int t, q, i;
+        if (STRIDED) {
+            t = row >> 4, i = (row >> 2) & 3, q = row & 3;
+        } else {
+            q = row >> 5, t = (row >> 2) & 7, i = row & 3;
+        }
+        const int m = 4 * q + i;
+        float* blk = img + (t * 8 + (s >> 2)) * 256 + (s & 3);
+        const float e[4] = {val.x, val.y, val.z, val.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) blk[4 * ((16 * k + m) ^ k)] = e[k];
+    }
+}
+
+// The 16 diagonal entries of a Gram accumulator (lane 16 g + v, register i holds row 4g + i,
+// column v), returned to every lane of column v.
+__device__ __forceinline__ float gram_diag(const f32x4& acc, int v) {
+    const int r = v & 3;
+    const float mine = r == 0 ? acc[0] : r == 1 ? acc[1] : r == 2 ? acc[2] : acc[3];
+    return __shfl(mine, v + 16 * (v >> 2));
+}
+
+template <int BITS>
+__device__ __forceinline__ void store_row(uint8_t* dst, const uint32_t* w) {
+    if constexpr (BITS == 4) {
+        *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
+    } else if constexpr (BITS == 2) {
+        *reinterpret_cast<uint2*>(dst) = make_uint2(w[0], w[1]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < BITS; ++k) reinterpret_cast<uint32_t*>(dst)[k] = w[k];
+    }
+}
+
+template <int BITS, bool PROD>
+__global__ __launch_bounds__(MQ_THREADS) void quantize_mfma_kernel(
+    const uint16_t* __restrict__ x, int heads, int64_t tokens, int64_t n_vec, int64_t x_sb, int64_t x_sh,
+    int64_t x_st, const float* __restrict__ R, const float* __restrict__ centers,
+    const float* __restrict__ boundaries, const float* __restrict__ S, uint8_t* __restrict__ codes,
+    uint16_t* __restrict__ norms, uint8_t* __restrict__ signs, uint16_t* __restrict__ rnorms, int64_t out_cap,
+    int64_t out_offset, FastDiv tok_div, FastDiv head_div) {
+    __shared__ float4 s_img[(PROD ? 2 : 1) * D * D / 4];                // R image (+ S image)
+    __shared__ uint32_t s_stage[PROD ? MQ_WAVES * 16 * 4 * 8 : 1];      // Q_prod code regrouping
+    __shared__ float s_cent[PROD ? (1 << BITS) : 1];
+    constexpr int NB = (1 << BITS) - 1;
+    __shared__ float2 s_lut[NB > 1 ? LUT_MAX : 1];
+    const BucketGrid grid = bucket_grid<NB>(boundaries);
+    const bool use_grid = __builtin_amdgcn_readfirstlane(grid.ok ? 1 : 0) != 0;
+    if (NB > 1 && use_grid) fill_bucket_grid<NB>(s_lut, grid, boundaries);
+    float* img = reinterpret_cast<float*>(s_img);
+    build_image<PROD>(img, R);
+    if constexpr (PROD) {
+        build_image<false>(img + D * D, S);
+        if (threadIdx.x < (1 << BITS)) s_cent[threadIdx.x] = centers[threadIdx.x];
+    }
+    __syncthreads();  // the only barrier: each wave then works on its own tiles
+
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int v = lane & 15, g = lane >> 4;
+    // v_perm_b32 selector: bf16 element g of a 4-element group -> high half of an fp32
+    const uint32_t sel = ((2u * g + 1u) << 24) | ((2u * g) << 16) | 0x0c0cu;
+    const float4* a_rot = s_img + (lane ^ g);
+    constexpr int ROW = D * BITS / 8;
+    const int64_t n_tiles = (n_vec + 15) / 16;
+
+    for (int64_t tile = (int64_t)blockIdx.x * MQ_WAVES + wave; tile < n_tiles;
+         tile += (int64_t)gridDim.x * MQ_WAVES) {
+        const uint32_t vi = (uint32_t)tile * 16u + (uint32_t)v;  // n_vec < 2^31
+        const bool live = vi < (uint64_t)n_vec;
+        int64_t slot = 0;
+        float xs[32];  // xs[s] = x[v][4s + g]
+        {
+            uint4 w[16];
+            if (live) {
+                const uint32_t gh = fdiv(vi, tok_div), t = vi - gh * (uint32_t)tokens;
+                const uint32_t b = fdiv(gh, head_div), h = gh - b * (uint32_t)heads;
+                slot = (int64_t)gh * out_cap + out_offset + t;
+                const uint4* x4 =
+                    reinterpret_cast<const uint4*>(x + (int64_t)b * x_sb + (int64_t)h * x_sh + (int64_t)t * x_st);
+#pragma unroll
+                for (int c = 0; c < 16; ++c) w[c] = x4[c];
+            } else {
+#pragma unroll
+                for (int c = 0; c < 16; ++c) w[c] = make_uint4(0u, 0u, 0u, 0u);
+            }
+#pragma unroll
+            for (int c = 0; c < 16; ++c) {
+                xs[2 * c] = __uint_as_float(__builtin_amdgcn_perm(w[c].y, w[c].x, sel));
+                xs[2 * c + 1] = __uint_as_float(__builtin_amdgcn_perm(w[c].w, w[c].z, sel));
+            }
+        }
+        // ---- norm: Gram diagonal; u = x / n
+        f32x4 gacc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < 32; ++s) gacc = mfma_f32(xs[s], xs[s], gacc);
+        float n = tq::sqrt_rn(gram_diag(gacc, v));
+        if (!(n > 0.0f)) n = 1.0f;
+        float u[32];
+#pragma unroll
+        for (int s = 0; s < 32; ++s) u[s] = tq::div_rn(xs[s], n);
+        const uint32_t n16 = tq::f32_to_f16(n);
+        if (live && g == 0) norms[slot] = (uint16_t)n16;
+        // Q_prod: the input elements again at the residual, held as bf16 pairs meanwhile
+        uint32_t xp[PROD ? 16 : 1];
+        if constexpr (PROD) {
+#pragma unroll
+            for (int c = 0; c < 16; ++c)
+                xp[c] = __builtin_amdgcn_perm(__float_as_uint(xs[2 * c + 1]), __float_as_uint(xs[2 * c]), 0x07060302u);
+        }
+
+        // ---- rotation and codes
+        f32x4 acc[8];
+        image_products(a_rot, u, acc);
+        uint32_t out[BITS];
+        BitWriter bw;
+        auto code_of = [&](float z, auto grid_path) -> uint32_t {
+            if constexpr (NB == 1) return boundaries[0] < z ? 1u : 0u;
+            else if constexpr (decltype(grid_path)::value) return bucket_lookup(z, s_lut, grid);
+            else return bucket_search<BITS>(z, boundaries);
+        };
+        if constexpr (!PROD) {
+            auto pack = [&](auto grid_path) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) bw.put(code_of(acc[t][i], grid_path), BITS, out);
+            };
+            if (use_grid) pack(std::true_type{});
+            else pack(std::false_type{});
+            if (live) store_row<BITS>(codes + slot * ROW + 4 * BITS * g, out);
+        } else {
+            // codes of indices 4s + g; regroup through LDS into [32g, 32g + 32) for packing
+            uint32_t cw[8];
+            float cv[32];  // C[code] of index 4s + g: the residual decode's B operand
+#pragma unroll
+            for (int k = 0; k < 8; ++k) cw[k] = 0u;
+            auto codes_of = [&](auto grid_path) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int s = 4 * t + i;
+                        const uint32_t c = code_of(acc[t][i], grid_path);
+                        cw[s >> 2] |= c << (8 * (s & 3));
+                        cv[s] = s_cent[c];
+                    }
+            };
+            if (use_grid) codes_of(std::true_type{});
+            else codes_of(std::false_type{});
+            uint32_t* stg = s_stage + wave * (16 * 4 * 8);
+            uint4* st4 = reinterpret_cast<uint4*>(stg + (v * 4 + g) * 8);
+            st4[0] = make_uint4(cw[0], cw[1], cw[2], cw[3]);
+            st4[1] = make_uint4(cw[4], cw[5], cw[6], cw[7]);
+            // the wave's LDS accesses complete in issue order; keep the compiler from moving
+            // the reads above the writes (or the next tile's writes above these reads)
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            uint2 rd[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) rd[q] = reinterpret_cast<const uint2*>(stg + (v * 4 + q) * 8)[g];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int a = 0; a < 8; ++a)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t wd = a < 4 ? rd[q].x : rd[q].y;
+                    bw.put((wd >> (8 * (a & 3))) & 0xFFu, BITS, out);
+                }
+            if (live) store_row<BITS>(codes + slot * ROW + 4 * BITS * g, out);
+
+            // ---- residual decode khat = C[code] @ R: A = R transposed, read from the STRIDED
+            // image 4 bytes at a time; output row 4g + i of tile t is dim 4(4t + i) + g
+            const int qv = v >> 2, iv = v & 3;
+            int off[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) off[c] = 4 * (16 * qv + 4 * g + (c ^ qv)) + iv;
+            f32x4 kacc[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) kacc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            // k-step block sb covers s' = 4 sb + e; its 32 A values are read one block ahead
+            float ka[8][4], kn[8][4];
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) ka[t][e] = img[t * 256 + off[e]];
+#pragma unroll
+            for (int sb = 0; sb < 8; ++sb) {
+                if (sb + 1 < 8) {
+#pragma unroll
+                    for (int t = 0; t < 8; ++t)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) kn[t][e] = img[((sb + 1) * 8 + t) * 256 + off[e]];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) kacc[t] = mfma_f32(ka[t][e], cv[4 * sb + e], kacc[t]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < 8; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) ka[t][e] = kn[t][e];
+            }
+            const float nf = tq::f16_to_f32(n16);
+            float r[32];
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int s = 4 * t + i;
+                    const float x = __uint_as_float((s & 1) ? (xp[s >> 1] & 0xFFFF0000u) : (xp[s >> 1] << 16));
+                    r[s] = x - tq::bf16_to_f32(tq::f32_to_bf16(kacc[t][i] * nf));
+                }
+            f32x4 racc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int s = 0; s < 32; ++s) racc = mfma_f32(r[s], r[s], racc);
+            float rho = tq::sqrt_rn(gram_diag(racc, v));
+            if (!(rho > 0.0f)) rho = 1.0f;
+#pragma unroll
+            for (int s = 0; s < 32; ++s) r[s] = tq::div_rn(r[s], rho);
+            if (live && g == 0) rnorms[slot] = (uint16_t)tq::f32_to_f16(rho);
+
+            // ---- QJL signs of rhat @ S^T (CONTIG image): lane g holds signs [32g, 32g + 32)
+            f32x4 pacc[8];
+            image_products(a_rot + D * D / 4, r, pacc);
+            uint32_t sb = 0u;
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sb |= (pacc[t][i] >= 0.0f ? 1u : 0u) << (4 * t + i);
+            if (live) reinterpret_cast<uint32_t*>(signs + slot * (D / 8))[g] = sb;
+        }
+    }
+}
+
 // ------------------------------------------------------------------- decoders
 // out = bf16((C[code] @ R) * f32(norm)); with QJL (keys of Q_prod) the reference's
 // correction is added in bf16: corr = bf16(((s @ S) * rnorm) * sqrt(pi/2)/D),
@@ -374,6 +757,25 @@ int launch_append(const tqenc::EncodeArgs& a, hipStream_t s) {
     return launch_append_by<BITS, PROD, 4>(a, s);
 }
 
+// Calls of at least MQ_MIN_VECTORS vectors: one pass of the matrix-core encoder where it is ahead.
+template <int BITS, bool PROD>
+int launch_prefill(const tqenc::EncodeArgs& a, hipStream_t s) {
+    const int64_t groups = ((a.n_vec + 15) / 16 + MQ_WAVES - 1) / MQ_WAVES;
+    if (a.n_vec <= (PROD ? PASS_MIN_PROD : PASS_MIN_MSE) || groups > resident_groups<quantize_mfma_kernel<BITS, PROD>>())
+        return tqenc::launch_encode(a, BITS, false, s);
+    hipLaunchKernelGGL((quantize_mfma_kernel<BITS, PROD>), dim3((unsigned)groups), dim3(MQ_THREADS), 0, s, a.x, a.heads,
+                       a.tokens, a.n_vec, a.x_sb, a.x_sh, a.x_st, a.R, a.centers, a.boundaries, a.S, a.codes, a.norms,
+                       a.signs, a.rnorms, a.out_cap, a.out_offset, make_fastdiv((uint32_t)a.tokens),
+                       make_fastdiv((uint32_t)a.heads));
+    TQ_CHECK_LAUNCH();
+    return TQ_OK;
+}
+
+template <int BITS, bool PROD>
+int launch_quantize(const tqenc::EncodeArgs& a, hipStream_t s) {
+    return prefill_size(a.n_vec) ? launch_prefill<BITS, PROD>(a, s) : launch_append<BITS, PROD>(a, s);
+}
+
 }  // namespace
 
 extern "C" int tq_quantize_mse(const uint16_t* x, int batch, int heads, int64_t tokens, int dim, int64_t x_sb,
@@ -387,12 +789,11 @@ extern "C" int tq_quantize_mse(const uint16_t* x, int batch, int heads, int64_t 
     const tqenc::EncodeArgs a = plain_args(x, batch, heads, tokens, x_sb, x_sh, x_st, rotation, nullptr, boundaries,
                                            nullptr, codes, norms, nullptr, nullptr, out_cap, out_offset);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (bits >= 1 && bits <= 4 && prefill_size(a.n_vec)) return tqenc::launch_encode(a, bits, false, s);
     switch (bits) {
-        case 1: return launch_append<1, false>(a, s);
-        case 2: return launch_append<2, false>(a, s);
-        case 3: return launch_append<3, false>(a, s);
-        case 4: return launch_append<4, false>(a, s);
+        case 1: return launch_quantize<1, false>(a, s);
+        case 2: return launch_quantize<2, false>(a, s);
+        case 3: return launch_quantize<3, false>(a, s);
+        case 4: return launch_quantize<4, false>(a, s);
         default: return TQ_ERR_INVALID_ARGUMENT;
     }
 }
@@ -410,11 +811,10 @@ extern "C" int tq_quantize_prod(const uint16_t* x, int batch, int heads, int64_t
     const tqenc::EncodeArgs a = plain_args(x, batch, heads, tokens, x_sb, x_sh, x_st, rotation, centers, boundaries, qjl,
                                            codes, norms, signs, rnorms, out_cap, out_offset);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (mse_bits >= 1 && mse_bits <= 3 && prefill_size(a.n_vec)) return tqenc::launch_encode(a, mse_bits, false, s);
     switch (mse_bits) {
-        case 1: return launch_append<1, true>(a, s);
-        case 2: return launch_append<2, true>(a, s);
-        case 3: return launch_append<3, true>(a, s);
+        case 1: return launch_quantize<1, true>(a, s);
+        case 2: return launch_quantize<2, true>(a, s);
+        case 3: return launch_quantize<3, true>(a, s);
         default: return TQ_ERR_INVALID_ARGUMENT;
     }
 }
