@@ -146,9 +146,13 @@ class _Store:
             setattr(self, name, None)
         self._alloc(cap)
 
+    #: up to here the buffers are parts of one allocation, cleared by one launch: six took 12 us of a short
+    #: prompt's 67.  Above, clearing is bound by bandwidth, and buffers of their own let a growing store give
+    #: back each old one as soon as it is copied.
+    ONE_BLOCK_BYTES = 16 << 20
+
     def _alloc(self, cap: int) -> None:
-        """New buffers of ``cap`` slots, zero past the tokens carried over: parts of one allocation, so that
-        one launch clears them all (six took 12 us of a short prompt's 67)."""
+        """New buffers of ``cap`` slots, zero past the tokens carried over."""
         n = self.length
         parts, total = [], 0
         for name, entry in self.spec.items():
@@ -158,9 +162,12 @@ class _Store:
             nbytes = self.B * self.H * cap * prod(row) * dtype.itemsize
             parts.append((name, row, dtype, total, nbytes))
             total += -(-nbytes // 256) * 256
-        flat = torch.zeros(total, dtype=torch.uint8, device=self.device)
+        flat = torch.zeros(total, dtype=torch.uint8, device=self.device) if total <= self.ONE_BLOCK_BYTES else None
         for name, row, dtype, start, nbytes in parts:
-            buf = flat[start:start + nbytes].view(dtype).view(self.B, self.H, cap, *row)
+            if flat is not None:
+                buf = flat[start:start + nbytes].view(dtype).view(self.B, self.H, cap, *row)
+            else:
+                buf = torch.zeros(self.B, self.H, cap, *row, dtype=dtype, device=self.device)
             old = getattr(self, name)
             if old is not None and n:
                 buf[:, :, :n].copy_(old[:, :, :n])
