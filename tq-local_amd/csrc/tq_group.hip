@@ -285,9 +285,10 @@ __global__ __launch_bounds__(GBLOCK) void dequantize_group_kernel(
 // ------------------------------------------------------------------ channel energies
 // sum over all vectors of x_c^2, keys and values together: what the outlier channels are chosen by.
 // Reads each tensor once (as torch operations it took three passes and fp32 copies: 220 us for
-// 2 x 8 x 16384 keys and values of a split prefill, 21 us here).  A thread holds 8 channels and walks
-// rows 16 apart; a workgroup's 16 row lanes meet in LDS, the workgroups in energy_sum_kernel, in a
-// fixed order.
+// 2 x 8 x 16384 keys and values of a split prefill, 31 us a call here).  A thread holds 8 channels and
+// walks rows 16 apart, 32 of them to a partial sum, so that the error does not grow with a prompt's
+// length (on 2M rows at most 2.3e-7; 1e-6 as torch operations); a workgroup's 16 row lanes meet in
+// LDS, the workgroups in energy_sum_kernel, in a fixed order.
 constexpr int EB = TQ_ENERGY_BLOCKS;
 
 __global__ __launch_bounds__(GBLOCK) void channel_energy_kernel(const uint16_t* __restrict__ k,
@@ -307,19 +308,27 @@ __global__ __launch_bounds__(GBLOCK) void channel_energy_kernel(const uint16_t* 
     const int64_t per = (n_vec + gridDim.x - 1) / gridDim.x;
     const int64_t end = std::min<int64_t>(((int64_t)blockIdx.x + 1) * per, n_vec);
     for (int64_t i = (int64_t)blockIdx.x * per; i < end;) {
-        const int64_t gh = i / tokens, t0 = i - gh * tokens, b = gh / heads, h = gh - b * heads;
-        const int64_t run = std::min<int64_t>(tokens - t0, end - i);  // rows of this head
-        const uint16_t* base = x + b * sb + h * sh + t0 * st + 8 * c;
-#pragma unroll 4
-        for (int64_t t = r; t < run; t += GBLOCK / 16) {
-            const uint4 w = *reinterpret_cast<const uint4*>(base + t * st);
-            const uint32_t p[4] = {w.x, w.y, w.z, w.w};
+        const int64_t gh = i / tokens, first = i - gh * tokens, b = gh / heads, h = gh - b * heads;
+        const int64_t run = std::min<int64_t>(tokens - first, end - i);  // rows of this head
+        const uint16_t* base = x + b * sb + h * sh + first * st + 8 * c;
+        for (int64_t t0 = r; t0 < run; t0 += 32 * (GBLOCK / 16)) {
+            const int64_t t1 = std::min<int64_t>(t0 + 32 * (GBLOCK / 16), run);
+            float part[8];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float lo = tq::bf16_to_f32(p[e] & 0xFFFFu), hi = __uint_as_float(p[e] & 0xFFFF0000u);
-                acc[2 * e] = __builtin_fmaf(lo, lo, acc[2 * e]);
-                acc[2 * e + 1] = __builtin_fmaf(hi, hi, acc[2 * e + 1]);
+            for (int e = 0; e < 8; ++e) part[e] = 0.0f;
+#pragma unroll 4
+            for (int64_t t = t0; t < t1; t += GBLOCK / 16) {
+                const uint4 w = *reinterpret_cast<const uint4*>(base + t * st);
+                const uint32_t p[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float lo = tq::bf16_to_f32(p[e] & 0xFFFFu), hi = __uint_as_float(p[e] & 0xFFFF0000u);
+                    part[2 * e] = __builtin_fmaf(lo, lo, part[2 * e]);
+                    part[2 * e + 1] = __builtin_fmaf(hi, hi, part[2 * e + 1]);
+                }
             }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[e] += part[e];
         }
         i += run;
     }
