@@ -74,6 +74,19 @@ def test_dense_attention_matches_fp64(cuda, dtype, B, Hkv, g, Sq, n, mask, split
     check(got, ref, dtype)
 
 
+@pytest.mark.parametrize("Sq,n", [(1, 1), (1, 40), (40, 70)])
+def test_an_infinite_value_stays_infinite(cuda, Sq, n):
+    """A weight of few bits (1 for a single token, 1 / n for equal keys) has zero lower terms."""
+    q, k = randn((1, 4, Sq, D), 1, torch.bfloat16), torch.zeros((1, 1, n, D), dtype=torch.bfloat16, device="cuda")
+    v = randn((1, 1, n, D), 2, torch.bfloat16)
+    v[0, 0, n // 2, 5] = float("inf")
+    v[0, 0, n - 1, 7] = float("-inf")
+    out = K.DenseAttention(q, 1, 1).add(k, v, n, 0, 1, SCALE, out=torch.float32)
+    assert (out[..., 5] == float("inf")).all() and (out[..., 7] == float("-inf")).all()
+    rest = [d for d in range(D) if d not in (5, 7)]
+    check(out[..., rest], oracle(q, k, v[..., rest], None), torch.float32)
+
+
 @pytest.mark.parametrize("Sq", [1, 20])
 def test_position_bounds_continued_partials_and_another_part(cuda, Sq):
     B, Hkv, g, n = 3, 2, 4, 300

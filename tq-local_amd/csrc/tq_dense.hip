@@ -59,6 +59,16 @@ __device__ __forceinline__ uint32_t high_halves(float a, float b) {
 }
 __device__ __forceinline__ float drop_high(float a) { return a - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u); }
 
+// A pair of weight terms, zeros raised to the smallest normal bf16: a weight of few bits has zero
+// lower terms, and 0 x inf would make NaN of the infinity that a value's own product gives.  Next to
+// the weights, whose largest is 1 in every split, 2^-126 is nothing.  16 instructions per tile; where
+// nothing is attended they leave sums that the merge weighs with 2^-inf = 0.
+__device__ __forceinline__ uint32_t not_zero(uint32_t p) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    const u16x2 tiny = {0x0080, 0x0080};
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, p), tiny));
+}
+
 // 2^x (v_exp_f32, 1 ulp; 2^-inf = 0).
 __device__ __forceinline__ float exp2_(float x) { return __builtin_amdgcn_exp2f(x); }
 constexpr float LOG2E = 1.44269504f;
@@ -328,8 +338,8 @@ __global__ __launch_bounds__(64 * W, QT == 1 && W > 1 ? 2 : 1) void dense_attn_k
                 float p0 = s[8 * kb16 + 2 * k], p1 = s[8 * kb16 + 2 * k + 1];
                 p[0].u[k] = high_halves(p0, p1);
                 p0 = drop_high(p0), p1 = drop_high(p1);
-                p[1].u[k] = high_halves(p0, p1);
-                p[2].u[k] = high_halves(drop_high(p0), drop_high(p1));
+                p[1].u[k] = not_zero(high_halves(p0, p1));
+                p[2].u[k] = not_zero(high_halves(drop_high(p0), drop_high(p1)));
             }
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
