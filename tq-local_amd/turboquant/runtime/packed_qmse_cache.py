@@ -147,8 +147,9 @@ class _Store:
         self._alloc(cap)
 
     #: up to here the buffers are parts of one allocation, cleared by one launch: six took 12 us of a short
-    #: prompt's 67, twelve 32 us of the 546 of a split layer of 36 MB.  Above, clearing is bound by bandwidth, and buffers of their own let a growing store give
-    #: back each old one as soon as it is copied.
+    #: prompt's 67, twelve 32 us of the 546 of a split layer of 36 MB.  Above, clearing is bound by
+    #: bandwidth, and buffers of their own let a growing store give back each old one as soon as it is
+    #: copied.
     ONE_BLOCK_BYTES = 64 << 20
 
     def _alloc(self, cap: int) -> None:
