@@ -642,9 +642,13 @@ __global__ __launch_bounds__(MQ_THREADS) void dequantize_kernel(
     // the first item's rows are on their way while the images are built
     int64_t item = (int64_t)blockIdx.x * MQ_WAVES + wave;
     fetch(item);
-    float* img = reinterpret_cast<float*>(s_img);
-    build_image_transposed(img, R);
-    if constexpr (QJL) build_image_transposed(img + D * D, S);
+    {
+        TransposedImage r, q;
+        r.load(R);
+        if constexpr (QJL) q.load(S);
+        r.store(s_img);
+        if constexpr (QJL) q.store(s_img + D * D / 4);
+    }
     if (threadIdx.x < (1 << BITS)) s_cent[threadIdx.x] = centers[threadIdx.x];
     __syncthreads();  // the only barrier: each wave then works on its own tiles
 
@@ -666,7 +670,8 @@ __global__ __launch_bounds__(MQ_THREADS) void dequantize_kernel(
         centers_of<BITS>(w, g, s_cent, cv);
         // the next item's rows beside this one's products (Q_mse kernels, four waves on a SIMD, would
         // lose one to the registers)
-        if (QJL) fetch(item + (int64_t)gridDim.x * MQ_WAVES);
+        const int64_t next = item + (int64_t)gridDim.x * MQ_WAVES;
+        if (QJL && next < n_items) fetch(next);
         f32x4 acc[NT];
         image_products<NT>(a_img, cv, acc);
         uint32_t kh[2 * NT];  // bf16 pairs of dims 32g + 4 t0 + 2p, + 2p + 1
@@ -695,7 +700,7 @@ __global__ __launch_bounds__(MQ_THREADS) void dequantize_kernel(
 #pragma unroll
             for (int i = 0; i < NT / 2; ++i) o4[i] = make_uint4(kh[4 * i], kh[4 * i + 1], kh[4 * i + 2], kh[4 * i + 3]);
         }
-        if (!QJL) fetch(item + (int64_t)gridDim.x * MQ_WAVES);
+        if (!QJL && next < n_items) fetch(next);
     }
 }
 
