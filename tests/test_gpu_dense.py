@@ -87,6 +87,43 @@ def test_an_infinite_value_stays_infinite(cuda, Sq, n):
     check(out[..., rest], oracle(q, k, v[..., rest], None), torch.float32)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("Sq", [1, 12, 40])  # one, two and four waves per workgroup
+@pytest.mark.parametrize("form", ["mask", "bounds", "far below", "faint"])
+def test_values_of_unattended_tokens_add_nothing(cuda, dtype, Sq, form):
+    """A weight of 0 (masked, out of bounds, 2^-x that underflows) leaves out a value of the type's
+    largest magnitude; a faint one (2^-120) adds its product, beside an infinity elsewhere in the tile."""
+    n, tok = 70, 37
+    q, k = randn((1, 4, Sq, D), 1, dtype), torch.zeros((1, 1, n, D), dtype=torch.bfloat16, device="cuda")
+    v = randn((1, 1, n, D), 2, torch.bfloat16)
+    v[0, 0, tok, 6], v[0, 0, tok, 9] = torch.finfo(torch.bfloat16).max, -torch.finfo(torch.bfloat16).max
+    v[0, 0, tok + 1, 5] = float("inf")
+    add, kw = torch.zeros(1, 1, 1, n, device="cuda"), {}
+    if form == "mask":
+        add[..., tok] = float("-inf")
+        kw["mask"] = add == 0
+    elif form == "bounds":
+        add[..., :tok + 1] = float("-inf")
+        kw["starts"] = torch.tensor([tok + 1], dtype=torch.int32, device="cuda")
+        kw["ends"] = torch.tensor([n], dtype=torch.int32, device="cuda")
+    else:
+        q[..., 0] = 16.0
+        k[0, 0, tok, 0] = -200.0 if form == "far below" else -58.75  # logits of -283 and -83.1
+    out = K.DenseAttention(q, 1, 1).add(k, v, n, 0, 1, SCALE, out=torch.float32, **kw)
+    assert (out[..., 5] == float("inf")).all()
+    rest = [d for d in range(D) if d != 5]
+    ref = oracle(q, k, v[..., rest], add)
+    # a logit of 83 is rounded at 2^-24 of it, twice: 1e-5 of a faint weight, 2e-5 with exp2's own error;
+    # and a weight's third term ends at 2^-133, the last bit of bf16
+    err = (out[..., rest].double() - ref).abs().amax((0, 1, 2))
+    scale = ref.abs().amax((0, 1, 2))
+    if form == "faint":
+        last = 2.0 ** -133 * v[..., rest].abs().double().amax((0, 1, 2)) / (n - 1)
+        assert (err <= 4e-5 * scale.clamp(min=1.0) + last).all()
+    else:
+        assert (err <= TOL32 * scale.clamp(min=1.0)).all()
+
+
 @pytest.mark.parametrize("Sq", [1, 20])
 def test_position_bounds_continued_partials_and_another_part(cuda, Sq):
     B, Hkv, g, n = 3, 2, 4, 300
