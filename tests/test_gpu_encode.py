@@ -111,6 +111,50 @@ def test_group_prefill_encoder_on_hard_rows(cuda, d, bits, extra, qjl, T):
             assert int(t[:, :, :2].count_nonzero()) == 0 and int(t[:, :, T + 2:].count_nonzero()) == 0
 
 
+@pytest.mark.parametrize("T", [17 * 1024 + 5, 25 * 1024 + 5])  # one and two tiles per wave
+@pytest.mark.parametrize("group", [False, True])
+@pytest.mark.parametrize("scale", [1e-30, 1e-37, float("inf")])
+def test_prefill_encoder_with_matrices_outside_the_bounds_range(cuda, scale, group, T):
+    """Matrices whose rows' squares vanish (1e-30), whose second bf16 terms are lost (1e-37), or that
+    hold an infinity, which makes NaN of a zero vector's products too: the chains decide all of it."""
+    x = hard_rows(T, 5)
+    sc = split_codecs(np.setdiff1d(np.arange(D), [3, 40, 41, 90]), np.array([3, 40, 41, 90]), 4, 1, 0, True, cuda)
+    lc = layer_codecs(D, 4, 0, True, cuda)
+    val, key, S = (sc.value_normal, sc.key_normal, sc.key_normal.qjl) if group else (lc.value, lc.key, lc.qjl)
+
+    def bad(m):
+        m = m.clone() if scale == float("inf") else m * scale
+        if scale == float("inf"):
+            m[5, 7] = scale
+        return m
+
+    def space(m, c):
+        return None if m is None else torch.from_numpy(K.group_matrix(m.cpu().numpy(), c.channels)).to(cuda)
+
+    rows = u16(x).reshape(-1, D)
+    rows = rows[:, val.channels] if group else rows
+    by = 1.0 if scale == float("inf") else scale
+    for c, R, Bd, Sq in ((val, bad(val.rotation), val.boundaries * by, None), (key, key.rotation, key.boundaries, bad(S))):
+        kc, kn, ks, kr = buffers(x, K.row_bytes(rows.shape[1], c.bits), K.row_bytes(rows.shape[1], 1))
+        if group:
+            codec = K.GroupCodec(c.channels, c.bits, R, c.centers, Bd, space(R, c), Sq, space(Sq, c))
+            K.quantize_group(x, codec, kc, kn, *((ks, kr) if Sq is not None else ()), offset=2)
+        else:
+            codec = K.CodecParams(bits=c.bits, rotation=R, centers=c.centers, boundaries=Bd)
+            if Sq is None:
+                K.quantize_mse(x, codec, kc, kn, offset=2)
+            else:
+                K.quantize_prod(x, codec, Sq, kc, kn, ks, kr, offset=2)
+        h = [t.cpu().numpy() for t in (R, c.centers, Bd)]
+        if Sq is None:
+            compare(x, (kc, kn), O.encode_mse(rows, c.bits, h[0], h[2]), T)
+        else:
+            ref = O.encode_prod(rows, c.bits, h[0], h[1], h[2], Sq.cpu().numpy())
+            if group:
+                ref[3][ref[1] == 0x7C00] = 0x3C00  # as above
+            compare(x, (kc, kn, ks, kr), ref, T)
+
+
 @pytest.mark.parametrize("B,H,T", [(1, 1, 1), (2, 3, 17), (1, 8, 1000), (3, 2, 40001)])
 def test_channel_energy_matches_fp64(cuda, B, H, T):
     """Strided keys and values, workgroups whose runs cross heads; fp32 sums of at most

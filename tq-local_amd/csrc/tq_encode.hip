@@ -24,7 +24,9 @@
 //     boundary's magnitude B where it matters: 6.3e-6 B;
 //   the table's boundaries, whose low bits hold a code: 2^bits * 2^-23 B.
 // r is measured when the matrix is staged; a matrix or vector outside the range where these
-// hold (not finite, squares that under- or overflow) takes the chain for every output.  The fp16
+// hold (not finite, squares that under- or overflow, r below 1e-15: with n >= 1e-12 a second term or a
+// product that is lost below 2^-126 is still 1e-3 of the slack left in 1.33e-5 r) takes the chain for
+// every output, a zero vector too (0 x inf).  The fp16
 // norm is handled alike: where the bound straddles a rounding boundary of fp16, the chain decides.
 //
 // Outputs that need their chain wait in a per-wave queue in LDS, their row of codes with them, and
@@ -191,7 +193,7 @@ __global__ __launch_bounds__(CT) void codes_kernel(EncodeArgs a) {
     const float g_scale = 1.0f / w;
     const float g_off = -e0 * g_scale;
     // outside the bounds' range every output takes its chain
-    const bool exact_all = !(r_norm < 1e18f) || !(b_max < 1e18f);
+    const bool exact_all = !(r_norm < 1e18f) || !(r_norm > 1e-15f) || !(b_max < 1e18f);
     const bool use_grid = sorted && w > 16.0f * eps && span < (float)(LUT_MAX - 5) && fabsf(g_off) < 4096.0f &&
                           fabsf(sh.bound[NB - 1] * g_scale) < 4096.0f;
     const int cells = use_grid ? (int)ceilf(span) + 4 : 0;
@@ -388,12 +390,12 @@ __global__ __launch_bounds__(CT) void codes_kernel(EncodeArgs a) {
             any &= 0x7FFF7FFFu;
             any |= (uint32_t)__shfl_xor((int)any, 16);
             any |= (uint32_t)__shfl_xor((int)any, 32);
-            const bool zero = any == 0u;  // norm 1, every chain 0
+            const bool zero = any == 0u;  // norm 1, every chain 0 (where the matrix is finite)
             const float n_ = zero ? 1.0f : __builtin_sqrtf(ss);
             rn[n] = __builtin_amdgcn_rcpf(n_);
             rg[n] = rn[n] * q_scale;
             mg[n] = zero ? -1.0f : eps;
-            const bool bad = !zero && (!(ss > 1e-24f) || !(ss < 1e30f) || exact_all);
+            const bool bad = exact_all || (!zero && (!(ss > 1e-24f) || !(ss < 1e30f)));
             const uint32_t h0 = tq::f32_to_f16(n_ * (1.0f - 7e-6f)), h1 = tq::f32_to_f16(n_ * (1.0f + 7e-6f));
             if (bad || (h0 != h1 && !zero)) n_amb |= 1u << n;
             if (bad) special |= 1u << n;
@@ -623,7 +625,7 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
     __syncthreads();  // the last barrier: each wave then works on its own tiles
     const float s_norm = __builtin_sqrtf(__uint_as_float(s_max)) * 1.0001f;
     const float eps = s_norm * 2.25e-5f;
-    const bool exact_all = !(s_norm < 1e15f);
+    const bool exact_all = !(s_norm < 1e15f) || !(s_norm > 1e-15f);
     const float4* a_img = s_img + (lane ^ g);
     const uint32_t mw = g == 0 ? a.mask[0] : g == 1 ? a.mask[1] : g == 2 ? a.mask[2] : a.mask[3];
     const int row_bytes = GROUP ? (sub_dim * BITS + 7) >> 3 : D * BITS / 8;
@@ -730,7 +732,7 @@ __global__ __launch_bounds__(MQ_THREADS) void residual_kernel(EncodeArgs a) {
         }
         rs += __shfl_xor(rs, 16);
         rs += __shfl_xor(rs, 32);
-        const bool bad = rs != 0.0f && (!(rs > 1e-24f) || !(rs < 1e30f) || exact_all);
+        const bool bad = exact_all || (rs != 0.0f && (!(rs > 1e-24f) || !(rs < 1e30f)));
         // a sum of squares of 0 can hide residuals whose squares vanish; the chain's does as well
         const float rho = rs == 0.0f ? 1.0f : __builtin_sqrtf(rs);
         const uint32_t h0 = tq::f32_to_f16(rho * (1.0f - 7e-6f)), h1 = tq::f32_to_f16(rho * (1.0f + 7e-6f));
