@@ -12,7 +12,7 @@ from oracle import oracle as O
 from turboquant.quantization.turboquant_mse import codebook_f32
 from turboquant.runtime import kernels as K
 from turboquant.runtime.attention import _group_buffers, fused_attention
-from turboquant.runtime.packed_qmse_cache import PackedMSELayer
+from turboquant.runtime.packed_qmse_cache import PackedMSELayer, detect_outlier_channels
 from turboquant.runtime.params import split_codecs
 from turboquant.runtime.synthetic import kv_bf16, query_bf16
 
@@ -120,6 +120,21 @@ def test_group_small_batch_and_lane_encoders_agree(cuda, prod):
     torch.cuda.synchronize()
     for a, b in zip(whole, parts):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n_out", [3, 4, 17])
+def test_channels_of_equal_energy_are_the_public_function_s(cuda, n_out):
+    """Energies tied between 64 channels (exactly: sums of ones): a layer splits at the channels that
+    detect_outlier_channels names, which are those of the device's topk over the torch reductions."""
+    k = torch.ones(1, 2, 40, D, dtype=torch.bfloat16, device=cuda)
+    k[..., ::2] = -2.0
+    v = torch.ones_like(k)
+    layer = PackedMSELayer(bits=4, num_outlier_channels=n_out)
+    layer.initialize_from_dense(k, v)
+    outlier, normal = detect_outlier_channels(k, v, n_out)
+    energy = k.float().pow(2).sum(dim=(0, 1, 2)) + v.float().pow(2).sum(dim=(0, 1, 2))
+    assert torch.equal(outlier, torch.topk(energy, n_out).indices.sort().values)
+    assert torch.equal(layer._split.outlier_indices, outlier) and torch.equal(layer._split.normal_indices, normal)
 
 
 def test_quantize_group_strided_input_and_decode_append(cuda):

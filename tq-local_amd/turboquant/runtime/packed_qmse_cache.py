@@ -28,6 +28,7 @@ from dataclasses import dataclass
 from math import prod, sqrt
 from typing import Any
 
+import numpy as np
 import torch
 from transformers.cache_utils import Cache, CacheLayerMixin
 
@@ -115,19 +116,15 @@ def _channel_energy(key_states: torch.Tensor, value_states: torch.Tensor) -> tor
     return key_states.float().pow(2).sum(dim=(0, 1, 2)) + value_states.float().pow(2).sum(dim=(0, 1, 2))
 
 
-def _split_channels(combined: torch.Tensor, num_outlier_channels: int) -> tuple[torch.Tensor, torch.Tensor]:
-    """(outlier, normal) channel indices, both ascending, of the channel energies."""
-    outlier = torch.topk(combined, num_outlier_channels).indices.sort().values
-    keep = torch.ones(combined.shape[0], dtype=torch.bool, device=combined.device)
-    keep[outlier] = False
-    return outlier, torch.arange(combined.shape[0], device=combined.device)[keep]
-
-
 def detect_outlier_channels(key_states: torch.Tensor, value_states: torch.Tensor,
                             num_outlier_channels: int) -> tuple[torch.Tensor, torch.Tensor]:
     """(outlier, normal) channel indices, both ascending: the channels of largest
     combined key + value energy (reference runtime/packed_qmse_cache.py:95-114)."""
-    return _split_channels(_channel_energy(key_states, value_states), num_outlier_channels)
+    combined = _channel_energy(key_states, value_states)
+    outlier = torch.topk(combined, num_outlier_channels).indices.sort().values
+    keep = torch.ones(combined.shape[0], dtype=torch.bool, device=combined.device)
+    keep[outlier] = False
+    return outlier, torch.arange(combined.shape[0], device=combined.device)[keep]
 
 
 class _Store:
@@ -239,11 +236,12 @@ class PackedMSELayer(CacheLayerMixin):
         self.device = key_states.device
         D = int(key_states.shape[-1])
         if 0 < self.num_outlier_channels < D:
-            # the channels are needed on the host: the 128 energies go there, once, and are sorted there
-            outlier, normal = _split_channels(_channel_energy(key_states, value_states).cpu(),
-                                              self.num_outlier_channels)
-            self._split = split_codecs(normal.numpy(), outlier.numpy(), self.bits, self.outlier_extra_bits, self.seed,
-                                       self.use_qjl_keys, self.device, self.grid_size)
+            # the choice of detect_outlier_channels, among equal energies too (the device's topk); the
+            # channels are needed on the host, where they go once and are sorted
+            top = torch.topk(_channel_energy(key_states, value_states), self.num_outlier_channels).indices
+            outlier = np.sort(top.cpu().numpy())
+            self._split = split_codecs(np.setdiff1d(np.arange(D), outlier), outlier, self.bits, self.outlier_extra_bits,
+                                       self.seed, self.use_qjl_keys, self.device, self.grid_size)
         else:
             self.codecs = layer_codecs(D, self.bits, self.seed, self.use_qjl_keys, self.device, self.grid_size)
         self.is_initialized = True
