@@ -6,6 +6,7 @@ attention matches fp64 attention over the same decoded rows."""
 import numpy as np
 import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
 
 import turboquant
 from oracle import oracle as O
@@ -135,6 +136,36 @@ def test_channels_of_equal_energy_are_the_public_function_s(cuda, n_out):
     energy = k.float().pow(2).sum(dim=(0, 1, 2)) + v.float().pow(2).sum(dim=(0, 1, 2))
     assert torch.equal(outlier, torch.topk(energy, n_out).indices.sort().values)
     assert torch.equal(layer._split.outlier_indices, outlier) and torch.equal(layer._split.normal_indices, normal)
+
+
+def _energy_prompt(seed, ch):
+    k, v = kv_bf16((1, 2, 40, D), seed=seed), kv_bf16((1, 2, 40, D), seed=seed + 1)
+    k[..., ch] *= 8.0
+    return k, v
+
+
+@pytest.mark.parametrize("form", ["traced", "jit", "grad", "forward", "unaligned", "parameter"])
+def test_detect_outlier_channels_where_torch_operations_are_watched(cuda, form):
+    """A trace holds the operations and not the channels it was made with, transforms see their own
+    tensors, and rows at any address are taken."""
+    (k, v), (k2, v2) = _energy_prompt(1, [3, 9, 80]), _energy_prompt(5, [0, 64, 127])
+    want, want2 = (torch.tensor(c, device=cuda) for c in ([3, 9, 80], [0, 64, 127]))
+    detect = lambda a, b: detect_outlier_channels(a, b, 3)[0]  # noqa: E731
+    if form == "traced":
+        assert torch.equal(make_fx(detect)(k, v)(k2, v2), want2)
+    elif form == "jit":
+        assert torch.equal(torch.jit.trace(detect, (k, v))(k2, v2), want2)
+    elif form == "grad":
+        g = torch.func.grad(lambda a: a[..., detect(a, v)].sum())(k)
+        assert g[..., want].eq(1).all() and g.sum() == 3 * 80
+    elif form == "forward":
+        _, t = torch.func.jvp(lambda a: a[..., detect(a, v)].sum(), (k,), (torch.ones_like(k),))
+        assert t == 3 * 80
+    elif form == "unaligned":
+        flat = torch.empty(k.numel() + 3, dtype=k.dtype, device=cuda)[3:].view(k.shape).copy_(k)
+        assert flat.is_contiguous() and flat.data_ptr() % 16 and torch.equal(detect(flat, v), want)
+    else:
+        assert torch.equal(detect(torch.nn.Parameter(k), v), want)
 
 
 def test_quantize_group_strided_input_and_decode_append(cuda):

@@ -30,7 +30,6 @@ from typing import TYPE_CHECKING
 
 import torch
 import torch.nn.functional as F
-from torch.autograd import forward_ad
 
 from turboquant.runtime import _lib
 from turboquant.runtime import kernels as K
@@ -215,12 +214,11 @@ def _repeat_kv(t: torch.Tensor, n_rep: int) -> torch.Tensor:
 
 def _native_rows(query: torch.Tensor, *rows: torch.Tensor) -> bool:
     """Whether libtq's attention over bf16 rows takes this query and these keys and values.
-    Autograd, transforms, tracing and dispatch modes need torch operations; rows of another
-    dtype would be rounded."""
+    Autograd needs torch operations, as do the callers of ``K.torch_operations_watched``; rows of
+    another dtype would be rounded."""
     dev, grad = query.device, torch.is_grad_enabled()
     if (dev.type != "cuda" or query.shape[-1] != K.HEAD_DIM or query.dtype == torch.float64 or query.numel() == 0
-            or (grad and query.requires_grad) or torch._C._len_torch_dispatch_stack() or torch._C._is_tracing()
-            or torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0):
+            or (grad and query.requires_grad) or K.torch_operations_watched()):
         return False
     for t in rows:
         if (t.dtype != torch.bfloat16 or t.device != dev or t.dim() != 4 or t.shape[0] != query.shape[0]

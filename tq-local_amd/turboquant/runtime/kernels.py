@@ -26,6 +26,7 @@ from dataclasses import dataclass
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from turboquant.runtime import _lib
 
@@ -63,6 +64,13 @@ def _require_gpu(*tensors: torch.Tensor | None) -> None:
             raise RuntimeError(
                 f"TurboQuant kernels run on the GPU only (libtq, gfx950); got a tensor on {t.device}"
             )
+
+
+def torch_operations_watched() -> bool:
+    """Whether a transform, a trace or a dispatch mode follows the torch operations of the calling
+    thread: a libtq kernel in their place would be missed."""
+    return bool(torch._C._len_torch_dispatch_stack() or torch._C._is_tracing()
+                or torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0)
 
 
 def row_bytes(dim: int, bits: int) -> int:
@@ -196,7 +204,7 @@ _ENERGY_BLOCKS = 256  # TQ_ENERGY_BLOCKS
 
 def channel_energy(k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
     """Per channel the sum of squares over all keys and values, fp32 [D]; k, v bf16 [B,H,T,D] on the GPU."""
-    k, v = _as_encoder_input(k), _as_encoder_input(v)
+    k, v = rows16(_as_encoder_input(k)), rows16(_as_encoder_input(v))
     _require_gpu(k, v)
     B, H, T, D = k.shape
     buf = torch.empty(2 * _ENERGY_BLOCKS * D + D, dtype=torch.float32, device=k.device)

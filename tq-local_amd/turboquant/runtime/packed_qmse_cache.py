@@ -109,9 +109,12 @@ def _packed_rows(t: torch.Tensor) -> torch.Tensor:
 
 def _channel_energy(key_states: torch.Tensor, value_states: torch.Tensor) -> torch.Tensor:
     """Key plus value energy of each channel, fp32 [D].  bf16 prompts on the GPU take libtq's one-pass
-    kernel; other dtypes, devices and shapes torch's reductions."""
-    if all(t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 4 and t.shape[-1] == K.HEAD_DIM and t.numel()
-           for t in (key_states, value_states)) and key_states.shape == value_states.shape:
+    kernel; other dtypes, devices and shapes torch's reductions, as do calls whose torch operations
+    are watched."""
+    if (all(type(t) is torch.Tensor and t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 4
+            and t.shape[-1] == K.HEAD_DIM and t.numel() for t in (key_states, value_states))
+            and key_states.shape == value_states.shape and key_states.device == value_states.device
+            and not K.torch_operations_watched()):
         return K.channel_energy(key_states.detach(), value_states.detach())
     return key_states.float().pow(2).sum(dim=(0, 1, 2)) + value_states.float().pow(2).sum(dim=(0, 1, 2))
 
