@@ -170,3 +170,31 @@ def test_chunked_native_route_agrees_with_torch_operations(cuda, dtype, monkeypa
     ref = A.chunked_turboquant_attention(qg, layer, **kw)
     assert len(calls) == 1 and ref.requires_grad
     check(got, ref.detach().double(), dtype)
+
+
+def test_calls_beyond_the_grid_take_torch_operations(cuda, monkeypatch):
+    """65536 KV heads of a batch, then both routes with the limit lowered."""
+    B, Hkv, n = 8192, 8, 2
+    q, k, v = (randn((B, Hkv, s, D), i, torch.bfloat16) for i, s in enumerate((1, n, n)))
+    got = A.chunked_turboquant_attention(q, PackedMSELayer(bits=3), new_key=k, new_value=v)
+    check(got, oracle(q, k, v, None), torch.bfloat16)
+    del q, k, v
+
+    layer = PackedMSELayer(bits=3, quantize_decode=False)
+    layer.initialize_from_dense(kv_bf16((2, 2, 300, D), seed=1), kv_bf16((2, 2, 300, D), seed=2))
+    layer._lazy_update = True
+    layer.update(kv_bf16((2, 2, 5, D), seed=3), kv_bf16((2, 2, 5, D), seed=4))
+    q = randn((2, 8, 1, D), 7, torch.bfloat16)
+    calls, add = [], K.DenseAttention.add
+    monkeypatch.setattr(K.DenseAttention, "add", lambda *a, **kw: calls.append(1) or add(*a, **kw))
+    for route in (lambda: A.fused_attention(q, layer, 4),
+                  lambda: A.chunked_turboquant_attention(q, layer, n_kv_groups=4)):
+        calls.clear()
+        native = route()
+        assert calls
+        calls.clear()
+        with monkeypatch.context() as m:
+            m.setattr(K.DenseAttention, "MAX_BLOCKS", 3)
+            ref = route()
+        assert not calls
+        check(native, ref.double(), torch.bfloat16)

@@ -510,7 +510,10 @@ extern "C" int tq_dense_attention(const void* q, int q_is_f32, int batch, int q_
     const int64_t heads = (int64_t)batch * kv_heads, rows = heads * rows_per_head;
     const int w = rows_per_head <= 32 ? 1 : rows_per_head <= 64 ? 2 : 4;
     const int64_t row_blocks = (rows_per_head + 32 * w - 1) / (32 * w);
-    if (heads > 65535 || row_blocks > 65535 || rows_per_head >= ((int64_t)1 << 31) - 128 || rows >= (int64_t)1 << 31)
+    // the merge's launch of 256 threads to a row, or to four rows, holds fewer than 2^32
+    const int64_t merge_blocks = slots > 8 ? rows : (rows + 3) / 4;
+    if (heads > 65535 || row_blocks > 65535 || rows_per_head >= ((int64_t)1 << 31) - 128 ||
+        merge_blocks >= (int64_t)1 << 24)
         return TQ_ERR_UNSUPPORTED;
     float* const part_o = partials + (int64_t)first_slot * rows * D;
     float2* const all_ms = reinterpret_cast<float2*>(partials + (int64_t)slots * rows * D);
@@ -534,10 +537,10 @@ extern "C" int tq_dense_attention(const void* q, int q_is_f32, int batch, int q_
     TQ_CHECK_LAUNCH();
     if (out_f32 || out_bf16) {
         if (slots > 8)
-            hipLaunchKernelGGL(dense_merge_kernel<8>, dim3((unsigned)rows), dim3(256), 0, s, partials, all_ms, slots, rows,
+            hipLaunchKernelGGL(dense_merge_kernel<8>, dim3((unsigned)merge_blocks), dim3(256), 0, s, partials, all_ms, slots, rows,
                                prev, prev_lse, out_f32, out_bf16);
         else
-            hipLaunchKernelGGL(dense_merge_kernel<2>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, partials, all_ms,
+            hipLaunchKernelGGL(dense_merge_kernel<2>, dim3((unsigned)merge_blocks), dim3(256), 0, s, partials, all_ms,
                                slots, rows, prev, prev_lse, out_f32, out_bf16);
         TQ_CHECK_LAUNCH();
     }

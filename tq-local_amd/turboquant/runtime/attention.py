@@ -168,7 +168,8 @@ def fused_attention(query_states: torch.Tensor, packed_layer: "PackedMSELayer", 
         return out.to(query_states.dtype).view(B, Hq, 1, D)
     _, o_packed, lse_packed = outs
     dk, dv = packed_layer._dense_buf  # capacity buffers: the first n_dense tokens are attended
-    if _native_rows(query_states, dk, dv) and dk.shape[1] * n_kv_groups == Hq:
+    if (_native_rows(query_states, dk, dv) and dk.shape[1] * n_kv_groups == Hq
+            and K.DenseAttention.takes(query_states, dk.shape[1])):
         # two launches: the dense tokens' partials, and their merge with the packed part.  The torch
         # operations below take ~22 (at B=4, Hq=32, N=8192 and 203 dense tokens 278 us a call, of
         # which the packed part takes 17)
@@ -311,6 +312,7 @@ def chunked_turboquant_attention(query_states: torch.Tensor, packed_layer: "Pack
             and (n_packed == 0 or packed_layer.dtype in (torch.bfloat16, torch.float32))
             and _native_rows(query_states, *parts) and _native_mask(attention_mask, query_states, total)
             and all(t.shape[1] * n_kv_groups == Q for t in parts)
+            and K.DenseAttention.takes(query_states, Q // n_kv_groups)
             and all(a is None or a.shape == b.shape for a, b in ((dense[0], dense[1]), (new_key, new_value)))
             and (n_packed == 0 or packed_layer._shape == (B, Q // n_kv_groups, D))):
         return _native_chunked(query_states, packed_layer, new_key, new_value, attention_mask, chunk_size,

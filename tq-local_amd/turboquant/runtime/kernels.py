@@ -468,6 +468,18 @@ class DenseAttention:
         self.partials = torch.empty(slots * (q.numel() + 2 * (q.numel() // HEAD_DIM)), dtype=torch.float32,
                                     device=q.device)
 
+    #: workgroups along one grid dimension (KV heads of the batch, and blocks of their query rows), and
+    #: query rows whose merge is one launch
+    MAX_BLOCKS = 65535
+    MAX_ROWS = 1 << 25
+
+    @classmethod
+    def takes(cls, q: torch.Tensor, kv_heads: int) -> bool:
+        """Whether the kernel's grid covers this many KV heads and query rows."""
+        B, Hq, Sq, _ = q.shape
+        rows = Hq // kv_heads * Sq  # in blocks of at least 32, of 128 from 65 rows on
+        return B * kv_heads <= cls.MAX_BLOCKS and -(-rows // 128) <= cls.MAX_BLOCKS and B * Hq * Sq <= cls.MAX_ROWS
+
     @staticmethod
     def split_count(q: torch.Tensor, kv_heads: int, tokens: int, most: int) -> int:
         """Splits of ``tokens`` tokens that fill the device without leaving any of them empty.
