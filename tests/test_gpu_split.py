@@ -138,6 +138,34 @@ def test_channels_of_equal_energy_are_the_public_function_s(cuda, n_out):
     assert torch.equal(layer._split.outlier_indices, outlier) and torch.equal(layer._split.normal_indices, normal)
 
 
+@pytest.mark.parametrize("B,H,T", [(3, 2, (1 << 31) // 6 + 3), (1, 3, (1 << 31) // 3 + 3), (1, 1, (1 << 31) + 5)])
+@pytest.mark.parametrize("prod", [False, True])
+def test_quantize_group_of_two_to_the_31_vectors(cuda, prod, B, H, T):
+    """Cut through the batch, the heads and the tokens.  One vector per (batch row, head), at every token."""
+    outl = _channels(3, 1)
+    sc = split_codecs(np.setdiff1d(np.arange(D), outl), outl, 2, 1, 0, True, cuda)
+    g = sc.key_outlier if prod else sc.value_outlier
+    assert B * H * T >= 1 << 31
+    x = kv_bf16((B, H, 1, D), seed=11, device=cuda)
+
+    def encode(x, slots, offset):
+        b = [torch.zeros(B, H, slots, K.row_bytes(g.dim, g.bits), dtype=torch.uint8, device=cuda),
+             torch.zeros(B, H, slots, dtype=torch.float16, device=cuda)]
+        if prod:
+            b += [torch.zeros(B, H, slots, 1, dtype=torch.uint8, device=cuda), torch.zeros_like(b[1])]
+        K.quantize_group(x, g, *b, offset=offset)
+        return b
+
+    want = encode(x, 1, 0)
+    got = encode(x.expand(B, H, T, D), T + 2, 1)
+    for w, o in zip(want, got):
+        for b in range(B):
+            for h in range(H):
+                row = o[b, h]
+                assert (row[1:T + 1] == w[b, h]).all()
+                assert int(row[0].count_nonzero()) == 0 and int(row[T + 1].count_nonzero()) == 0
+
+
 def _energy_prompt(seed, ch):
     k, v = kv_bf16((1, 2, 40, D), seed=seed), kv_bf16((1, 2, 40, D), seed=seed + 1)
     k[..., ch] *= 8.0

@@ -433,7 +433,21 @@ extern "C" int tq_quantize_group(const uint16_t* x, int batch, int heads, int64_
     if (n_vec == 0) return TQ_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (!aligned16(rotation) || (prod && !aligned16(qjl))) return TQ_ERR_UNSUPPORTED;
-    if (n_vec < GQ_SMALL || n_vec >= ((int64_t)1 << 31)) {
+    if (n_vec >= (int64_t)1 << 31) {  // the kernels count vectors in 31 bits: the call as two halves
+        const int b = batch / 2, h = batch > 1 ? 0 : heads / 2;
+        const int64_t t = batch > 1 || heads > 1 ? 0 : tokens / 2;
+        const int64_t slots = ((int64_t)b * heads + h) * out_cap;  // of the first half, but for a cut through the tokens
+        auto part = [&](int nb, int nh, int64_t nt, int64_t dx, int64_t rows, int64_t first) {
+            return tq_quantize_group(x + dx, nb, nh, nt, dim, x_sb, x_sh, x_st, channels, sub_dim, bits, rotation, centers,
+                                     boundaries, qjl, codes + rows * ((sub_dim * bits + 7) >> 3), norms + rows,
+                                     prod ? signs + rows * ((sub_dim + 7) >> 3) : nullptr, prod ? rnorms + rows : nullptr,
+                                     out_cap, first, stream);
+        };
+        st = part(b ? b : batch, h ? h : heads, t ? t : tokens, 0, 0, out_offset);
+        if (st != TQ_OK) return st;
+        return part(batch - b, heads - h, tokens - t, b * x_sb + h * x_sh + t * x_st, slots, out_offset + t);
+    }
+    if (n_vec < GQ_SMALL) {
         const int64_t sblocks = (n_vec + GAV - 1) / GAV;
         if (prod)
             hipLaunchKernelGGL((quantize_group_small_kernel<true>), dim3((unsigned)sblocks), dim3(GAT), 0, s, x,
