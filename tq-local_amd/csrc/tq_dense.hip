@@ -32,6 +32,7 @@
 // them up: 4 query tokens against the same rows take 18 us with 43 splits, 33 us with 21.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "tq_common.h"
 
@@ -60,15 +61,12 @@ __device__ __forceinline__ uint32_t high_halves(float a, float b) {
 }
 __device__ __forceinline__ float drop_high(float a) { return a - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u); }
 
-// A weight of few bits has zero lower terms, and 0 x inf would make NaN of the infinity that its leading
-// term's product with an infinite value gives.  So a tile that holds an infinity or a NaN is known when
-// it is staged; there the leading terms meet those alone, and then all terms the finite values.  Looking
-// at the values costs 0.6 us of the 155 of a call of 256 query tokens over 8192 packed ones.
-__device__ __forceinline__ uint32_t larger_halves(uint32_t a, uint32_t b) {  // of a and the magnitudes of b
-    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(
-        uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b & 0x7FFF7FFFu)));
-}
+// A weight of few bits has zero lower terms, and 0 x inf makes NaN of the infinity that its leading
+// term's product with an infinite value gives.  Either leaves an output that is not finite, whatever
+// follows, so a workgroup that ends with one walks its tokens a second time, with care: the leading terms
+// meet the infinities and NaN alone, and then all terms the finite values.  Looking at the outputs once
+// leaves a call of 4 query tokens over 8192 (32 query heads, 8 KV heads, boolean mask) at 23.6 us and one
+// of 256 at 92.5; looking at each tile's values as it is staged took 25.5 and 94.2, no care at all 23.3.
 // All ones in the halves of a bf16 pair that are not finite.
 __device__ __forceinline__ uint32_t special_mask(uint32_t p) {
     return ((p & 0x7FFFu) >= 0x7F80u ? 0x0000FFFFu : 0u) | ((p & 0x7FFF0000u) >= 0x7F800000u ? 0xFFFF0000u : 0u);
@@ -113,9 +111,6 @@ __global__ __launch_bounds__(64 * W, QT == 1 && W > 1 ? 2 : 1) void dense_attn_k
     constexpr int VP = TK / 2 * 16 / T; // (token pair, chunk) items of V
     __shared__ uint4 s_k[TK * 16];
     __shared__ uint32_t s_v[D * TK / 2];
-    __shared__ uint32_t s_special;  // the last tile whose values are not all finite
-    if (threadIdx.x == 0) s_special = ~0u;
-    __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane & 31, h = lane >> 5;
     const int b = blockIdx.z / a.kv_heads, kvh = blockIdx.z % a.kv_heads;
@@ -163,25 +158,6 @@ __global__ __launch_bounds__(64 * W, QT == 1 && W > 1 ? 2 : 1) void dense_attn_k
     int64_t lo = 0, hi = a.tokens;
     if (a.starts) lo = std::max<int64_t>(lo, a.starts[b] - a.pos0);
     if (a.ends) hi = std::min<int64_t>(hi, a.ends[b] - a.pos0);
-
-    f32x16 o[4];
-    float m = -__builtin_inff(), sum = 0.0f;  // running maximum of the logits, sum of the weights
-#pragma unroll
-    for (int d = 0; d < 4; ++d)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[d][i] = 0.0f;
-    if (a.accumulate && live) {
-        const float2 ms = a.part_ms[slot];
-        m = ms.x;
-        sum = h == 0 ? ms.y : 0.0f;
-#pragma unroll
-        for (int d = 0; d < 4; ++d)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float4 w = *reinterpret_cast<const float4*>(a.part_o + slot * D + 32 * d + 8 * j + 4 * h);
-                o[d][4 * j] = w.x, o[d][4 * j + 1] = w.y, o[d][4 * j + 2] = w.z, o[d][4 * j + 3] = w.w;
-            }
-    }
 
     const uint16_t* kb = a.k + b * a.k_sb + kvh * a.k_sh;
     const uint16_t* vb = a.v + b * a.v_sb + kvh * a.v_sh;
@@ -238,8 +214,7 @@ __global__ __launch_bounds__(64 * W, QT == 1 && W > 1 ? 2 : 1) void dense_attn_k
             }
         }
     };
-    auto store_tile = [&](uint32_t tile) {
-        uint32_t top_v = 0u;
+    auto store_tile = [&]() {
 #pragma unroll
         for (int i = 0; i < KC; ++i) {
             const int id = threadIdx.x + i * T, tok = id >> 4, c = id & 15;
@@ -253,8 +228,6 @@ __global__ __launch_bounds__(64 * W, QT == 1 && W > 1 ? 2 : 1) void dense_attn_k
             const uint32_t x[4] = {pv[i][0].x, pv[i][0].y, pv[i][0].z, pv[i][0].w};
             const uint32_t y[4] = {pv[i][1].x, pv[i][1].y, pv[i][1].z, pv[i][1].w};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) top_v = larger_halves(larger_halves(top_v, x[e]), y[e]);
-#pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const int dim = 8 * c + e;
                 const uint32_t w = (e & 1) ? __builtin_amdgcn_perm(y[e >> 1], x[e >> 1], 0x07060302u)
@@ -262,131 +235,156 @@ __global__ __launch_bounds__(64 * W, QT == 1 && W > 1 ? 2 : 1) void dense_attn_k
                 s_v[dim * (TK / 2) + ((chunk ^ v_swizzle(dim)) << 2) + pair] = w;
             }
         }
-        if (special_mask(top_v)) s_special = tile;
     };
 
     // four waves hold the next tile's 6 KB of registers while they compute; with one or two waves
     // a thread's share would not fit beside the accumulators, and the tile is loaded when needed
     constexpr bool AHEAD = W == 4;
     const float c2 = a.scale * LOG2E;
-    float top = LOGITS ? m : m / a.scale;  // the running maximum in the scores' unit
-    if (AHEAD && t_begin < t_end) load_tile(t_begin);
-    for (int64_t t0 = t_begin; t0 < t_end; t0 += TK) {
-        if (t0 != t_begin) __syncthreads();  // every wave is done with the previous tile
-        if (!AHEAD) load_tile(t0);
-        const uint32_t tile = (uint32_t)(t0 / TK);  // a number met again only sends a tile the longer way
-        store_tile(tile);
-        __syncthreads();
-        const uint32_t special = s_special;  // on its way while the scores are computed
-
-        // the tile's mask, before the next one's takes its place
-        uint32_t mb[MASK == MASK_BOOL ? 4 : 1];
-        float add[LOGITS ? 16 : 1];
-        if constexpr (MASK == MASK_BOOL) {
+    f32x16 o[4];
+    float top, sum;  // running maximum in the scores' unit, sum of the weights
+    auto walk = [&](auto careful) {
+        float m = -__builtin_inff();  // of the logits
+        sum = 0.0f;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) mb[j] = next_mb[j];
-        } else if constexpr (LOGITS) {
+        for (int d = 0; d < 4; ++d)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) add[i] = next_add[i];
-        }
-        if (AHEAD && t0 + TK < t_end) load_tile(t0 + TK);
-
-        // ---- scores
-        f32x16 s;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = 0.0f;
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            Frag kf;
-            kf.q = s_k[r * 16 + ((2 * ks + h) ^ (r & 15))];
-#pragma unroll
-            for (int t = QT - 1; t >= 0; --t) s = mfma_32(kf, q[t][ks], s);
-        }
-        if constexpr (LOGITS) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) s[i] = s[i] * a.scale + add[i];
-        }
-        if constexpr (MASK == MASK_BOOL) {  // most tiles of a causal mask are attended whole
-            const uint32_t all = mb[0] & mb[1] & mb[2] & mb[3];
-            if (__any(all != 0x01010101u)) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    if (!((mb[i >> 2] >> (8 * (i & 3))) & 0xFFu)) s[i] = -__builtin_inff();
-            }
-        }
-        if (t0 < lo || t0 + TK > hi) {  // uniform: some position is not attended
-            const int lo_t = (int)std::min<int64_t>(std::max<int64_t>(lo - t0, 0), TK);
-            const int hi_t = (int)std::min<int64_t>(std::max<int64_t>(hi - t0, 0), TK);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int tok = 8 * (i >> 2) + 4 * h + (i & 3);
-                if (tok < lo_t || tok >= hi_t) s[i] = -__builtin_inff();
-            }
-        }
-        float mx = top;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float safe = mx == -__builtin_inff() ? 0.0f : mx;  // nothing attended so far
-        if (__any(mx > top)) {
-            const float corr = LOGITS ? exp2_((top - safe) * LOG2E) : exp2_(__builtin_fmaf(top, c2, -safe * c2));
-            sum *= corr;
+            for (int i = 0; i < 16; ++i) o[d][i] = 0.0f;
+        if (a.accumulate && live) {
+            const float2 ms = a.part_ms[slot];
+            m = ms.x;
+            sum = h == 0 ? ms.y : 0.0f;
 #pragma unroll
             for (int d = 0; d < 4; ++d)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) o[d][i] *= corr;
+                for (int j = 0; j < 4; ++j) {
+                    const float4 w = *reinterpret_cast<const float4*>(a.part_o + slot * D + 32 * d + 8 * j + 4 * h);
+                    o[d][4 * j] = w.x, o[d][4 * j + 1] = w.y, o[d][4 * j + 2] = w.z, o[d][4 * j + 3] = w.w;
+                }
         }
-        top = mx;
-        const float base = safe * c2;
+        top = LOGITS ? m : m / a.scale;
+        if (AHEAD && t_begin < t_end) load_tile(t_begin);
+        for (int64_t t0 = t_begin; t0 < t_end; t0 += TK) {
+            if (t0 != t_begin) __syncthreads();  // every wave is done with the previous tile
+            if (!AHEAD) load_tile(t0);
+            store_tile();
+            __syncthreads();
+
+            // the tile's mask, before the next one's takes its place
+            uint32_t mb[MASK == MASK_BOOL ? 4 : 1];
+            float add[LOGITS ? 16 : 1];
+            if constexpr (MASK == MASK_BOOL) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            s[i] = LOGITS ? exp2_((s[i] - safe) * LOG2E) : exp2_(__builtin_fmaf(s[i], c2, -base));
-            sum += s[i];
-        }
-        if (__builtin_amdgcn_readfirstlane((int)special) == (int)tile) {  // uniform over the workgroup
+                for (int j = 0; j < 4; ++j) mb[j] = next_mb[j];
+            } else if constexpr (LOGITS) {
 #pragma unroll
-            for (int kb16 = 0; kb16 < TK / 16; ++kb16) {
-                Frag p;
+                for (int i = 0; i < 16; ++i) add[i] = next_add[i];
+            }
+            if (AHEAD && t0 + TK < t_end) load_tile(t0 + TK);
+
+            // ---- scores
+            f32x16 s;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) p.u[k] = high_halves(s[8 * kb16 + 2 * k], s[8 * kb16 + 2 * k + 1]);
+            for (int i = 0; i < 16; ++i) s[i] = 0.0f;
 #pragma unroll
-                for (int d = 0; d < 4; ++d) {
-                    const int dim = 32 * d + r;
-                    Frag vf;
-                    vf.q = reinterpret_cast<const uint4*>(s_v)[dim * (TK / 8) + ((2 * kb16 + h) ^ v_swizzle(dim))];
+            for (int ks = 0; ks < 8; ++ks) {
+                Frag kf;
+                kf.q = s_k[r * 16 + ((2 * ks + h) ^ (r & 15))];
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) vf.u[k] &= special_mask(vf.u[k]);
-                    o[d] = mfma_32(vf, p, o[d]);
+                for (int t = QT - 1; t >= 0; --t) s = mfma_32(kf, q[t][ks], s);
+            }
+            if constexpr (LOGITS) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s[i] = s[i] * a.scale + add[i];
+            }
+            if constexpr (MASK == MASK_BOOL) {  // most tiles of a causal mask are attended whole
+                const uint32_t all = mb[0] & mb[1] & mb[2] & mb[3];
+                if (__any(all != 0x01010101u)) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        if (!((mb[i >> 2] >> (8 * (i & 3))) & 0xFFu)) s[i] = -__builtin_inff();
                 }
             }
-            __syncthreads();
+            if (t0 < lo || t0 + TK > hi) {  // uniform: some position is not attended
+                const int lo_t = (int)std::min<int64_t>(std::max<int64_t>(lo - t0, 0), TK);
+                const int hi_t = (int)std::min<int64_t>(std::max<int64_t>(hi - t0, 0), TK);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int tok = 8 * (i >> 2) + 4 * h + (i & 3);
+                    if (tok < lo_t || tok >= hi_t) s[i] = -__builtin_inff();
+                }
+            }
+            float mx = top;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const float safe = mx == -__builtin_inff() ? 0.0f : mx;  // nothing attended so far
+            if (__any(mx > top)) {
+                const float corr = LOGITS ? exp2_((top - safe) * LOG2E) : exp2_(__builtin_fmaf(top, c2, -safe * c2));
+                sum *= corr;
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) o[d][i] *= corr;
+            }
+            top = mx;
+            const float base = safe * c2;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                s[i] = LOGITS ? exp2_((s[i] - safe) * LOG2E) : exp2_(__builtin_fmaf(s[i], c2, -base));
+                sum += s[i];
+            }
+            if constexpr (careful) {
+#pragma unroll
+                for (int kb16 = 0; kb16 < TK / 16; ++kb16) {
+                    Frag p;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) p.u[k] = high_halves(s[8 * kb16 + 2 * k], s[8 * kb16 + 2 * k + 1]);
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const int dim = 32 * d + r;
+                        Frag vf;
+                        vf.q = reinterpret_cast<const uint4*>(s_v)[dim * (TK / 8) + ((2 * kb16 + h) ^ v_swizzle(dim))];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) vf.u[k] &= special_mask(vf.u[k]);
+                        o[d] = mfma_32(vf, p, o[d]);
+                    }
+                }
+                __syncthreads();
 #pragma unroll 1
-            for (int i = threadIdx.x; i < D * TK / 2; i += T) s_v[i] &= ~special_mask(s_v[i]);
-            __syncthreads();
-        }
-        // ---- values: 16 tokens per step
-#pragma unroll
-        for (int kb16 = 0; kb16 < TK / 16; ++kb16) {
-            Frag p[3];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                float p0 = s[8 * kb16 + 2 * k], p1 = s[8 * kb16 + 2 * k + 1];
-                p[0].u[k] = high_halves(p0, p1);
-                p0 = drop_high(p0), p1 = drop_high(p1);
-                p[1].u[k] = high_halves(p0, p1);
-                p[2].u[k] = high_halves(drop_high(p0), drop_high(p1));
+                for (int i = threadIdx.x; i < D * TK / 2; i += T) s_v[i] &= ~special_mask(s_v[i]);
+                __syncthreads();
             }
+            // ---- values: 16 tokens per step
 #pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                Frag vf;
-                const int dim = 32 * d + r;
-                vf.q = reinterpret_cast<const uint4*>(s_v)[dim * (TK / 8) + ((2 * kb16 + h) ^ v_swizzle(dim))];
+            for (int kb16 = 0; kb16 < TK / 16; ++kb16) {
+                Frag p[3];
 #pragma unroll
-                for (int t = 2; t >= 0; --t) o[d] = mfma_32(vf, p[t], o[d]);
+                for (int k = 0; k < 4; ++k) {
+                    float p0 = s[8 * kb16 + 2 * k], p1 = s[8 * kb16 + 2 * k + 1];
+                    p[0].u[k] = high_halves(p0, p1);
+                    p0 = drop_high(p0), p1 = drop_high(p1);
+                    p[1].u[k] = high_halves(p0, p1);
+                    p[2].u[k] = high_halves(drop_high(p0), drop_high(p1));
+                }
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    Frag vf;
+                    const int dim = 32 * d + r;
+                    vf.q = reinterpret_cast<const uint4*>(s_v)[dim * (TK / 8) + ((2 * kb16 + h) ^ v_swizzle(dim))];
+#pragma unroll
+                    for (int t = 2; t >= 0; --t) o[d] = mfma_32(vf, p[t], o[d]);
+                }
             }
         }
-    }
-
+    };
+    walk(std::false_type{});
+    uint32_t largest = 0u;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) largest = max(largest, __float_as_uint(o[d][i]) & 0x7FFFFFFFu);
+    if (__syncthreads_or(largest >= 0x7F800000u)) walk(std::true_type{});
     sum += __shfl_xor(sum, 32);
     if (!live) return;
     if (h == 0) a.part_ms[slot] = make_float2(LOGITS ? top : top * a.scale, sum);
