@@ -89,6 +89,35 @@ def test_an_infinite_value_stays_infinite(cuda, Sq, n):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("Sq", [1, 12, 40])  # one, two and four waves per workgroup
+@pytest.mark.parametrize("form", ["key", "few bits", "query"])
+def test_infinite_products_keep_their_sign(cuda, dtype, Sq, form):
+    """Logits of -inf leave their token out, whatever terms an fp32 query is held in (a query element of
+    few bits has zero lower terms, an infinity no others); +inf makes NaN of its row and no other."""
+    n, tok = 70, 37
+    q, k, v = randn((1, 4, Sq, D), 1, dtype), randn((1, 1, n, D), 2, torch.bfloat16), randn((1, 1, n, D), 3, torch.bfloat16)
+    add = torch.zeros(1, 1, 1, n, device="cuda")
+    if form == "query":  # head 1: -inf for every token
+        k[..., 7] = -1.0 - k[..., 7].abs()
+        q[0, 1, :, 7] = float("inf")
+        out = K.DenseAttention(q, 1, 1).add(k, v, n, 0, 1, SCALE, out=torch.float32)
+        assert (out[0, 1] == 0).all()  # nothing attended
+        q[0, 1, :, 7] = float("-inf")
+        assert K.DenseAttention(q, 1, 1).add(k, v, n, 0, 1, SCALE, out=torch.float32)[0, 1].isnan().all()
+    else:
+        k[0, 0, tok, 9] = float("-inf")
+        q[..., 9] = 1.5 if form == "few bits" else q[..., 9].abs() + 0.1
+        q[0, 1, :, 9] *= -1
+        add[..., tok] = float("-inf")
+        out = K.DenseAttention(q, 1, 1).add(k, v, n, 0, 1, SCALE, out=torch.float32)
+        assert out[0, 1].isnan().all()
+    heads = [0, 2, 3]
+    k = k.masked_fill(k.isinf(), 0.0)
+    q = q.masked_fill(q.isinf(), 0.0)
+    check(out[:, heads], oracle(q[:, heads], k, v, add), torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("Sq", [1, 12, 40])  # one, two and four waves per workgroup
 @pytest.mark.parametrize("form", ["mask", "bounds", "far below", "faint"])
 def test_values_of_unattended_tokens_add_nothing(cuda, dtype, Sq, form):
     """A weight of 0 (masked, out of bounds, 2^-x that underflows) leaves out a value of the type's

@@ -61,12 +61,19 @@ __device__ __forceinline__ uint32_t high_halves(float a, float b) {
 }
 __device__ __forceinline__ float drop_high(float a) { return a - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u); }
 
+// The same for a query element, of which an infinity leaves nothing and a NaN stays one.
+__device__ __forceinline__ float drop_high_query(float a) {
+    return __builtin_fabsf(a) == __builtin_inff() ? 0.0f : drop_high(a);
+}
+
 // A weight of few bits has zero lower terms, and 0 x inf makes NaN of the infinity that its leading
 // term's product with an infinite value gives.  Either leaves an output that is not finite, whatever
 // follows, so a workgroup that ends with one walks its tokens a second time, with care: the leading terms
 // meet the infinities and NaN alone, and then all terms the finite values.  Looking at the outputs once
 // leaves a call of 4 query tokens over 8192 (32 query heads, 8 KV heads, boolean mask) at 23.6 us and one
 // of 256 at 92.5; looking at each tile's values as it is staged took 25.5 and 94.2, no care at all 23.3.
+// An fp32 query's terms meet the keys alike.
+
 // All ones in the halves of a bf16 pair that are not finite.
 __device__ __forceinline__ uint32_t special_mask(uint32_t p) {
     return ((p & 0x7FFFu) >= 0x7F80u ? 0x0000FFFFu : 0u) | ((p & 0x7FFF0000u) >= 0x7F800000u ? 0xFFFF0000u : 0u);
@@ -137,7 +144,7 @@ __global__ __launch_bounds__(64 * W, QT == 1 && W > 1 ? 2 : 1) void dense_attn_k
                 for (int k = 0; k < 4; ++k) {
                     float e0 = live ? e[2 * k] : 0.0f, e1 = live ? e[2 * k + 1] : 0.0f;
                     q[0][s].u[k] = high_halves(e0, e1);
-                    e0 = drop_high(e0), e1 = drop_high(e1);
+                    e0 = drop_high_query(e0), e1 = drop_high_query(e1);
                     q[QT - 2][s].u[k] = high_halves(e0, e1);
                     q[QT - 1][s].u[k] = high_halves(drop_high(e0), drop_high(e1));
                 }
@@ -290,6 +297,16 @@ __global__ __launch_bounds__(64 * W, QT == 1 && W > 1 ? 2 : 1) void dense_attn_k
             for (int ks = 0; ks < 8; ++ks) {
                 Frag kf;
                 kf.q = s_k[r * 16 + ((2 * ks + h) ^ (r & 15))];
+                if constexpr (careful && QT > 1) {
+                    Frag inf;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        inf.u[k] = kf.u[k] & special_mask(kf.u[k]);
+                        kf.u[k] ^= inf.u[k];
+                    }
+                    // none: an infinite query element would make NaN of the zeros
+                    if (__any((inf.u[0] | inf.u[1] | inf.u[2] | inf.u[3]) != 0u)) s = mfma_32(inf, q[0][ks], s);
+                }
 #pragma unroll
                 for (int t = QT - 1; t >= 0; --t) s = mfma_32(kf, q[t][ks], s);
             }
