@@ -86,7 +86,8 @@ def test_plain_prefill_encoder_on_hard_rows(cuda, bits, prod, rotation, T):
         compare(x, (kc, kn), O.encode_mse(rows, bits, h[0], h[2]), T)
 
 
-@pytest.mark.parametrize("T", [521, 8192 + 19, 12 * 1024 + 19])
+# a tile per workgroup, and one and two tiles per wave (on 256 CUs)
+@pytest.mark.parametrize("T", [521, 8192 + 19, 12 * 1024 + 19, 25 * 1024 + 19])
 @pytest.mark.parametrize("d,bits,extra,qjl", [(3, 4, 1, True), (4, 4, 4, False), (8, 3, 4, True), (13, 2, 3, False),
                                               (33, 1, 1, False), (40, 2, 2, True), (60, 4, 3, True)])
 def test_group_prefill_encoder_on_hard_rows(cuda, d, bits, extra, qjl, T):

@@ -79,8 +79,9 @@ def test_quantize_prod_bit_exact(cuda, bits):
 
 def _matrix_core_input(cuda, seed, T=2101):
     """[2, 3, T, D] bf16 keys as a strided [B, H, T, D] view of a [B, T, H, D] buffer, with the
-    special rows at tokens 100..105: 6 T vectors (>= 4096, so the matrix-core encoder runs),
-    a tile count that is not a multiple of 16 vectors."""
+    special rows at tokens 100..105: 6 T vectors, not whole tiles of 16.  On 256 CUs 2004 and 12606
+    (keys) vectors take the encoder of a tile per workgroup, 12606 (values) and 16812 the one of a
+    single fp32 pass, 34830 and 51210 the bf16 products at one and two tiles per wave."""
     x = kv_bf16((2, 3, T, D), seed=seed, device=cuda)
     x[:, :, 100:106] = _special_rows(cuda)[0, 0]
     x = x.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
@@ -89,8 +90,9 @@ def _matrix_core_input(cuda, seed, T=2101):
 
 
 @pytest.mark.parametrize("bits", [1, 2, 3, 4])
-def test_quantize_mse_matrix_core_bit_exact(cuda, bits):
-    x = _matrix_core_input(cuda, 30 + bits)
+@pytest.mark.parametrize("T", [334, 2101, 5805, 8535])
+def test_quantize_mse_matrix_core_bit_exact(cuda, bits, T):
+    x = _matrix_core_input(cuda, 30 + bits, T)
     codec = layer_codecs(D, bits, 0, False, cuda).value
     B, H, n, _ = x.shape
     cap, off = n + 7, 3
@@ -108,8 +110,9 @@ def test_quantize_mse_matrix_core_bit_exact(cuda, bits):
 
 
 @pytest.mark.parametrize("bits", [2, 3, 4])
-def test_quantize_prod_matrix_core_bit_exact(cuda, bits):
-    x = _matrix_core_input(cuda, 50 + bits)
+@pytest.mark.parametrize("T", [334, 2101, 2802, 5805, 8535])
+def test_quantize_prod_matrix_core_bit_exact(cuda, bits, T):
+    x = _matrix_core_input(cuda, 50 + bits, T)
     lc = layer_codecs(D, bits, 0, True, cuda)
     B, H, n, _ = x.shape
     cap, off = n + 5, 2
@@ -132,13 +135,14 @@ def test_quantize_prod_matrix_core_bit_exact(cuda, bits):
         assert int(t[:, :, :off].count_nonzero()) == 0 and int(t[:, :, off + n:].count_nonzero()) == 0
 
 
+@pytest.mark.parametrize("T", [334, 2101, 5805, 8535])
 @pytest.mark.parametrize("irregular", ["repeated", "outlying", "unsorted"])
-def test_quantize_mse_matrix_core_irregular_boundaries(cuda, irregular):
+def test_quantize_mse_matrix_core_irregular_boundaries(cuda, irregular, T):
     """Boundary sets the uniform bucketize grid does not cover (a repeated boundary, one far
     outside the others, an unsorted pair) go through the binary search; codes still equal the
     oracle's #{b < z}.  For the unsorted set the search no longer counts (it assumes order),
     so only its own determinism is checked there."""
-    x = _matrix_core_input(cuda, 77)
+    x = _matrix_core_input(cuda, 77, T)
     base = layer_codecs(D, 4, 0, False, cuda).value
     b = base.boundaries.clone()
     if irregular == "repeated":
@@ -187,16 +191,16 @@ def test_quantize_strided_input_and_decode_append(cuda):
     assert np.array_equal(u16(bufs[3]).reshape(-1), rr)
 
 
+# where a call changes kernels: two and four vectors per workgroup, a tile per workgroup, a single fp32
+# pass (values, keys), the bf16 products at one and two tiles per wave (the last two on 256 CUs)
+@pytest.mark.parametrize("n", [257, 513, 1025, 12289, 16385, 32769, 49153])
 @pytest.mark.parametrize("bits,prod", [(1, False), (3, False), (4, False), (2, True), (4, True)])
-def test_small_batch_and_matrix_core_encoders_agree(cuda, bits, prod):
-    """The same 4096 vectors encoded by one call (the matrix-core kernel, 4096 and up) and by
-    two calls of 4095 and 1 vectors (the small-batch kernel) are bit-identical: codes, norms,
-    and for Q_prod signs and residual norms."""
-    B, H, T = 4, 8, 128  # 4096 vectors
-    x = kv_bf16((B, H, T, D), seed=60 + bits, device=cuda).reshape(1, 1, B * H * T, D)
+def test_encoders_agree_across_the_size_lines(cuda, bits, prod, n):
+    """n vectors encoded by one call, on the upper side of a line, and by calls of n - 1 (the lower
+    side) and 1 are bit-identical: codes, norms, and for Q_prod signs and residual norms."""
+    x = kv_bf16((1, 1, n, D), seed=60 + bits, device=cuda)
     lc = layer_codecs(D, bits, 0, prod, cuda)
     codec = lc.key if prod else lc.value
-    n = x.shape[2]
 
     def bufs():
         b = [torch.zeros(1, 1, n, K.row_bytes(D, codec.bits), dtype=torch.uint8, device=cuda),

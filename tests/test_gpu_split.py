@@ -95,16 +95,18 @@ def test_quantize_group_prod_bit_exact(cuda, d, bits, extra):
         assert np.array_equal(u16(rnorms).reshape(-1), rr)
 
 
+# where a call changes kernels: a tile per workgroup, the bf16 products (values, keys), two tiles per
+# wave (on 256 CUs)
+@pytest.mark.parametrize("n", [1025, 20480, 24576, 49153])
 @pytest.mark.parametrize("prod", [False, True])
-def test_group_small_batch_and_lane_encoders_agree(cuda, prod):
-    """One group of 8192 vectors encoded by one call (the lane-per-vector kernel, 8192 and up) and
-    by calls of 8191 and 1 vectors (the small-batch kernel) is bit-identical."""
+def test_group_encoders_agree_across_the_size_lines(cuda, prod, n):
+    """One group of n vectors encoded by one call, on the upper side of a line, and by calls of
+    n - 1 (the lower side) and 1 vectors is bit-identical."""
     outl = _channels(13, 5)
     sc = split_codecs(np.setdiff1d(np.arange(D), outl), outl, 3, 2, 0, True, cuda)
     g = sc.key_outlier if prod else sc.value_normal
-    x = _with_specials(kv_bf16((1, 1, 8187, D), seed=77, device=cuda), outl)
-    n = x.shape[2]
-    assert n == 8192
+    x = _with_specials(kv_bf16((1, 1, n - 5, D), seed=77, device=cuda), outl)
+    assert x.shape[2] == n
 
     def bufs():
         b = [torch.zeros(1, 1, n, K.row_bytes(g.dim, g.bits), dtype=torch.uint8, device=cuda),
