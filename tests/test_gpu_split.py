@@ -126,12 +126,17 @@ def test_group_encoders_agree_across_the_size_lines(cuda, prod, n):
 
 
 @pytest.mark.parametrize("n_out", [3, 4, 17])
-def test_channels_of_equal_energy_are_the_public_function_s(cuda, n_out):
-    """Energies tied between 64 channels (exactly: sums of ones): a layer splits at the channels that
+@pytest.mark.parametrize("form", ["tied at the line", "tied above it", "NaN"])
+def test_channels_of_equal_energy_are_the_public_function_s(cuda, n_out, form):
+    """Energies tied between channels (exactly: sums of ones): a layer splits at the channels that
     detect_outlier_channels names, which are those of the device's topk over the torch reductions."""
     k = torch.ones(1, 2, 40, D, dtype=torch.bfloat16, device=cuda)
     k[..., ::2] = -2.0
     v = torch.ones_like(k)
+    if form == "tied above it":
+        k[..., 100:100 + n_out] = 4.0
+    elif form == "NaN":
+        k[..., 3, 70] = float("nan")
     layer = PackedMSELayer(bits=4, num_outlier_channels=n_out)
     layer.initialize_from_dense(k, v)
     outlier, normal = detect_outlier_channels(k, v, n_out)

@@ -147,9 +147,9 @@ class _Store:
         self._alloc(cap)
 
     #: up to here the buffers are parts of one allocation, cleared by one launch: six took 12 us of a short
-    #: prompt's 67, twelve 32 us of the 546 of a split layer of 36 MB.  Above, clearing is bound by
-    #: bandwidth, and buffers of their own let a growing store give back each old one as soon as it is
-    #: copied.
+    #: prompt's 67, twelve 32 us of the 546 of a split layer of 36 MB.  The line bounds what a kept view of
+    #: one buffer holds on to, and what a growing store holds twice: buffers of their own are given back
+    #: each as soon as it is copied.  A larger layer still pays for its launches.
     ONE_BLOCK_BYTES = 64 << 20
 
     def _alloc(self, cap: int) -> None:
@@ -239,12 +239,16 @@ class PackedMSELayer(CacheLayerMixin):
         self.device = key_states.device
         D = int(key_states.shape[-1])
         if 0 < self.num_outlier_channels < D:
-            # the choice of detect_outlier_channels, among equal energies too (the device's topk); the
-            # channels are needed on the host, where they go once and are sorted
-            top = torch.topk(_channel_energy(key_states, value_states), self.num_outlier_channels).indices
-            outlier = np.sort(top.cpu().numpy())
-            self._split = split_codecs(np.setdiff1d(np.arange(D), outlier), outlier, self.bits, self.outlier_extra_bits,
-                                       self.seed, self.use_qjl_keys, self.device, self.grid_size)
+            # the channels are needed on the host: the 128 energies go there, once, and are sorted there.
+            # Where the choice is between equal energies (or NaN) it is left to the device's topk, as in
+            # detect_outlier_channels: always taking that one cost a prompt of 2 x 16384 tokens 28 us of 552
+            n, energy = self.num_outlier_channels, _channel_energy(key_states, value_states)
+            top = torch.topk(energy.cpu(), n + 1)
+            unique = bool(top.values[n - 1] > top.values[n])
+            outlier = np.sort((top.indices[:n] if unique else torch.topk(energy, n).indices.cpu()).numpy())
+            normal = np.delete(np.arange(D), outlier)
+            self._split = split_codecs(normal, outlier, self.bits, self.outlier_extra_bits, self.seed,
+                                       self.use_qjl_keys, self.device, self.grid_size)
         else:
             self.codecs = layer_codecs(D, self.bits, self.seed, self.use_qjl_keys, self.device, self.grid_size)
         self.is_initialized = True
