@@ -310,6 +310,9 @@ int tq_decode_attention_groups(const uint16_t* q, int batch, int q_heads, int kv
  *            and normalised after this call's tokens; a row with nothing attended is 0.  prev /
  *            prev_lse (nullable together): another part of the same softmax, normalised fp32 rows
  *            and their log-sum-exp (tq_decode_attention's out_f32 and lse_out), weighed in
+ *
+ * TQ_ERR_UNSUPPORTED beyond 65535 KV heads of the batch, 65535 blocks of 128 query rows of one of
+ * them, or 2^26 query rows (2^24 with more than 8 slots).
  */
 int tq_dense_attention(const void* q, int q_is_f32, int batch, int q_heads, int kv_heads, int q_len, int dim,
                        int64_t q_sb, int64_t q_sh, int64_t q_ss, const uint16_t* k, const uint16_t* v,

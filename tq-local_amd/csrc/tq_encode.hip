@@ -42,7 +42,9 @@ namespace {
 using namespace tqmx;
 using tqenc::EncodeArgs;
 constexpr int D = TQ_DIM;
-constexpr int CW = 12;          // waves per workgroup of the codes kernel
+// Waves per workgroup of the codes kernel: 168 registers each, of which the variants of two tiles per wave
+// spill 16-32 bytes a lane (channel groups up to 172).  16 waves spill more: 415 us against 300 at 2M vectors.
+constexpr int CW = 12;
 constexpr int CT = 64 * CW;
 constexpr uint32_t NORM_ONLY = 255;
 

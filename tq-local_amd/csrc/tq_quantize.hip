@@ -286,6 +286,7 @@ constexpr int64_t MQ_MIN_VECTORS = 1025;
 //   vectors   12288        16384        20480        32768        40960
 //   here      39.0 / 17.0  39.7 / 17.3  40.1 / 17.4  41.9 / 18.2  72.9 / 29.3
 //   there     26.8 / 13.9  35.0 / 18.1  42.5 / 18.8  46.8 / 19.4  61.3 / 22.6
+// The lower lines are of 256 CUs, as those of tq_encode.hip; the upper one follows the device.
 constexpr int64_t PASS_MIN_PROD = 16384, PASS_MIN_MSE = 12288;  // more than this many vectors
 constexpr int LUT_MAX = 512;                // cells of the bucketize grid
 
@@ -668,8 +669,8 @@ __global__ __launch_bounds__(MQ_THREADS) void dequantize_kernel(
         const float rn = tq::f16_to_f32(raw_rnorm);
         float cv[32];
         centers_of<BITS>(w, g, s_cent, cv);
-        // the next item's rows beside this one's products (Q_mse kernels, four waves on a SIMD, would
-        // lose one to the registers)
+        // the next item's rows beside this one's products (not in the Q_mse kernels: the 1- and 2-bit ones, at
+        // 126 registers two workgroups on a CU, would lose one; the 3- and 4-bit ones, at 129 and 130, have one)
         const int64_t next = item + (int64_t)gridDim.x * MQ_WAVES;
         if (QJL && next < n_items) fetch(next);
         f32x4 acc[NT];
