@@ -118,6 +118,23 @@ def test_infinite_products_keep_their_sign(cuda, dtype, Sq, form):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("Sq", [1, 12, 40])  # one, two and four waves per workgroup
+@pytest.mark.parametrize("tok", [3, 140, 299])  # in the first, the second and the last range
+def test_an_infinite_value_in_continued_partials(cuda, dtype, Sq, tok):
+    """The second walk of a range starts from the partials it was given, whole or already infinite."""
+    n = 300
+    q, k, v = randn((1, 4, Sq, D), 1, dtype), randn((1, 1, n, D), 2, torch.bfloat16), randn((1, 1, n, D), 3, torch.bfloat16)
+    v[0, 0, tok, 5], v[0, 0, tok, 7] = float("inf"), float("-inf")
+    att = K.DenseAttention(q, 1, 2)
+    for a, b in ((0, 128), (128, 200), (200, n)):
+        out = att.add(k[:, :, a:b], v[:, :, a:b], b - a, 0, 2, SCALE, accumulate=a > 0,
+                      out=torch.float32 if b == n else None)
+    assert (out[..., 5] == float("inf")).all() and (out[..., 7] == float("-inf")).all()
+    rest = [d for d in range(D) if d not in (5, 7)]
+    check(out[..., rest], oracle(q, k, v[..., rest], None), torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("Sq", [1, 12, 40])  # one, two and four waves per workgroup
 @pytest.mark.parametrize("form", ["mask", "bounds", "far below", "faint"])
 def test_values_of_unattended_tokens_add_nothing(cuda, dtype, Sq, form):
     """A weight of 0 (masked, out of bounds, 2^-x that underflows) leaves out a value of the type's
